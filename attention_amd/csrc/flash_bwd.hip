@@ -413,6 +413,23 @@ static void launch_dkv(const FlashBwdParams& m, dim3 grid, dim3 block, hipStream
     }
 }
 
+// Launch geometry of the dQ and dK/dV kernels (tiles, pairing, the map from workgroups to tiles).
+static int plan_bwd(FlashBwdParams& m, int64_t B, int64_t H_kv, bool causal, bool ragged) {
+    m.n_tiles = (m.N + kFlashRows - 1) / kFlashRows;
+    // causal launches: a workgroup takes a long and a short tile of its head, so that all (of a sequence) do the same work
+    m.paired = (causal && m.n_tiles >= 2 && tuning().bwd_pair.load() != 0) ? 1 : 0;
+    m.spread = ragged ? 1 : 0;
+    m.n_bh = (int32_t)(B * m.H);
+    const int64_t units = bwd_units(m), pairs_q = B * m.H, pairs_kv = B * H_kv;
+    const int64_t total_q = pairs_q * units, total_kv = pairs_kv * units;
+    const int64_t per_q = ragged ? (pairs_q + 7) / 8 * units : (total_q + 7) / 8;
+    const int64_t per_kv = ragged ? (pairs_kv + 7) / 8 * units : (total_kv + 7) / 8;
+    if (per_q * 8 > 0x7FFFFFF0ll || per_kv * 8 > 0x7FFFFFF0ll) return AHPC_ERR_BAD_SHAPE;
+    m.total_q = (int32_t)total_q; m.per_xcd_q = (int32_t)per_q;
+    m.total_kv = (int32_t)total_kv; m.per_xcd_kv = (int32_t)per_kv;
+    return AHPC_OK;
+}
+
 // Statistics, dQ, dK and dV.  pm: the packed copy of a dense mask (dense launches only), or null.
 template <typename T, int D, bool VARLEN>
 static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const void* o_kept, const float* stats_kept, int64_t B,
@@ -438,14 +455,7 @@ static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const v
     const FlashStatsOut st{p.d_out, lse2, delta, p.rows_padded};
     const dim3 block(kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));
-    m.n_tiles = (p.N + kFlashRows - 1) / kFlashRows;
-    // causal dense launches: a workgroup takes a long and a short tile of its head, so that all do the same work
-    m.paired = (causal && !VARLEN && m.n_tiles >= 2 && tuning().bwd_pair.load() != 0) ? 1 : 0;
-    const int64_t units = bwd_units(m);
-    const int64_t total_q = B * p.H * units, total_kv = B * H_kv * units;
-    if (total_q > 0x7FFFFFF0ll) return AHPC_ERR_BAD_SHAPE;
-    m.total_q = (int32_t)total_q; m.per_xcd_q = (int32_t)((total_q + 7) / 8);
-    m.total_kv = (int32_t)total_kv; m.per_xcd_kv = (int32_t)((total_kv + 7) / 8);
+    if (int rc = plan_bwd(m, B, H_kv, causal, VARLEN)) return rc;
     const dim3 grid_q((unsigned)(m.per_xcd_q * 8)), grid_kv((unsigned)(m.per_xcd_kv * 8));
     auto launch = [&](auto causal_c, auto masked_c) {
         constexpr bool C = decltype(causal_c)::value, M = decltype(masked_c)::value;
@@ -513,14 +523,7 @@ static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, int64_t H_kv, 
     const dim3 block(kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));
     FlashBwdParams m = p;
-    m.n_tiles = (p.N + kFlashRows - 1) / kFlashRows;
-    // causal dense launches: a workgroup takes a long and a short tile of its head, so that all do the same work
-    m.paired = (causal && !VARLEN && m.n_tiles >= 2 && tuning().bwd_pair.load() != 0) ? 1 : 0;
-    const int64_t units = bwd_units(m);
-    const int64_t total_q = B * p.H * units, total_kv = B * H_kv * units;
-    if (total_q > 0x7FFFFFF0ll) return AHPC_ERR_BAD_SHAPE;
-    m.total_q = (int32_t)total_q; m.per_xcd_q = (int32_t)((total_q + 7) / 8);
-    m.total_kv = (int32_t)total_kv; m.per_xcd_kv = (int32_t)((total_kv + 7) / 8);
+    if (int rc = plan_bwd(m, B, H_kv, causal, VARLEN)) return rc;
     const dim3 grid_q((unsigned)(m.per_xcd_q * 8)), grid_kv((unsigned)(m.per_xcd_kv * 8));
     if (causal) {
         hipLaunchKernelGGL((flash_bwd_stats_f32_mfma_kernel<D, true, VARLEN>), grid_stats, block, 0, stream, f, st);

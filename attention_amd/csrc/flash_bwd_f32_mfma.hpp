@@ -77,7 +77,7 @@ __global__ __launch_bounds__(kFlashThreads, (D == 128 ? 1 : 2)) void flash_bwd_d
     const int lane = tid & 63;
     const int col = lane & 31;
     const int half = lane >> 5;
-    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_q, p.per_xcd_q, bwd_units(p));
+    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_q, p.per_xcd_q, bwd_units(p), p.spread ? p.n_bh : 0);
     if (!work.valid) return;
     const int b = work.bh / p.H, h = work.bh - b * p.H;
     const int hk = h / p.kv_group;
@@ -93,6 +93,8 @@ __global__ __launch_bounds__(kFlashThreads, (D == 128 ? 1 : 2)) void flash_bwd_d
         base = (int64_t)b * p.stride_b + (int64_t)h * p.stride_h;
         kv_base = (int64_t)b * p.kv_stride_b + (int64_t)hk * p.kv_stride_h;
     }
+    const int n_own = VARLEN ? (L + kFlashRows - 1) / kFlashRows : p.n_tiles;  // tiles of this sequence
+    if (VARLEN && work.tile >= bwd_units(p.paired, n_own)) return;
     const float* const gq = static_cast<const float*>(p.q) + base;
     const float* const gdo = static_cast<const float*>(p.d_out) + base;
     const float* const gk = static_cast<const float*>(p.k) + kv_base;
@@ -121,10 +123,9 @@ __global__ __launch_bounds__(kFlashThreads, (D == 128 ? 1 : 2)) void flash_bwd_d
     for (int part = 0; part < 2; ++part) {
         // long tiles first: under a causal mask the late query tiles walk the most keys; a paired workgroup then takes the
         // early tile that completes its share
-        const int tile = part == 0 ? work.tile : p.n_tiles - 1 - work.tile;
+        const int tile = part == 0 ? work.tile : n_own - 1 - work.tile;
         if (part == 1 && (!p.paired || tile == work.tile)) break;
-        const int q_tile0 = (p.n_tiles - 1 - tile) * kFlashRows;
-        if (q_tile0 >= L) continue;  // ragged batches: a sequence shorter than the longest one
+        const int q_tile0 = (n_own - 1 - tile) * kFlashRows;
         if (part == 1) __syncthreads();  // every wavefront is done with the first pass's last tile
         int k_end = L;
         if (CAUSAL) k_end = (q_tile0 + kFlashRows) < L ? (q_tile0 + kFlashRows) : L;
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(kFlashThreads, (PART == 2 ? 1 : 2)) void flash_bwd_
     const int lane = tid & 63;
     const int col = lane & 31;
     const int half = lane >> 5;
-    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_kv, p.per_xcd_kv, bwd_units(p));
+    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_kv, p.per_xcd_kv, bwd_units(p), p.spread ? p.n_bh / p.kv_group : 0);
     if (!work.valid) return;
     const int heads_kv = p.H / p.kv_group;
     const int b = work.bh / heads_kv, hk = work.bh - b * heads_kv;
@@ -281,6 +282,8 @@ __global__ __launch_bounds__(kFlashThreads, (PART == 2 ? 1 : 2)) void flash_bwd_
         seq0 = p.cu_seqlens[b];
         L = p.cu_seqlens[b + 1] - seq0;
     }
+    const int n_own = VARLEN ? (L + kFlashRows - 1) / kFlashRows : p.n_tiles;  // tiles of this sequence
+    if (VARLEN && work.tile >= bwd_units(p.paired, n_own)) return;
     const int64_t kv_base = VARLEN ? (int64_t)seq0 * p.kv_stride_n + (int64_t)hk * p.kv_stride_h
                                    : (int64_t)b * p.kv_stride_b + (int64_t)hk * p.kv_stride_h;
     const float* const gk = static_cast<const float*>(p.k) + kv_base;
@@ -303,10 +306,9 @@ __global__ __launch_bounds__(kFlashThreads, (PART == 2 ? 1 : 2)) void flash_bwd_
     for (int part = 0; part < 2; ++part) {
         // under a causal mask the early key tiles see the most queries: they go first; a paired workgroup then takes the
         // late tile that completes its share
-        const int tile = part == 0 ? work.tile : p.n_tiles - 1 - work.tile;
+        const int tile = part == 0 ? work.tile : n_own - 1 - work.tile;
         if (part == 1 && (!p.paired || tile == work.tile)) break;
         const int k_tile0 = tile * kFlashRows;
-        if (k_tile0 >= L) continue;  // ragged batches: a sequence shorter than the longest one
         const int kw = k_tile0 + wave * 32;  // first key of this wavefront
         const int key = kw + col;
         f32x4 kreg[MS], vreg[kDoK ? MS : 1];
