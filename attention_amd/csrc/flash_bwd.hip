@@ -20,6 +20,7 @@
 #include "flash_bwd_mfma.hpp"
 #include "mask_pack.hpp"
 #include "flash_bwd_f32_mfma.hpp"
+#include "flash_f32_split.hpp"
 #include "tuning.hpp"
 
 namespace ahpc {
@@ -414,10 +415,10 @@ static void launch_dkv(const FlashBwdParams& m, dim3 grid, dim3 block, hipStream
 }
 
 // Launch geometry of the dQ and dK/dV kernels (tiles, pairing, the map from workgroups to tiles).
-static int plan_bwd(FlashBwdParams& m, int64_t B, int64_t H_kv, bool causal, bool ragged) {
-    m.n_tiles = (m.N + kFlashRows - 1) / kFlashRows;
+static int plan_bwd(FlashBwdParams& m, int64_t B, int64_t H_kv, bool causal, bool ragged, int rows = kFlashRows) {
+    m.n_tiles = (m.N + rows - 1) / rows;
     // causal launches: a workgroup takes a long and a short tile of its head, so that all (of a sequence) do the same work
-    m.paired = (causal && m.n_tiles >= 2 && tuning().bwd_pair.load() != 0) ? 1 : 0;
+    m.paired = (causal && rows == kFlashRows && m.n_tiles >= 2 && tuning().bwd_pair.load() != 0) ? 1 : 0;
     m.spread = ragged ? 1 : 0;
     m.n_bh = (int32_t)(B * m.H);
     const int64_t units = bwd_units(m), pairs_q = B * m.H, pairs_kv = B * H_kv;
@@ -506,7 +507,15 @@ static int launch_mfma(const FlashBwdParams& p, const PackedMask* pm, const void
     return AHPC_ERR_UNSUPPORTED_HEAD_DIM;
 }
 
-// fp32 tensors: the same three steps on the fp32 matrix instructions (flash_bwd_f32_mfma.hpp), dK and dV always in two walks
+// The tuning value bwd_split as f32_split_for takes it: 1 and 2 are the 128-row kernels' one and two walks, 3 the kernels whose
+// workgroups own 32 rows and share the walk, 0 = by shape.
+static int64_t bwd_rows_wanted() {
+    const int64_t t = tuning().bwd_split.load();
+    return t == 3 ? kSplitRows : t == 1 || t == 2 ? kFlashRows : 0;
+}
+
+// fp32 tensors: the same three steps on the fp32 matrix instructions (flash_bwd_f32_mfma.hpp), dK and dV always in two walks;
+// launches too small for those: flash_f32_split.hpp, dK and dV in one
 template <int D, bool VARLEN>
 static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, int64_t H_kv, bool causal, float* lse2, float* delta,
                               hipStream_t stream) {
@@ -518,13 +527,26 @@ static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, int64_t H_kv, 
     f.cu_seqlens = p.cu_seqlens;
     f.scale_log2 = p.scale_log2;
     f.d_real = p.d_real;
-    if (int rc = flash_plan_launch(f, B, causal, kFlashRows, tuning().flash_pair_min_tiles.load(), VARLEN)) return rc;
+    const bool split = f32_split_for(bwd_rows_wanted(), kSharedBackward, causal, VARLEN, B * p.H, p.kv_group, p.N);
+    if (int rc = split ? flash_plan_launch(f, B, causal, kSplitRows, kNeverPair, VARLEN)
+                       : flash_plan_launch(f, B, causal, kFlashRows, tuning().flash_pair_min_tiles.load(), VARLEN)) return rc;
     const FlashStatsOut st{p.d_out, lse2, delta, p.rows_padded};
-    const dim3 block(kFlashThreads);
+    const dim3 block(split ? kWave * kSplitWaves : kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));
     FlashBwdParams m = p;
-    if (int rc = plan_bwd(m, B, H_kv, causal, VARLEN)) return rc;
+    if (int rc = plan_bwd(m, B, H_kv, causal, VARLEN, split ? kSplitRows : kFlashRows)) return rc;
     const dim3 grid_q((unsigned)(m.per_xcd_q * 8)), grid_kv((unsigned)(m.per_xcd_kv * 8));
+    if (split) {
+        auto launch = [&](auto causal_c) {
+            constexpr bool C = decltype(causal_c)::value;
+            hipLaunchKernelGGL((flash_bwd_stats_f32_split_kernel<D, C, VARLEN>), grid_stats, block, 0, stream, f, st);
+            hipLaunchKernelGGL((flash_bwd_dq_f32_split_kernel<D, C, VARLEN>), grid_q, block, 0, stream, m);
+            hipLaunchKernelGGL((flash_bwd_dkv_f32_split_kernel<D, C, VARLEN>), grid_kv, block, 0, stream, m);
+        };
+        if (causal) launch(std::true_type{});
+        else launch(std::false_type{});
+        return static_cast<int>(hipGetLastError());
+    }
     if (causal) {
         hipLaunchKernelGGL((flash_bwd_stats_f32_mfma_kernel<D, true, VARLEN>), grid_stats, block, 0, stream, f, st);
         hipLaunchKernelGGL((flash_bwd_dq_f32_mfma_kernel<D, true, VARLEN>), grid_q, block, 0, stream, m);

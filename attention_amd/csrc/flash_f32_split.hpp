@@ -1,0 +1,594 @@
+// fp32 forward and backward for launches with too few 128-row tiles to fill the chip.
+//
+// The kernels of flash_fwd_f32_mfma.hpp and flash_bwd_f32_mfma.hpp give a workgroup 128 rows, 32 to a wavefront.  A small
+// launch then has a few dozen workgroups for 256 CUs, each with a long walk over the other side's tiles.  Here a workgroup
+// owns 32 rows: its four wavefronts share the WALK out (wavefront w takes tiles w, w + 4, ...), each with accumulators of
+// its own, and the four partial results meet in LDS once at the end, in a fixed order (no atomics; results do not depend on
+// which wavefront is faster).  Four times the workgroups, a quarter of the walk.
+//
+// Same products, layouts and contraction order within a tile as those kernels (see there).  The operands come straight from
+// memory: a v_mfma_f32_32x32x2_f32 takes 64 cycles, a tile's two products 4096 (d = 64), and its operands are 16 KB, so one
+// load instruction in flight per few matrix instructions keeps up and there is nothing to stage, swizzle or synchronise:
+//   rows operand   (A of the products over d)     a lane reads 16-byte pieces of tile row lane % 32
+//   columns operand (A of the products over rows)  a lane reads one float per instruction, 128 bytes of a row per half
+// Each operand is requested one product (2048 cycles at d = 64) ahead of the product that uses it, so that two or three operand
+// sets are in registers at a time; the workgroup's own 32 rows, the B operands of the products over d, are the same for all
+// its wavefronts and wait in LDS.  With that the forward at d = 64 leaves two
+// workgroups to a CU; everything else takes one with up to 512 registers and no scratch.
+// Bound: the fp32 matrix rate where the launch fills the chip (2 x 512 x 8, d = 64: 1024 wavefronts of four tiles each, 14.6 us of
+// which 7 are matrix instructions and the rest the launch, the first loads, the exchange), the length of one walk below that.
+#pragma once
+
+#include "flash_bwd_f32_mfma.hpp"
+
+namespace ahpc {
+
+constexpr int kSplitRows = 32;   // rows per workgroup
+constexpr int kSplitWaves = 4;   // wavefronts that share its walk
+constexpr int64_t kNeverPair = int64_t(1) << 40;  // flash_plan_launch: these workgroups take one block each
+
+// Which fp32 launches run here.  Times in units of one 128-row tile's whole walk on a CU of its own, n = 128-row tiles of a
+// sequence, 256 CUs that hold the 128-row kernels' workgroups one at a time (two share the matrix cores and take twice as
+// long): the 128-row form takes a round per 256 workgroups, a causal pair (a long and a short tile) (n + 1) / n of a round;
+// the grouped heads of a dK/dV workgroup are walked one after the other.  This form spreads evenly, at `kShared` times the
+// work: it reads every operand from the caches.  Measured at H = 8 to 16, d = 64 (forward / backward, us, 128-row form ->
+// this one), where the model draws its line:
+//     tiles  64 (2 x 512 x 8)     causal 38.7 -> 14.7 / 247 -> 60    not causal 38.3 -> 14.7 / 196 -> 60
+//     tiles 128 (2 x 1024 x 8)    causal 74 -> 47 / 432 -> 143       not causal 72 -> 49 / 372 -> 206
+//     tiles 256 (1 x 2048 x 16)   causal 144 -> 105 / 804 -> 434     not causal 139 -> 175 / 732 -> 751
+//     tiles 512 (2 x 2048 x 16)   causal 157 -> 206 / 923 -> 861     not causal 257 -> 341 / 1364 -> 1492
+// `rows`: 32 or 128 forces a form (the tuning values flash_rows and bwd_split), anything else = by shape.  `group`: query heads
+// per K/V head where they are walked serially (backward), 1 otherwise.
+constexpr double kSharedForward = 1.35, kSharedBackward = 1.07;
+inline bool f32_split_for(int64_t rows, double shared, bool causal, bool ragged, int64_t pairs, int64_t group, int64_t N) {
+    if (rows == kSplitRows) return true;
+    if (rows == kFlashRows || rows == kFlashWideRows) return false;
+    const int64_t n = (N + kFlashRows - 1) / kFlashRows, tiles = pairs * n;
+    if (ragged) return tiles <= 768;  // counted from the longest sequence: about half of them exist
+    auto rounds = [](int64_t workgroups) { return (double)((workgroups + 255) / 256); };
+    auto tile_form = [&](int64_t heads) {  // `heads` (sequence, head) pairs own the tiles
+        const double single = rounds(heads * n);
+        if (!causal || n == 1) return single;
+        const double paired = rounds(heads * ((n + 1) / 2)) * (double)(n + 1) / (double)n;
+        return single < paired ? single : paired;
+    };
+    const double there = group == 1 ? tile_form(pairs) : 0.5 * (tile_form(pairs) + (double)group * tile_form(pairs / group));
+    const double walk = causal ? (double)(n + 1) / (double)(2 * n) : 1.0;
+    return shared * walk * (double)tiles / 256.0 < there;
+}
+
+// Loads of one tile of 32 rows of a [rows][d] tensor, first row `t0`, rows at or beyond L as zeros (columns from d_real on: see
+// FlashParams::d_real; the callers' other operand is zero there or the result is not stored).
+template <int D> struct F32SplitTile {
+    static constexpr int MS = D / 8, MB = D / 32;
+
+    // rows operand: rows[m] = 4 floats from d = 8 m + 4 half of row t0 + col
+    __device__ static void load_rows(f32x4 (&rows)[MS], const float* base, int64_t stride, int t0, int L, int col, int half, int d_real) {
+        const int row = t0 + col;
+        const float* const src = base + (int64_t)(row < L ? row : L - 1) * stride;
+        const int last = d_real - 4;  // the last piece the row has
+#pragma unroll
+        for (int m = 0; m < MS; ++m) {
+            const int at = 8 * m + 4 * half;
+            rows[m] = *reinterpret_cast<const f32x4*>(src + (at < last ? at : last));
+        }
+        if (t0 + kF32Keys > L) {  // (uniform)
+#pragma unroll
+            for (int m = 0; m < MS; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rows[m][e] = row < L ? rows[m][e] : 0.0f;
+        }
+    }
+
+    // columns operand: cols[r][mb] = float 32 mb + col of row t0 + 8 (r / 4) + 4 half + r % 4
+    __device__ static void load_cols(float (&cols)[16][MB], const float* base, int64_t stride, int t0, int L, int col, int half, int d_real) {
+        int at[MB];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) at[mb] = 32 * mb + col < d_real ? 32 * mb + col : 0;
+        if (t0 + kF32Keys <= L) {  // (uniform)
+            const float* const tile = base + (int64_t)t0 * stride;
+            const uint32_t lane_row = (uint32_t)(4 * half) * (uint32_t)stride;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float* const src = tile + (int64_t)(8 * (r >> 2) + (r & 3)) * stride;
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) cols[r][mb] = src[lane_row + (uint32_t)at[mb]];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = t0 + 8 * (r >> 2) + 4 * half + (r & 3);
+                const float* const src = base + (int64_t)(row < L ? row : L - 1) * stride;
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) {
+                    const float x = src[at[mb]];
+                    cols[r][mb] = row < L ? x : 0.0f;
+                }
+            }
+        }
+    }
+
+    // acc += A^T B over the 32 rows of the tile: step r contracts rows 8 (r / 4) + r % 4 (half 0) and 4 further (half 1)
+    __device__ static void product_over_rows(f32x16 (&acc)[MB], const float (&cols)[16][MB], const f32x16& b) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) acc[mb] = mfma_32x32x2_f32(cols[r][mb], b[r], acc[mb]);
+    }
+
+    // c + (rows . own) over d, in two chains so that consecutive matrix instructions are independent
+    __device__ static f32x16 product_over_d(const f32x4 (&rows)[MS], const float* own, int lane, const f32x16& c) {
+        f32x16 even = c, odd;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) odd[r] = 0.0f;
+#pragma unroll
+        for (int m = 0; m < MS; m += 2) {
+            const u32x4 b0 = lds_read_b128(reinterpret_cast<const unsigned char*>(own + (m * kWave + lane) * 4));
+            const u32x4 b1 = lds_read_b128(reinterpret_cast<const unsigned char*>(own + ((m + 1) * kWave + lane) * 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                even = mfma_32x32x2_f32(rows[m][e], as_f32(b0[e]), even);
+                odd = mfma_32x32x2_f32(rows[m + 1][e], as_f32(b1[e]), odd);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) even[r] += odd[r];
+        return even;
+    }
+
+    // The workgroup's own rows as B operands in LDS, multiplied by c (zeros from d_real on): piece m of lane `lane` at
+    // own + (m * 64 + lane) * 4.  The wavefronts share the pieces out; the caller's barrier follows.
+    static constexpr int kOwnFloats = MS * kWave * 4;
+    __device__ static void put_own(float* own, const float* row_ptr, int wave, int lane, float c, int d_real) {
+#pragma unroll
+        for (int i = 0; i < MS / kSplitWaves; ++i) {
+            const int m = i * kSplitWaves + wave;
+            const int at = 8 * m + 4 * (lane >> 5);
+            const f32x4 raw = at < d_real ? *reinterpret_cast<const f32x4*>(row_ptr + at) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            *reinterpret_cast<f32x4*>(own + (m * kWave + lane) * 4) = f32x4{raw[0] * c, raw[1] * c, raw[2] * c, raw[3] * c};
+        }
+    }
+};
+
+// Partial accumulators of the workgroup's wavefronts in LDS: [wavefront][32-row block][group of 4 registers][lane] 16 bytes each.
+// Wavefront w collects register group w of every block: elements 32 mb + 8 w + 4 half .. + 3 of row `col`.
+template <int MB> struct SplitExchange {
+    static constexpr int kFloats = kSplitWaves * MB * 4 * kWave * 4;
+    __device__ static void put(float* lds, const f32x16 (&acc)[MB], int wave, int lane) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4)
+                *reinterpret_cast<f32x4*>(lds + (((wave * MB + mb) * 4 + g4) * kWave + lane) * 4) =
+                    f32x4{acc[mb][4 * g4], acc[mb][4 * g4 + 1], acc[mb][4 * g4 + 2], acc[mb][4 * g4 + 3]};
+    }
+    __device__ static f32x4 get(const float* lds, int from, int mb, int wave, int lane) {
+        return *reinterpret_cast<const f32x4*>(lds + (((from * MB + mb) * 4 + wave) * kWave + lane) * 4);
+    }
+};
+
+// Work map: flash_work_of_block over blocks of 32 query rows (flash_plan_launch with 32 rows per workgroup, never paired).
+template <int D, bool CAUSAL, bool VARLEN, bool STATS>
+__device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, const FlashStatsOut& st) {
+    typedef F32SplitTile<D> TL;
+    constexpr int MS = TL::MS, MB = TL::MB;
+    typedef SplitExchange<MB> X;
+    static_assert(TL::kOwnFloats <= X::kFloats, "the own rows and the exchange share their LDS");
+    __shared__ __attribute__((aligned(1024))) float lds[X::kFloats];
+    __shared__ float lds_m[kSplitWaves][kSplitRows], lds_l[kSplitWaves][kSplitRows], lds_part[kSplitWaves][kSplitRows];
+
+    const int wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int col = lane & 31;
+    const int half = lane >> 5;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const FlashWork work = flash_work_of_block(blockIdx.x, p);
+    if (!work.valid) return;
+    if (work.bh < 0 || work.bh >= p.n_bh || work.slot < 0 || work.slot >= flash_per_head(p)) return;
+    const int b = work.bh / p.H;
+    const int h = work.bh - b * p.H;
+    const int hk = h / p.kv_group;
+    int L;
+    int64_t base, kv_base;
+    if (VARLEN) {
+        const int s0 = p.cu_seqlens[b];
+        L = p.cu_seqlens[b + 1] - s0;
+        base = (int64_t)s0 * p.stride_n + (int64_t)h * p.stride_h;
+        kv_base = (int64_t)s0 * p.kv_stride_n + (int64_t)hk * p.kv_stride_h;
+    } else {
+        L = p.N;
+        base = (int64_t)b * p.stride_b + (int64_t)h * p.stride_h;
+        kv_base = (int64_t)b * p.kv_stride_b + (int64_t)hk * p.kv_stride_h;
+    }
+    const int n_q = VARLEN ? (L + kSplitRows - 1) / kSplitRows : p.n_qtiles;
+    if (work.slot >= n_q) return;
+    const int q0 = (n_q - 1 - work.slot) * kSplitRows;  // long walks first
+    const float* const gk = static_cast<const float*>(p.k) + kv_base;
+    const float* const gv = static_cast<const float*>(p.v) + kv_base;
+    const int64_t sn = p.stride_n, skv = p.kv_stride_n;
+    const int d_real = (p.d_real > 0 && p.d_real < D) ? p.d_real : D;
+    const int qrow = q0 + col;
+
+    int k_end = L;
+    if (CAUSAL) k_end = q0 + kSplitRows < L ? q0 + kSplitRows : L;
+    const int n_tiles = (k_end + kF32Keys - 1) / kF32Keys;
+
+    f32x4 kq[MS];
+    float vc[16][MB];
+    if (wave_u < n_tiles) TL::load_rows(kq, gk, skv, wave_u * kF32Keys, L, col, half, d_real);
+    TL::put_own(lds, static_cast<const float*>(p.q) + base + (int64_t)(qrow < L ? qrow : L - 1) * sn, wave, lane, p.scale_log2, d_real);
+    __syncthreads();
+
+    f32x16 oacc[MB], neg_m;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) neg_m[r] = 0.0f;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) oacc[mb] = neg_m;
+    float l_run = 0.0f;
+    bool first = true;
+    constexpr float kRaise = 8.0f;  // the reference maximum is raised only when exceeded by 2^8 (flash_fwd_mfma.hpp)
+
+    for (int t = wave_u; t < n_tiles; t += kSplitWaves) {
+        const int k0 = t * kF32Keys;
+        const bool more = t + kSplitWaves < n_tiles;
+        TL::load_cols(vc, gv, skv, k0, L, col, half, d_real);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x16 s = TL::product_over_d(kq, lds, lane, neg_m);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) TL::load_rows(kq, gk, skv, k0 + kSplitWaves * kF32Keys, L, col, half, d_real);
+        __builtin_amdgcn_sched_barrier(0);
+        // key of register r: k0 + 8 (r / 4) + 4 half + r % 4; visible iff key <= min(qrow, L - 1)
+        if ((k0 + kF32Keys > L) || (CAUSAL && (k0 + kF32Keys - 1 > q0))) {
+            int lim = L - 1;
+            if (CAUSAL) lim = qrow < lim ? qrow : lim;
+            lim -= k0 + 4 * half;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = (8 * (r >> 2) + (r & 3)) <= lim ? s[r] : -INFINITY;
+        }
+        float mx = max3(s[0], s[1], s[2]);
+#pragma unroll
+        for (int r = 3; r < 15; r += 2) mx = max3(mx, s[r], s[r + 1]);
+        mx = max3(mx, s[15], s[15]);
+        if (first || __builtin_amdgcn_ballot_w64(mx > kRaise) != 0) {
+            mx = halves_max(mx);  // both lanes of a query agree
+            const float delta = first ? mx : fmaxf(mx, 0.0f);
+            const float alpha = fast_exp2(-delta);
+            l_run *= alpha;
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[mb][r] *= alpha;
+            const float nm = neg_m[0] - delta;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[r] -= delta;
+                neg_m[r] = nm;
+            }
+            first = false;
+        }
+        float sum = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            s[r] = fast_exp2(s[r]);
+            sum += s[r];
+        }
+        l_run += sum;
+        TL::product_over_rows(oacc, vc, s);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();  // the own rows' LDS is the exchange's
+
+    // ---- the four partial results: (m, l) per query, the accumulators through LDS
+    {
+        const float l = halves_sum(l_run);
+        if (half == 0) {
+            lds_m[wave][col] = first ? -INFINITY : -neg_m[0];  // (a wavefront without a tile)
+            lds_l[wave][col] = l;
+        }
+        X::put(lds, oacc, wave, lane);
+    }
+    __syncthreads();
+    float m = -INFINITY, l = 0.0f, f[kSplitWaves];
+#pragma unroll
+    for (int w = 0; w < kSplitWaves; ++w) m = fmaxf(m, lds_m[w][col]);
+#pragma unroll
+    for (int w = 0; w < kSplitWaves; ++w) {
+        f[w] = m > -INFINITY ? fast_exp2(lds_m[w][col] - m) : 0.0f;
+        l = __builtin_fmaf(lds_l[w][col], f[w], l);
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    f32x4 out[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        f32x4 a = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < kSplitWaves; ++w) {
+            const f32x4 x = X::get(lds, w, mb, wave, lane);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] = __builtin_fmaf(x[e], f[w], a[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[mb][e] = a[e] * inv;
+    }
+    const int at = 8 * wave + 4 * half;  // this lane's elements of a 32-element block
+    if constexpr (STATS) {
+        float part = 0.0f;
+        if (qrow < L) {
+            const float* src = static_cast<const float*>(st.d_out) + base + (int64_t)qrow * sn + at;
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                if (32 * mb + at >= d_real) continue;  // columns the tensors do not have
+                const f32x4 w = *reinterpret_cast<const f32x4*>(src + 32 * mb);
+                part += out[mb][0] * w[0] + out[mb][1] * w[1] + out[mb][2] * w[2] + out[mb][3] * w[3];
+            }
+        }
+        part = halves_sum(part);
+        if (half == 0) lds_part[wave][col] = part;
+        __syncthreads();
+        if (wave == 0) {
+            const int64_t row0 = (int64_t)work.bh * st.rows_padded;
+            if (half == 0) {
+                const float delta = (lds_part[0][col] + lds_part[1][col]) + (lds_part[2][col] + lds_part[3][col]);
+                const bool live = qrow < L && l > 0.0f;
+                st.neg_lse2[row0 + qrow] = live ? -m - __builtin_log2f(l) : -INFINITY;
+                st.neg_delta[row0 + qrow] = live ? -delta : 0.0f;
+            }
+            // the statistics of a sequence are read up to whole 128-row tiles
+            if (q0 + kSplitRows >= L) {
+                const int end = (L + kFlashRows - 1) / kFlashRows * kFlashRows;
+                for (int row = q0 + kSplitRows + lane; row < end; row += kWave) {
+                    st.neg_lse2[row0 + row] = -INFINITY;
+                    st.neg_delta[row0 + row] = 0.0f;
+                }
+            }
+        }
+    } else if (qrow < L) {
+        float* dst = static_cast<float*>(p.o) + base + (int64_t)qrow * sn + at;
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+            if (32 * mb + at < d_real) *reinterpret_cast<f32x4*>(dst + 32 * mb) = out[mb];
+    }
+}
+
+template <int D, bool CAUSAL, bool VARLEN>
+__global__ __launch_bounds__(kWave * kSplitWaves, D > 64 ? 1 : 2) void flash_fwd_f32_split_kernel(const FlashParams p) {
+    flash_fwd_f32_split_body<D, CAUSAL, VARLEN, false>(p, FlashStatsOut{});
+}
+template <int D, bool CAUSAL, bool VARLEN>
+__global__ __launch_bounds__(kWave * kSplitWaves, D > 64 ? 1 : 2) void flash_bwd_stats_f32_split_kernel(const FlashParams p, const FlashStatsOut st) {
+    flash_fwd_f32_split_body<D, CAUSAL, VARLEN, true>(p, st);
+}
+
+// Stores the sum of the wavefronts' partial accumulators, times f, at dst_row (row `col` of the block).
+template <int MB>
+__device__ inline void split_store_sum(float* dst_row, const float* lds, int wave, int lane, float f, int d_real) {
+    const int at = 8 * wave + 4 * (lane >> 5);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        f32x4 a = SplitExchange<MB>::get(lds, 0, mb, wave, lane);
+#pragma unroll
+        for (int w = 1; w < kSplitWaves; ++w) {
+            const f32x4 x = SplitExchange<MB>::get(lds, w, mb, wave, lane);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] += x[e];
+        }
+        if (32 * mb + at < d_real) *reinterpret_cast<f32x4*>(dst_row + 32 * mb + at) = f32x4{a[0] * f, a[1] * f, a[2] * f, a[3] * f};
+    }
+}
+
+// Work map of both backward kernels: bwd_work_of_block over blocks of 32 rows (FlashBwdParams::n_tiles counts those, never paired).
+template <int D, bool CAUSAL, bool VARLEN>
+__global__ __launch_bounds__(kWave * kSplitWaves, 1) void flash_bwd_dq_f32_split_kernel(const FlashBwdParams p) {
+    typedef F32SplitTile<D> TL;
+    constexpr int MS = TL::MS, MB = TL::MB;
+    typedef SplitExchange<MB> X;
+    static_assert(2 * TL::kOwnFloats <= X::kFloats, "the own rows and the exchange share their LDS");
+    __shared__ __attribute__((aligned(1024))) float lds[X::kFloats];
+    float* const lds_do = lds + TL::kOwnFloats;
+
+    const int wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int col = lane & 31;
+    const int half = lane >> 5;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_q, p.per_xcd_q, p.n_tiles, p.spread ? p.n_bh : 0);
+    if (!work.valid) return;
+    const int b = work.bh / p.H, h = work.bh - b * p.H;
+    const int hk = h / p.kv_group;
+    int L;
+    int64_t base, kv_base;
+    if (VARLEN) {
+        const int s0 = p.cu_seqlens[b];
+        L = p.cu_seqlens[b + 1] - s0;
+        base = (int64_t)s0 * p.stride_n + (int64_t)h * p.stride_h;
+        kv_base = (int64_t)s0 * p.kv_stride_n + (int64_t)hk * p.kv_stride_h;
+    } else {
+        L = p.N;
+        base = (int64_t)b * p.stride_b + (int64_t)h * p.stride_h;
+        kv_base = (int64_t)b * p.kv_stride_b + (int64_t)hk * p.kv_stride_h;
+    }
+    const int n_q = (L + kSplitRows - 1) / kSplitRows;
+    if (work.tile >= n_q) return;
+    const int q0 = (n_q - 1 - work.tile) * kSplitRows;  // long walks first
+    const float* const gk = static_cast<const float*>(p.k) + kv_base;
+    const float* const gv = static_cast<const float*>(p.v) + kv_base;
+    const int64_t sn = p.stride_n, skv = p.kv_stride_n;
+    const int d_real = (p.d_real > 0 && p.d_real < D) ? p.d_real : D;
+    const int qrow = q0 + col;
+    int k_end = L;
+    if (CAUSAL) k_end = q0 + kSplitRows < L ? q0 + kSplitRows : L;
+    const int n_tiles = (k_end + kF32Keys - 1) / kF32Keys;
+
+    f32x4 kr[MS], vr[MS];
+    float kc[16][MB];
+    if (wave_u < n_tiles) TL::load_rows(kr, gk, skv, wave_u * kF32Keys, L, col, half, d_real);
+    const int64_t own = base + (int64_t)(qrow < L ? qrow : L - 1) * sn;
+    TL::put_own(lds, static_cast<const float*>(p.q) + own, wave, lane, p.scale_log2, d_real);
+    TL::put_own(lds_do, static_cast<const float*>(p.d_out) + own, wave, lane, 1.0f, d_real);
+    f32x16 neg_lse, neg_delta, acc[MB];
+    {
+        const int64_t stat = (int64_t)work.bh * p.rows_padded + qrow;  // qrow < rows_padded always
+        const float a = p.neg_lse2[stat], d0 = p.neg_delta[stat];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            neg_lse[r] = a;
+            neg_delta[r] = d0;
+        }
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mb][r] = 0.0f;
+
+    __syncthreads();
+    for (int t = wave_u; t < n_tiles; t += kSplitWaves) {
+        const int k0 = t * kF32Keys, k_next = k0 + kSplitWaves * kF32Keys;
+        TL::load_rows(vr, gv, skv, k0, L, col, half, d_real);
+        __builtin_amdgcn_sched_barrier(0);
+        const f32x16 s = TL::product_over_d(kr, lds, lane, neg_lse);
+        __builtin_amdgcn_sched_barrier(0);
+        TL::load_cols(kc, gk, skv, k0, L, col, half, d_real);
+        __builtin_amdgcn_sched_barrier(0);
+        const f32x16 dp = TL::product_over_d(vr, lds_do, lane, neg_delta);
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + kSplitWaves < n_tiles) TL::load_rows(kr, gk, skv, k_next, L, col, half, d_real);
+        __builtin_amdgcn_sched_barrier(0);
+        int lim = 64;
+        if ((k0 + kF32Keys > L) || (CAUSAL && (k0 + kF32Keys - 1 > q0))) {
+            lim = L - 1;
+            if (CAUSAL) lim = qrow < lim ? qrow : lim;
+            lim -= k0 + 4 * half;
+        }
+        f32x16 ds;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ds[r] = (8 * (r >> 2) + (r & 3)) <= lim ? fast_exp2(s[r]) * dp[r] : 0.0f;
+        TL::product_over_rows(acc, kc, ds);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();  // the own rows' LDS is the exchange's
+    X::put(lds, acc, wave, lane);
+    __syncthreads();
+    if (qrow < L) split_store_sum<MB>(static_cast<float*>(p.d_q) + base + (int64_t)qrow * sn, lds, wave, lane, p.scale, d_real);
+}
+
+// dK and dV of 32 keys in one walk (four products per tile).  The wavefronts share out the tiles of all query heads of the
+// group: tile i of the walk is query tile t_begin + i % n of head i / n.
+template <int D, bool CAUSAL, bool VARLEN>
+__global__ __launch_bounds__(kWave * kSplitWaves, 1) void flash_bwd_dkv_f32_split_kernel(const FlashBwdParams p) {
+    typedef F32SplitTile<D> TL;
+    constexpr int MS = TL::MS, MB = TL::MB;
+    typedef SplitExchange<MB> X;
+    static_assert(2 * TL::kOwnFloats <= X::kFloats, "the own rows and the exchange share their LDS");
+    __shared__ __attribute__((aligned(1024))) float lds[X::kFloats];
+    float* const lds_v = lds + TL::kOwnFloats;
+
+    const int wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int col = lane & 31;
+    const int half = lane >> 5;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const int heads_kv = p.H / p.kv_group;
+    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_kv, p.per_xcd_kv, p.n_tiles, p.spread ? p.n_bh / p.kv_group : 0);
+    if (!work.valid) return;
+    const int b = work.bh / heads_kv, hk = work.bh - b * heads_kv;
+    int seq0 = 0;
+    int L = p.N;
+    if (VARLEN) {
+        seq0 = p.cu_seqlens[b];
+        L = p.cu_seqlens[b + 1] - seq0;
+    }
+    const int kw = work.tile * kSplitRows;  // (under a causal mask the early keys see the most queries: they go first)
+    if (kw >= L) return;
+    const int64_t sn = p.stride_n, skv = p.kv_stride_n;
+    const int64_t kv_base = VARLEN ? (int64_t)seq0 * skv + (int64_t)hk * p.kv_stride_h : (int64_t)b * p.kv_stride_b + (int64_t)hk * p.kv_stride_h;
+    const int64_t q_base = VARLEN ? (int64_t)seq0 * sn : (int64_t)b * p.stride_b;
+    const int d_real = (p.d_real > 0 && p.d_real < D) ? p.d_real : D;
+    const int key = kw + col;
+    const int t_begin = CAUSAL ? kw / kF32Keys : 0;
+    const int n_walk = (L + kF32Keys - 1) / kF32Keys - t_begin;  // query tiles per head
+    const int n_items = n_walk * p.kv_group;
+
+    const float *gq = nullptr, *gdo = nullptr, *lse2 = nullptr, *delta = nullptr;  // of the head the item in hand belongs to
+    auto item = [&](int i) {  // selects item i, returns its first query
+        const int g = i / n_walk;
+        const int h = hk * p.kv_group + g;
+        const int64_t base = q_base + (int64_t)h * p.stride_h;
+        gq = static_cast<const float*>(p.q) + base;
+        gdo = static_cast<const float*>(p.d_out) + base;
+        lse2 = p.neg_lse2 + ((int64_t)b * p.H + h) * p.rows_padded;
+        delta = p.neg_delta + ((int64_t)b * p.H + h) * p.rows_padded;
+        return (t_begin + i - g * n_walk) * kF32Keys;
+    };
+    // -lse2 or -delta of the tile's queries: register r belongs to query i0 + 8 (r / 4) + 4 half + r % 4
+    auto load_stats = [&](f32x16& out, const float* src, int i0) {
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+            const f32x4 w = *reinterpret_cast<const f32x4*>(src + i0 + 8 * g4 + 4 * half);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[4 * g4 + e] = w[e];
+        }
+    };
+
+    f32x4 qr[MS], dor[MS];
+    float qc[16][MB], doc[16][MB];
+    f32x16 nl, nd;
+    int i0 = 0;
+    if (wave_u < n_items) {
+        i0 = item(wave_u);
+        load_stats(nl, lse2, i0);
+        TL::load_rows(qr, gq, sn, i0, L, col, half, d_real);
+    }
+    const int64_t own = kv_base + (int64_t)(key < L ? key : L - 1) * skv;
+    TL::put_own(lds, static_cast<const float*>(p.k) + own, wave, lane, p.scale_log2, d_real);
+    TL::put_own(lds_v, static_cast<const float*>(p.v) + own, wave, lane, 1.0f, d_real);
+    f32x16 acc_k[MB], acc_v[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc_k[mb][r] = acc_v[mb][r] = 0.0f;
+
+    __syncthreads();
+    for (int i = wave_u; i < n_items; i += kSplitWaves) {
+        const int cur = i0;
+        load_stats(nd, delta, cur);
+        TL::load_rows(dor, gdo, sn, cur, L, col, half, d_real);
+        __builtin_amdgcn_sched_barrier(0);
+        const f32x16 s = TL::product_over_d(qr, lds, lane, nl);
+        __builtin_amdgcn_sched_barrier(0);
+        TL::load_cols(doc, gdo, sn, cur, L, col, half, d_real);
+        __builtin_amdgcn_sched_barrier(0);
+        const f32x16 dp = TL::product_over_d(dor, lds_v, lane, nd);
+        __builtin_amdgcn_sched_barrier(0);
+        TL::load_cols(qc, gq, sn, cur, L, col, half, d_real);
+        __builtin_amdgcn_sched_barrier(0);
+        // query row of register r: cur + 8 (r / 4) + 4 half + r % 4; rows beyond the sequence carry -lse2 = -inf: weight 0
+        int first_row = -64;
+        if (CAUSAL && cur < kw + 31) first_row = key - cur - 4 * half;
+        f32x16 pw, ds;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            pw[r] = (8 * (r >> 2) + (r & 3)) >= first_row ? fast_exp2(s[r]) : 0.0f;
+            ds[r] = pw[r] * dp[r];
+        }
+        TL::product_over_rows(acc_v, doc, pw);
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + kSplitWaves < n_items) {
+            i0 = item(i + kSplitWaves);
+            load_stats(nl, lse2, i0);
+            TL::load_rows(qr, gq, sn, i0, L, col, half, d_real);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        TL::product_over_rows(acc_k, qc, ds);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();  // the own rows' LDS is the exchange's
+    X::put(lds, acc_k, wave, lane);
+    __syncthreads();
+    if (key < L) split_store_sum<MB>(static_cast<float*>(p.d_k) + kv_base + (int64_t)key * skv, lds, wave, lane, p.scale, d_real);
+    __syncthreads();
+    X::put(lds, acc_v, wave, lane);
+    __syncthreads();
+    if (key < L) split_store_sum<MB>(static_cast<float*>(p.d_v) + kv_base + (int64_t)key * skv, lds, wave, lane, 1.0f, d_real);
+}
+
+}  // namespace ahpc

@@ -12,6 +12,7 @@
 #include "flash_fwd_wide.hpp"
 #include "mask_pack.hpp"
 #include "flash_fwd_f32_mfma.hpp"
+#include "flash_f32_split.hpp"
 #include "tuning.hpp"
 
 namespace ahpc {
@@ -387,8 +388,22 @@ static bool f32_mfma_eligible(int dtype, int64_t d, const void* q, const void* k
     return sq.n >= d && skv.n >= d && skv.n < (int64_t(1) << 24);
 }
 
+// Blocks of 32 query rows, walk shared by the workgroup's wavefronts (flash_f32_split.hpp).
+template <int D, bool VARLEN>
+static int launch_f32_split(FlashParams p, int64_t B, bool causal, hipStream_t stream) {
+    if (int rc = flash_plan_launch(p, B, causal, kSplitRows, kNeverPair, VARLEN)) return rc;
+    dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(kWave * kSplitWaves);
+    if (causal) hipLaunchKernelGGL((flash_fwd_f32_split_kernel<D, true, VARLEN>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((flash_fwd_f32_split_kernel<D, false, VARLEN>), grid, block, 0, stream, p);
+    return static_cast<int>(hipGetLastError());
+}
+
 template <bool VARLEN, bool MASKED>
 static int launch_f32_mfma(FlashParams p, int64_t B, int d, bool causal, hipStream_t stream) {
+    if constexpr (!MASKED) {
+        if (d <= 128 && f32_split_for(tuning().flash_rows.load(), kSharedForward, causal, VARLEN, B * p.H, 1, p.N))
+            return d == 128 ? launch_f32_split<128, VARLEN>(p, B, causal, stream) : launch_f32_split<64, VARLEN>(p, B, causal, stream);
+    }
     if (int rc = flash_plan_launch(p, B, causal, kFlashRows, tuning().flash_pair_min_tiles.load(), VARLEN)) return rc;
     dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(kFlashThreads);
     if (d == 256) {  // (one workgroup per CU: registers and LDS of twice the size)

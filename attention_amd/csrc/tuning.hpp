@@ -23,7 +23,8 @@ struct Tuning {
     // matrix-core kernels only.  (AHPC_DECODE_MFMA_MIN_GROUP)
     std::atomic<int64_t> decode_matrix_min_group;
     // backward: dK and dV in one walk over the query tiles (1), in two (2), or the launcher's choice (0, the default:
-    // one walk up to d = 128, two at d = 256).  (AHPC_BWD_SPLIT)
+    // by shape: one walk up to d = 128, two at d = 256, and for fp32 launches that leave CUs idle the kernels whose
+    // workgroups own 32 rows and share the walk, which 3 asks for).  (AHPC_BWD_SPLIT)
     std::atomic<int64_t> bwd_split;
     // forward with a dense mask on the matrix-core kernel: 1 (default) = the mask is packed to one bit per element in
     // front of the launch, into device memory the library keeps; 0 = the kernel reads the caller's fp32 mask in place
@@ -33,8 +34,8 @@ struct Tuning {
     // head each (equal work for all), 0 = one tile per workgroup, long tiles first.  (AHPC_BWD_PAIR)
     std::atomic<int64_t> bwd_pair;
     // forward on the 16-bit matrix-core kernel: query rows per workgroup, 128 (4 wavefronts, two workgroups per CU) or
-    // 256 (8 wavefronts, one workgroup per CU: one stream of K/V tiles feeds twice the rows); 0 (default) = by shape.
-    // (AHPC_FLASH_ROWS)
+    // 256 (8 wavefronts, one workgroup per CU: one stream of K/V tiles feeds twice the rows); fp32 forward: 128, or 32 (the
+    // wavefronts of a workgroup share the walk over the keys); 0 (default) = by shape.  (AHPC_FLASH_ROWS)
     std::atomic<int64_t> flash_rows;
     // KV block pool (host class): 1 (default) = slabs are address ranges that grow in place where the device has virtual
     // memory management; 0 = plain allocations that grow by reallocation and a device copy.  Read when a pool is
