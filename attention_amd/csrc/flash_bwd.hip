@@ -452,7 +452,7 @@ static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const v
         m.mask_bits_t = pm->bits_t;
         m.mask_tiles = pm->tiles;
     }
-    if (int rc = flash_plan_launch(f, B, causal, kFlashRows, tuning().flash_pair_min_tiles.load(), VARLEN)) return rc;
+    if (int rc = flash_plan_launch(f, B, causal, kFlashRows, rows_128_pair_threshold(D, false, VARLEN, B, f), VARLEN)) return rc;
     const FlashStatsOut st{p.d_out, lse2, delta, p.rows_padded};
     const dim3 block(kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));
@@ -529,7 +529,7 @@ static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, int64_t H_kv, 
     f.d_real = p.d_real;
     const bool split = f32_split_for(bwd_rows_wanted(), kSharedBackward, causal, VARLEN, B * p.H, p.kv_group, p.N);
     if (int rc = split ? flash_plan_launch(f, B, causal, kSplitRows, kNeverPair, VARLEN)
-                       : flash_plan_launch(f, B, causal, kFlashRows, tuning().flash_pair_min_tiles.load(), VARLEN)) return rc;
+                       : flash_plan_launch(f, B, causal, kFlashRows, rows_128_pair_threshold(D, true, VARLEN, B, f), VARLEN)) return rc;
     const FlashStatsOut st{p.d_out, lse2, delta, p.rows_padded};
     const dim3 block(split ? kWave * kSplitWaves : kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));

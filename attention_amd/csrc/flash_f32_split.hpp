@@ -25,7 +25,6 @@ namespace ahpc {
 
 constexpr int kSplitRows = 32;   // rows per workgroup
 constexpr int kSplitWaves = 4;   // wavefronts that share its walk
-constexpr int64_t kNeverPair = int64_t(1) << 40;  // flash_plan_launch: these workgroups take one block each
 
 // Which fp32 launches run here.  Times in units of one 128-row tile's whole walk on a CU of its own, n = 128-row tiles of a
 // sequence, 256 CUs that hold the 128-row kernels' workgroups one at a time (two share the matrix cores and take twice as

@@ -162,15 +162,23 @@ static int dispatch_simple(int dtype, const SimpleParams& p, int64_t B, hipStrea
 // ---------------------------------------------------------------------------------------------
 // Query rows per workgroup of the 16-bit forward without a mask: 128 (flash_fwd_mfma.hpp, two workgroups per CU) or 256
 // (flash_fwd_wide.hpp, one persistent workgroup per CU: dense launches at d = 64 and 128).  The tuning value when it
-// names one, else by shape.  Timed on MI355X over dense shapes from 1x256x32 to 1x32768x32: 256 rows is 3-8 % faster at
-// d = 128 from 2048 tokens on once every CU gets a workgroup, and 4-30 % slower on shorter sequences, smaller launches
-// and at d = 64 (where three 128-row workgroups share a CU).
-static int flash_rows_for(int D, bool varlen, int64_t B, int64_t N, int64_t H) {
+// names one, else by shape: d = 128 from 2048 tokens on (256 rows is 4-30 % slower on shorter sequences and at d = 64, where
+// three 128-row workgroups share a CU), where its workgroups - causal launches: pairs of tiles - fill their rounds of 256.
+// It is then 3-8 % faster; a round that is three quarters empty costs more than that.  Measured at N = 4096, us, workgroups
+// of 256 rows and their share of full rounds, 128 rows -> 256 rows (paired where causal):
+//   causal      128 (0.50) 77.9 -> 95.6     160 (0.63) 103.8 -> 97.9   192 (0.75) 110.6 -> 102.8   256 (1.0) 128.6 -> 122.9
+//               320 (0.63) 180.4 -> 210.2   384 (0.75) 200.3 -> 208.9  448 (0.88) 232.0 -> 222.3   640 (0.83) 329.7 -> 335.3
+//   not causal  320 (0.63) 178.9 -> 194.7   384 (0.75) 186.9 -> 195.6  448 (0.88) 224.8 -> 206.8   640 (0.83) 301.0 -> 304.7
+// (within the first round the 128-row form has CUs with one and CUs with two workgroups, which is why 160 pairs suffice there)
+static int flash_rows_for(int D, bool varlen, bool causal, int64_t B, int64_t N, int64_t H) {
     if (D == 256 || varlen) return kFlashRows;
     const int64_t t = tuning().flash_rows.load();
     if (t == kFlashRows || t == kFlashWideRows) return (int)t;
     if (D != 128 || N < 2048) return kFlashRows;
-    return B * H * ((N + kFlashWideRows - 1) / kFlashWideRows) >= 256 ? kFlashWideRows : kFlashRows;
+    const int64_t n = (N + kFlashWideRows - 1) / kFlashWideRows;
+    const int64_t workgroups = B * H * (causal ? (n + 1) / 2 : n), rounds = (workgroups + 255) / 256;
+    if (rounds == 1) return workgroups >= (causal ? 160 : 256) ? kFlashWideRows : kFlashRows;
+    return workgroups * 100 >= rounds * 256 * 84 ? kFlashWideRows : kFlashRows;
 }
 
 // Workgroups of a persistent launch: one per CU, a multiple of 8 (a workgroup's block ids then all map to the XCD it
@@ -194,15 +202,15 @@ static int persistent_grid(int n_block_ids) {
 template <typename T, int D, bool VARLEN>
 static int launch_mfma(FlashParams p, int64_t B, bool causal, hipStream_t stream) {
     if constexpr (D != 256 && !VARLEN) {
-        if (flash_rows_for(D, VARLEN, B, p.N, p.H) == kFlashWideRows) {
-            if (int rc = flash_plan_launch(p, B, causal, kFlashWideRows, tuning().flash_pair_min_tiles.load(), false)) return rc;
+        if (flash_rows_for(D, VARLEN, causal, B, p.N, p.H) == kFlashWideRows) {
+            if (int rc = flash_plan_launch(p, B, causal, kFlashWideRows, pair_threshold(true), false)) return rc;
             dim3 grid((unsigned)persistent_grid(p.n_block_ids)), block(64 * kFlashWideWaves);
             if (causal) hipLaunchKernelGGL((flash_fwd_wide_kernel<T, D, true>), grid, block, 0, stream, p);
             else hipLaunchKernelGGL((flash_fwd_wide_kernel<T, D, false>), grid, block, 0, stream, p);
             return static_cast<int>(hipGetLastError());
         }
     }
-    if (int rc = flash_plan_launch(p, B, causal, kFlashRows, tuning().flash_pair_min_tiles.load(), VARLEN)) return rc;
+    if (int rc = flash_plan_launch(p, B, causal, kFlashRows, rows_128_pair_threshold(D, false, VARLEN, B, p), VARLEN)) return rc;
     dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(kFlashThreads);
     if (causal) hipLaunchKernelGGL((flash_fwd_mfma_kernel<T, D, true, VARLEN>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((flash_fwd_mfma_kernel<T, D, false, VARLEN>), grid, block, 0, stream, p);
@@ -211,7 +219,7 @@ static int launch_mfma(FlashParams p, int64_t B, bool causal, hipStream_t stream
 
 template <typename T, int D, int MASK>
 static int launch_mfma_masked(FlashParams p, int64_t B, bool causal, hipStream_t stream) {
-    if (int rc = flash_plan_launch(p, B, causal, kFlashRows, tuning().flash_pair_min_tiles.load(), false)) return rc;
+    if (int rc = flash_plan_launch(p, B, causal, kFlashRows, rows_128_pair_threshold(D, false, false, B, p), false)) return rc;
     dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(kFlashThreads);
     if (causal) hipLaunchKernelGGL((flash_fwd_mfma_masked_kernel<T, D, true, MASK>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((flash_fwd_mfma_masked_kernel<T, D, false, MASK>), grid, block, 0, stream, p);
@@ -404,7 +412,7 @@ static int launch_f32_mfma(FlashParams p, int64_t B, int d, bool causal, hipStre
         if (d <= 128 && f32_split_for(tuning().flash_rows.load(), kSharedForward, causal, VARLEN, B * p.H, 1, p.N))
             return d == 128 ? launch_f32_split<128, VARLEN>(p, B, causal, stream) : launch_f32_split<64, VARLEN>(p, B, causal, stream);
     }
-    if (int rc = flash_plan_launch(p, B, causal, kFlashRows, tuning().flash_pair_min_tiles.load(), VARLEN)) return rc;
+    if (int rc = flash_plan_launch(p, B, causal, kFlashRows, rows_128_pair_threshold(d, true, VARLEN, B, p), VARLEN)) return rc;
     dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(kFlashThreads);
     if (d == 256) {  // (one workgroup per CU: registers and LDS of twice the size)
         if (causal) hipLaunchKernelGGL((flash_fwd_f32_mfma_kernel<256, true, VARLEN, MASKED>), grid, block, 0, stream, p);

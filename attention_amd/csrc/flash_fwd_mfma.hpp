@@ -42,6 +42,7 @@
 #include <cstdlib>
 
 #include "ahpc_device.hpp"
+#include "tuning.hpp"
 
 namespace ahpc {
 
@@ -710,6 +711,32 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
     }
 }
 
+// Whether a causal dense launch of the 128-row kernels pairs a late query tile with an early one in a workgroup (every
+// workgroup then has the same walk, (n + 1) / n times the longest single one for n tiles of a sequence), by shape.  Up to 256
+// tiles every tile has a CU of its own and single ones are done first; from about 350 on CUs get two, and where ids land two
+// long walks meet on one CU.  Measured, single -> paired, us:
+//   fp32 (MFMA-bound from the first workgroup)   384 tiles (2 x 1024 x 24, d = 64) 131 -> 86    512 (16 x 256 x 16) 39 -> 35
+//   16-bit, d = 128    256 (1 x 2048 x 16) 37.8 -> 42.7    384 (2 x 2048 x 12) 49.6 -> 43.5    512 (16 x 256 x 16) 17.6 -> 19.4
+//   16-bit, d = 256    256 (1 x 2048 x 16) 91.6 -> 102     384 (2 x 1024 x 24) 79.9 -> 64.2    512 (16 x 256 x 16) 43.6 -> 40.5
+//   16-bit, d = 64 (three workgroups to a CU even out by themselves)    512 (4 x 1024 x 16) 18.8 -> 19.1    768 (3 x 1024 x 32) 27.2 -> 24.7
+// Just above a full round of pairs (512 for two workgroups per CU) single tiles fill the second round better: d = 128,
+// 2048 tokens x 72 heads (576 pairs) 106.5 -> 95.5 us.
+inline bool flash_pair_by_shape(int D, bool f32, int64_t seq_heads, int64_t n) {
+    const int64_t tiles = seq_heads * n, pairs = seq_heads * ((n + 1) / 2);
+    if (n < 2) return false;
+    if (f32) return tiles >= 352;
+    if (D == 128 && pairs > 512 && pairs <= 620) return false;
+    if (tiles >= 1024) return true;
+    if (D == 64) return tiles >= 640 || (tiles >= 448 && n >= 16);
+    return tiles >= 352 && n >= 4;
+}
+
+// The threshold the launchers of the 128-row kernels hand to flash_plan_launch (p.N and p.H are set).
+inline int64_t rows_128_pair_threshold(int D, bool f32, bool ragged, int64_t B, const FlashParams& p) {
+    if (ragged) return tuning().flash_pair_min_tiles.load();
+    return pair_threshold(flash_pair_by_shape(D, f32, B * p.H, (p.N + kFlashRows - 1) / kFlashRows));
+}
+
 // Fills the launch geometry of the MFMA kernel (query tiles, pairing, workgroup count) from N, H and the batch size already in `p`.  Shared by the launcher and by the host-side dump
 // of the workgroup map.
 inline int flash_plan_launch(FlashParams& p, int64_t B, bool causal, int rows_per_workgroup = kFlashRows, int64_t pair_min_tiles = 1024,
@@ -717,9 +744,8 @@ inline int flash_plan_launch(FlashParams& p, int64_t B, bool causal, int rows_pe
     p.n_qtiles = (p.N + rows_per_workgroup - 1) / rows_per_workgroup;
     int64_t total = B * p.H * (int64_t)p.n_qtiles;
     if (total > 0x7FFFFFF0ll) return AHPC_ERR_BAD_SHAPE;
-    // Causal launches with enough workgroups to fill the chip twice over pair a late query tile with an
-    // early one, so that every workgroup walks the same number of key tiles
-    // (1024 tiles = two rounds of two workgroups on each of 256 CUs).
+    // Causal launches of at least pair_min_tiles tiles pair a late query tile with an early one, so that every workgroup
+    // walks the same number of key tiles.
     p.paired = (causal && p.n_qtiles >= 2 && total * rows_per_workgroup >= pair_min_tiles * kFlashRows) ? 1 : 0;
     if (p.paired) total = B * p.H * (int64_t)((p.n_qtiles + 1) / 2);
     p.total_blocks = (int32_t)total;

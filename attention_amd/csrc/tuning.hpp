@@ -10,7 +10,7 @@ namespace ahpc {
 
 struct Tuning {
     // forward, causal: a workgroup takes a late query tile and then an early one once the launch has at least
-    // this many query tiles (AHPC_FLASH_PAIR_MIN, default 1024: two rounds of two workgroups on each of 256 CUs)
+    // this many query tiles (AHPC_FLASH_PAIR_MIN; the default, 1024, leaves dense launches to their shape)
     std::atomic<int64_t> flash_pair_min_tiles;
     // decode: wavefronts per workgroup, 1..8 (AHPC_DECODE_WAVES, default 0 = the launcher's choice)
     std::atomic<int64_t> decode_waves;
@@ -45,5 +45,13 @@ struct Tuning {
 };
 
 Tuning& tuning();
+
+// Thresholds of query tiles for flash_plan_launch.
+constexpr int64_t kPairDefault = 1024, kAlwaysPair = 1, kNeverPair = int64_t(1) << 40;
+// The threshold of a dense launch: the tuning value when it was set, else what the launch's shape asks for.
+inline int64_t pair_threshold(bool paired_by_shape) {
+    const int64_t t = tuning().flash_pair_min_tiles.load();
+    return t != kPairDefault ? t : paired_by_shape ? kAlwaysPair : kNeverPair;
+}
 
 }  // namespace ahpc

@@ -79,7 +79,7 @@ def where(request):
         w = Gpu(request.getfixturevalue("gpu"))
     else:
         w = Executor()
-    before = {n: w.hip.get_tuning(n) for n in ("flash_rows", "bwd_split")}
+    before = {n: w.hip.get_tuning(n) for n in ("flash_rows", "bwd_split", "flash_pair_min_tiles")}
     yield w
     for n, v in before.items():
         w.hip.set_tuning(n, v)
@@ -90,6 +90,7 @@ def where(request):
 def force(where, rows):
     where.hip.set_tuning("flash_rows", rows)
     where.hip.set_tuning("bwd_split", 3 if rows == 32 else 1)
+    where.hip.set_tuning("flash_pair_min_tiles", 1)  # (128 rows: causal launches of two tiles and more take them in pairs)
 
 
 def check(got, want, dtype):
