@@ -375,15 +375,16 @@ __global__ __launch_bounds__(kFlashThreads, (D > 128 ? 1 : 2)) void flash_bwd_dq
 }
 
 // grid: 8 * per_xcd_kv workgroups, see bwd_work_of_block
-// PART: 0 = dK and dV in one walk over the query tiles (four products per tile; at d = 128 that is 324 registers, one
-// wavefront per SIMD), 1 = dV only (S and dV: two products, V and dO.V never touched), 2 = dK only (S, dP, dK).  The
+// PART: 0 = dK and dV in one walk over the query tiles (four products per tile; at d = 128 that is 400 registers, one
+// wavefront per SIMD; at d = 64 232, and bounding the kernel to 256 for two workgroups per CU took it from 336 to 254 us at
+// 8 x 2048 x 16, from 112 to 83 us under a causal mask at 4 x 2048 x 16), 1 = dV only (S and dV: two products, V and dO.V never touched), 2 = dK only (S, dP, dK).  The
 // two partial walks execute five products between them but each fits two wavefronts per SIMD, which hide each
 // other's softmax arithmetic and LDS waits: 5 % fewer cycles at d = 128, and still the slower way on inputs that hold
 // the board at its power limit, where four products beat five (the launcher picks).  The one walk overlaps its own
 // vector arithmetic with its matrix products by pipelining the two blocks of a tile (see compute_tile).
 // MASKED: as in the dQ kernel, with the transposed packed mask (the lane's key, 64 queries per word).
 template <typename T, int D, bool CAUSAL, bool VARLEN, int PART, bool MASKED = false>
-__global__ __launch_bounds__(kFlashThreads, (PART == 0 || D > 128 ? 1 : 2)) void flash_bwd_dkv_mfma_kernel(const FlashBwdParams p) {
+__global__ __launch_bounds__(kFlashThreads, ((PART == 0 && D > 64) || D > 128 ? 1 : 2)) void flash_bwd_dkv_mfma_kernel(const FlashBwdParams p) {
     static_assert(!(MASKED && VARLEN), "the mask belongs to dense launches");
     constexpr bool kDoK = PART != 1, kDoV = PART != 2;
     typedef FlashTile<D> TL;
