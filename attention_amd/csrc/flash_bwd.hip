@@ -448,6 +448,7 @@ static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const v
     if (pm) {
         f.mask_bits = pm->bits;
         f.mask_kt = pm->tiles;
+        f.mask_live = pm->live;
         m.mask_bits = pm->bits;
         m.mask_bits_t = pm->bits_t;
         m.mask_tiles = pm->tiles;

@@ -243,6 +243,7 @@ static int dispatch_mfma_masked(const FlashParams& p, int64_t B, int d, bool cau
 // With bits_t given the same pass also writes the transposed layout the backward's dK/dV kernels read: word
 // [(b * n_rb + query block) * N + key] holds the block's 64 queries, bit r set = mask[b][64 * block + r][key] != 0
 // (lane = key collects its wavefront's 16 bits of that word from the values it loads).
+// live: one byte per wavefront's share of a tile, whether anything of it stays (PackedMask::live).
 // Bound by the read of the mask, hence 16 rows per wavefront and no condition around a load (rows and keys behind the end
 // re-read the last ones): all 16 are in flight together, and a launch has four times the wavefronts of one that takes 64 rows
 // in turn with each load under its condition.  Mask [4,1001,1001]: 30.8 -> 6.1 us (16 MB).
@@ -250,7 +251,8 @@ constexpr int kMaskPackThreads = 256;
 constexpr int kMaskPackRows = 64 / (kMaskPackThreads / kWave);  // queries per wavefront
 template <bool TRANSPOSED>
 __global__ __launch_bounds__(kMaskPackThreads) void flash_mask_pack_kernel(const float* __restrict__ mask, uint64_t* __restrict__ bits,
-                                                                            uint64_t* __restrict__ bits_t, int N, int n_kt, int n_rb) {
+                                                                            uint64_t* __restrict__ bits_t, uint32_t* __restrict__ live,
+                                                                            int N, int n_kt, int n_rb) {
     static_assert(kMaskPackRows == 16, "a wavefront's share of a transposed word is stored as a uint16");
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
@@ -267,23 +269,25 @@ __global__ __launch_bounds__(kMaskPackThreads) void flash_mask_pack_kernel(const
         const int row = row0 + r < N ? row0 + r : N - 1;
         m[r] = __builtin_nontemporal_load(src + (int64_t)row * N);  // read once
     }
-    uint64_t mine = 0;
+    uint64_t mine = 0, any = 0;
     uint32_t mine_t = 0;
 #pragma unroll
     for (int r = 0; r < kMaskPackRows; ++r) {
         const bool keep = row0 + r < N && key < N && m[r] != 0.0f;
         const uint64_t word = __builtin_amdgcn_ballot_w64(keep);
         if (lane == r) mine = word;
+        any |= word;
         if constexpr (TRANSPOSED) mine_t |= (uint32_t)keep << r;
     }
     if (lane < kMaskPackRows && row0 + lane < N) bits[((int64_t)b * n_kt + kt) * N + row0 + lane] = mine;
+    if (lane == 0) reinterpret_cast<uint8_t*>(live + ((int64_t)b * n_rb + rb) * n_kt + kt)[wave] = any != 0 ? 1 : 0;
     if constexpr (TRANSPOSED) {
         if (key < N) reinterpret_cast<uint16_t*>(bits_t + ((int64_t)b * n_rb + rb) * N + key)[wave] = (uint16_t)mine_t;
     }
 }
 
 // The packed copy of a mask lives in device memory that the library owns: one buffer per device, grown on demand and kept
-// until the process ends (B * N * ceil(N / 64) * 8 bytes per layout: an eighth of a byte per mask element).  Calls on one
+// until the process ends (B * N * ceil(N / 64) * 8 bytes per layout, an eighth of a byte per mask element, and a word per 64 x 64 tile).  Calls on one
 // device share it: `done` is recorded behind the last launch that reads it, and the next call's stream waits for it
 // before the buffer is overwritten; the mutex covers the whole of that.
 struct MaskScratch {
@@ -311,8 +315,9 @@ int with_packed_mask(const float* mask, int64_t B, int64_t N, bool with_transpos
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return AHPC_OK;
     const int64_t n_kt = (N + 63) / 64, n_rb = (N + 63) / 64;
     const size_t one = (size_t)B * (size_t)n_kt * (size_t)N * sizeof(uint64_t);
-    const size_t need = with_transposed ? 2 * one : one;
-    if (need > kMaskScratchLimit) return AHPC_OK;
+    const size_t bits_bytes = with_transposed ? 2 * one : one;
+    if (bits_bytes > kMaskScratchLimit) return AHPC_OK;
+    const size_t need = bits_bytes + (size_t)B * (size_t)n_rb * (size_t)n_kt * sizeof(uint32_t);
     MaskScratch& sc = g_mask_scratch[dev];
     std::lock_guard<std::mutex> lock(sc.mu);
     if (!sc.done && hipEventCreateWithFlags(&sc.done, hipEventDisableTiming) != hipSuccess) {
@@ -337,13 +342,14 @@ int with_packed_mask(const float* mask, int64_t B, int64_t N, bool with_transpos
     PackedMask pm{};
     pm.bits = static_cast<const uint64_t*>(sc.ptr);
     pm.bits_t = with_transposed ? pm.bits + one / sizeof(uint64_t) : nullptr;
+    pm.live = reinterpret_cast<const uint32_t*>(static_cast<const unsigned char*>(sc.ptr) + bits_bytes);
     pm.tiles = (int32_t)n_kt;
     if (with_transposed)
         hipLaunchKernelGGL(flash_mask_pack_kernel<true>, dim3((unsigned)blocks), dim3(kMaskPackThreads), 0, stream, mask,
-                           const_cast<uint64_t*>(pm.bits), const_cast<uint64_t*>(pm.bits_t), (int)N, (int)n_kt, (int)n_rb);
+                           const_cast<uint64_t*>(pm.bits), const_cast<uint64_t*>(pm.bits_t), const_cast<uint32_t*>(pm.live), (int)N, (int)n_kt, (int)n_rb);
     else
         hipLaunchKernelGGL(flash_mask_pack_kernel<false>, dim3((unsigned)blocks), dim3(kMaskPackThreads), 0, stream, mask,
-                           const_cast<uint64_t*>(pm.bits), nullptr, (int)N, (int)n_kt, (int)n_rb);
+                           const_cast<uint64_t*>(pm.bits), nullptr, const_cast<uint32_t*>(pm.live), (int)N, (int)n_kt, (int)n_rb);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return static_cast<int>(e);
     *launched = true;
     const int rc = launch_on_bits(pm);
@@ -359,6 +365,7 @@ static int forward_on_packed_mask(FlashParams p, const float* mask, int64_t B, h
         p.mask = nullptr;
         p.mask_bits = pm.bits;
         p.mask_kt = pm.tiles;
+        p.mask_live = pm.live;
         return launch_on_bits(p);
     });
 }

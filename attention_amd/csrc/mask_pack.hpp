@@ -12,9 +12,12 @@ namespace ahpc {
 //   bits   [(b * tiles + key tile) * N + query]    the tile's 64 keys of one query   (bit j = key 64 * tile + j stays)
 //   bits_t [(b * tiles + query block) * N + key]   the block's 64 queries of one key (bit r = query 64 * block + r sees the key);
 //          null unless asked for
+//   live   [(b * tiles + query block) * tiles + key tile] byte w: the tile's keys and queries 16 * w .. 16 * w + 15 of the
+//          block share a pair that stays (0: a kernel may pass the tile by for them)
 struct PackedMask {
     const uint64_t* bits;
     const uint64_t* bits_t;
+    const uint32_t* live;
     int32_t tiles;  // ceil(N / 64)
 };
 
