@@ -41,6 +41,8 @@ def block_mask(B, N, share, seed):
     (O.F16, 2, 577, 2, 1, 64, False, 0.3), (O.BF16, 2, 577, 2, 1, 64, False, 0.3), (O.BF16, 2, 450, 1, 1, 128, True, 0.4),
     (O.F16, 1, 300, 2, 2, 96, False, 0.0), (O.F16, 1, 4100, 1, 1, 64, False, 0.01), (O.BF16, 1, 200, 1, 1, 256, False, 0.5)])
 def test_tiles_without_a_visible_pair(where, dtype, B, N, H, H_kv, d, causal, share):
+    if N > 4096 and isinstance(where, Executor):
+        pytest.skip("more tiles than one window: minutes on the executor")
     mask = block_mask(B, N, share, N + d)
     q = O.round_to(O.fill_normal((B, N, H, d), 61, 1), dtype)
     k, v = (O.round_to(O.fill_normal((B, N, H_kv, d), 61, t), dtype) for t in (2, 3))
