@@ -199,6 +199,23 @@ static int persistent_grid(int n_block_ids) {
     return n_block_ids < n ? n_block_ids : n;
 }
 
+// Walks over the keys per workgroup of the 128-row form (flash_fwd_two_walks_kernel).  A launch of at most one 128-row tile per
+// CU lasts as long as its longest walk, with one wavefront per SIMD; two sets of wavefronts that share the walk bring a second
+// one.  That costs 2 to 3 us at the end (the exchange), so the walk has to have some length, and a CU holds one such workgroup,
+// so a second round loses what the first gained, except behind long causal walks, whose second round is the short tiles.
+// Measured, bf16, us, one walk -> two, by tiles of the launch:
+//   d = 128 causal   N=400   64 tiles 11.4 -> 12.4   N=777  224: 18.6 -> 17.6   336: 22.9 -> 28.1   N=1024  256: 22.3 -> 20.9
+//                    N=2048 128: 37.2 -> 31.2  384: 43.7 -> 48.4   N=4096  128: 68.3 -> 54.7   256: 68.6 -> 55.9   512: 82.1 -> 76.6
+//   d = 128 full     N=400   64: 13.1 -> 13.3   N=1024  256: 24.5 -> 23.0   384: 35.1 -> 41.6   N=4096  256: 75.6 -> 66.7
+//   d = 64 causal    N=400   64: 8.3 -> 8.4     N=777  224: 12.9 -> 11.9    N=2048  256: 26.7 -> 21.8   N=4096  512: 51.8 -> 45.7
+//   d = 64 full      N=400   64: 9.4 -> 9.0     N=777  224: 13.9 -> 12.8    N=2048  256: 26.2 -> 23.7   384: 33.6 -> 40.9
+// Naming a row count (tuning value flash_rows = 128) asks for one walk.
+static int flash_walks_for(int D, bool causal, int64_t B, int64_t N, int64_t H) {
+    if (D == 256 || N <= 512 || tuning().flash_rows.load() == kFlashRows) return 1;
+    const int64_t tiles = B * H * ((N + kFlashRows - 1) / kFlashRows);
+    return tiles <= (causal && N >= 4096 ? 512 : 256) ? 2 : 1;
+}
+
 template <typename T, int D, bool VARLEN>
 static int launch_mfma(FlashParams p, int64_t B, bool causal, hipStream_t stream) {
     if constexpr (D != 256 && !VARLEN) {
@@ -207,6 +224,15 @@ static int launch_mfma(FlashParams p, int64_t B, bool causal, hipStream_t stream
             dim3 grid((unsigned)persistent_grid(p.n_block_ids)), block(64 * kFlashWideWaves);
             if (causal) hipLaunchKernelGGL((flash_fwd_wide_kernel<T, D, true>), grid, block, 0, stream, p);
             else hipLaunchKernelGGL((flash_fwd_wide_kernel<T, D, false>), grid, block, 0, stream, p);
+            return static_cast<int>(hipGetLastError());
+        }
+    }
+    if constexpr (D != 256) {
+        if (flash_walks_for(D, causal, B, p.N, p.H) == 2) {
+            if (int rc = flash_plan_launch(p, B, causal, kFlashRows, kNeverPair, VARLEN)) return rc;
+            dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(2 * kFlashThreads);
+            if (causal) hipLaunchKernelGGL((flash_fwd_two_walks_kernel<T, D, true, VARLEN>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((flash_fwd_two_walks_kernel<T, D, false, VARLEN>), grid, block, 0, stream, p);
             return static_cast<int>(hipGetLastError());
         }
     }

@@ -39,6 +39,8 @@
 // mask all workgroups then walk the same number of key tiles, which evens out the end of the launch.
 #pragma once
 
+#include <type_traits>
+
 #include <cstdlib>
 
 #include "ahpc_device.hpp"
@@ -300,9 +302,16 @@ struct FlashStatsOut {
 //              (documents packed side by side, padding, windows): [4,1001,1001] with documents of a third of the length,
 //              fp16, H = 16, d = 96: forward with packing 48.1 -> 40.1 us;
 //              [2,2048,2048], bf16, H = 16, d = 128: 61 us where the same mask without empty tiles takes 92.
-template <typename T, int D, bool CAUSAL, bool VARLEN, bool STATS, int MASK = 0>
+//
+// WALKS == 2: a workgroup has two sets of four wavefronts and of buffers.  Set w takes the key tiles w, w + 2, .. for the same
+// 128 queries; at the end the sets exchange halves of their accumulators through LDS and each stores its half of the columns.
+// See flash_walks_for for where that pays.
+template <typename T, int D, bool CAUSAL, bool VARLEN, bool STATS, int MASK = 0, int WALKS = 1>
 __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const FlashStatsOut& st) {
     constexpr bool MASKED = MASK != 0;
+    static_assert(WALKS == 1 || (WALKS == 2 && !STATS && !MASKED && D <= 128), "two walks: the plain forward");
+    // a query may see its first key in any tile of its wavefront's walk
+    constexpr bool LATE = MASKED || WALKS > 1;
     static_assert(!(MASKED && VARLEN), "the mask belongs to dense launches");
     static_assert(!(STATS && MASK == 1), "the statistics pass reads the packed mask only");
     typedef FlashTile<D> TL;
@@ -311,13 +320,18 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
     constexpr int RB = TL::kRowBytes;
 
     // two buffers, each its own array: the compiler can then tell a DMA into one from reads of the other
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_k0[TL::kBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_v0[TL::kBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_k1[TL::kBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_v1[TL::kBytes];
+    __shared__ __attribute__((aligned(1024))) unsigned char all_k0[WALKS * TL::kBytes];
+    __shared__ __attribute__((aligned(1024))) unsigned char all_v0[WALKS * TL::kBytes];
+    __shared__ __attribute__((aligned(1024))) unsigned char all_k1[WALKS * TL::kBytes];
+    __shared__ __attribute__((aligned(1024))) unsigned char all_v1[WALKS * TL::kBytes];
 
     const int tid = threadIdx.x;
-    const int wave = tid >> 6;
+    const int walk = WALKS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / kFlashThreads);
+    const int wave = WALKS == 1 ? tid >> 6 : (tid >> 6) & 3;
+    unsigned char* const lds_k0 = all_k0 + walk * TL::kBytes;
+    unsigned char* const lds_v0 = all_v0 + walk * TL::kBytes;
+    unsigned char* const lds_k1 = all_k1 + walk * TL::kBytes;
+    unsigned char* const lds_v1 = all_v1 + walk * TL::kBytes;
     const int lane = tid & 63;
     const int col = lane & 31;   // query column / operand row owned by this lane
     const int half = lane >> 5;
@@ -393,9 +407,9 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
         const unsigned nrec = rem_next <= 0 ? 0u : rem_next > 0xffffffffll ? 0xffffffffu : (unsigned)rem_next;
         dma_tile<D>(k_next, nrec, dma_off_k, dst_k, wave_u);
         dma_tile<D>(v_next, nrec, dma_off_v, dst_v, wave_u);
-        k_next += tile_elems;
-        v_next += tile_elems;
-        rem_next -= 2 * tile_elems;
+        k_next += WALKS * tile_elems;
+        v_next += WALKS * tile_elems;
+        rem_next -= WALKS * 2 * tile_elems;
     };
 
     // ---- LDS operand addresses (byte offsets inside a tile) -------------------------------------
@@ -444,13 +458,14 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
             }
             return n_tiles;
         };
-        const int t_first = MASK == 2 ? live_from(0) : 0;
+        const int t_first = MASK == 2 ? live_from(0) : walk;
 
         // first tile on its way before anything else
         dma_both(t_first * kFlashKeys, lds_k0, lds_v0);
-        k_next = gk + tile_elems;
-        v_next = gv + tile_elems;
-        rem_next = (int64_t)(L - kFlashKeys - 1) * skv * 2 + 2 * d_real;
+        const int t_second = WALKS + walk;
+        k_next = gk + t_second * tile_elems;
+        v_next = gv + t_second * tile_elems;
+        rem_next = (int64_t)(L - t_second * kFlashKeys - 1) * skv * 2 + 2 * d_real;
 
         // ---- Q^T operands, pre-multiplied by c = scale*log2(e), kept for the whole query tile --------
         const int qw = q_tile0 + wave * 32;  // first query row of this wavefront
@@ -483,7 +498,7 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
         for (int r = 0; r < 16; ++r) neg_m[r] = 0.0f;
         float l_run = 0.0f;
         bool first = true;
-        bool seen = false;  // masked launches: this lane's query has met a key it may attend to
+        bool seen = false;  // masked launches and two walks: this lane's query has met a key it may attend to
         constexpr float kRaise = 8.0f;  // raise the reference maximum only when exceeded by 2^8
         const float* const mrow = MASK == 1 ? p.mask + ((int64_t)b * p.N + (qrow < L ? qrow : L - 1)) * p.N : nullptr;
         uint64_t mw = 0;  // MASK == 2: this query's word of the tile in hand, requested a step ahead
@@ -581,12 +596,12 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
 #pragma unroll
             for (int r = 1; r < 16; ++r) mx = max3(mx, s[0][r], s[1][r]);
             bool adjust;
-            if constexpr (MASKED) adjust = __builtin_amdgcn_ballot_w64(seen ? mx > kRaise : mx > -INFINITY) != 0;
+            if constexpr (LATE) adjust = __builtin_amdgcn_ballot_w64(seen ? mx > kRaise : mx > -INFINITY) != 0;
             else adjust = first || __builtin_amdgcn_ballot_w64(mx > kRaise) != 0;
             if (adjust) {
                 mx = halves_max(mx);                       // both lanes of a query agree
                 float delta, alpha;
-                if constexpr (MASKED) {
+                if constexpr (LATE) {
                     // a query without a visible key so far has accumulated nothing: its maximum is set exactly,
                     // nothing is rescaled; one that still sees none stays as it is
                     delta = seen ? fmaxf(mx, 0.0f) : (mx > -INFINITY ? mx : 0.0f);
@@ -662,9 +677,10 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
             l_run += sum;
         };
 
-        // Tile t out of the cur buffers; tile t_next, which is behind it, into the nxt buffers.
+        // Tile t out of the cur buffers; tile t_next, which is behind it, into the nxt buffers.  (Two walks: t and t_next are
+        // set 0's tiles; set 1 is one further and may be behind the last tile, or request one that is.)
         auto step = [&](unsigned char* cur_k, unsigned char* cur_v, unsigned char* nxt_k, unsigned char* nxt_v, int t, int t_next) {
-            const int k0 = t * kFlashKeys;
+            const int k0 = (t + walk) * kFlashKeys;
             const bool more = t_next < n_tiles;
             f32x4 mk[2][4];
             uint64_t mw_next = 0;
@@ -685,7 +701,7 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
                 if (more) dma_next(nxt_k, nxt_v);
             }
             // a wavefront whose queries all precede this tile has nothing to add
-            if (!(CAUSAL && k0 > qw + 31) && (MASK != 2 || __builtin_amdgcn_ballot_w64(mw != 0) != 0)) compute_tile(cur_k, cur_v, k0, mk, mw);
+            if (!(CAUSAL && k0 > qw + 31) && (WALKS == 1 || t + walk < n_tiles) && (MASK != 2 || __builtin_amdgcn_ballot_w64(mw != 0) != 0)) compute_tile(cur_k, cur_v, k0, mk, mw);
             if (MASK == 1 || more) {
                 __builtin_amdgcn_s_waitcnt(0);  // this wave's part of the next tile has landed
                 __syncthreads();                // everyone's has, and everyone is done with the current one
@@ -707,14 +723,68 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
                 step(lds_k1, lds_v1, lds_k0, lds_v0, t1, t);
             }
         } else {
-            for (int t = 0; t < n_tiles; t += 2) {
-                step(lds_k0, lds_v0, lds_k1, lds_v1, t, t + 1);
-                if (t + 1 < n_tiles) step(lds_k1, lds_v1, lds_k0, lds_v0, t + 1, t + 2);
+            for (int t = 0; t < n_tiles; t += 2 * WALKS) {
+                step(lds_k0, lds_v0, lds_k1, lds_v1, t, t + WALKS);
+                if (t + WALKS < n_tiles) step(lds_k1, lds_v1, lds_k0, lds_v0, t + WALKS, t + 2 * WALKS);
             }
         }
 
+        // ---- two walks: set w hands the other set's half of its row blocks over, with its maximum and sum, and merges its
+        //      own half (softmax-merge rule; a set that saw no key of a query has weight 0)
+        float l = halves_sum(l_run);
+        if constexpr (WALKS == 2) {
+            constexpr int HB = MB / 2;
+            __shared__ float set_ml[2][2][kFlashThreads];
+            const int at = wave * 64 + lane;
+            auto piece = [&](int mb) { return (mb == 0 ? all_k0 : mb == 1 ? all_v0 : mb == 2 ? all_k1 : all_v1) + wave * 4096 + lane * 16; };
+            auto hand_over = [&](auto first_block) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < HB; ++i) {
+                    const f32x16& a = oacc[decltype(first_block)::value + i];
+#pragma unroll
+                    for (int g4 = 0; g4 < 4; ++g4)
+                        *reinterpret_cast<f32x4*>(piece(decltype(first_block)::value + i) + g4 * 1024) = f32x4{a[4 * g4], a[4 * g4 + 1], a[4 * g4 + 2], a[4 * g4 + 3]};
+                }
+            };
+            __syncthreads();  // every wavefront is done with its last tile
+            set_ml[walk][0][at] = seen ? -neg_m[0] : -INFINITY;
+            set_ml[walk][1][at] = l;
+            if (walk == 0) hand_over(std::integral_constant<int, HB>{});
+            else hand_over(std::integral_constant<int, 0>{});
+            __syncthreads();
+            const float m_own = seen ? -neg_m[0] : -INFINITY, m_other = set_ml[1 - walk][0][at];
+            const float m = fmaxf(m_own, m_other);
+            const float w_own = seen ? fast_exp2(m_own - m) : 0.0f, w_other = m_other > -INFINITY ? fast_exp2(m_other - m) : 0.0f;
+            l = walk == 0 ? l * w_own + set_ml[1][1][at] * w_other : set_ml[0][1][at] * w_other + l * w_own;
+            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+            auto merge = [&](auto first_block) __attribute__((always_inline)) {
+                T* const dst = go + (int64_t)qrow * sn + 4 * half;
+#pragma unroll
+                for (int i = 0; i < HB; ++i) {
+                    constexpr int mb0 = decltype(first_block)::value;
+                    const f32x16& a = oacc[mb0 + i];
+#pragma unroll
+                    for (int g4 = 0; g4 < 4; ++g4) {
+                        const f32x4 o = *reinterpret_cast<const f32x4*>(piece(mb0 + i) + g4 * 1024);
+                        float x[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) x[e] = (a[4 * g4 + e] * w_own + o[e] * w_other) * inv;
+                        if (qrow < L && 32 * (mb0 + i) + 8 * g4 + 4 * half < d_real)
+                            *reinterpret_cast<u32x2*>(dst + 32 * (mb0 + i) + 8 * g4) = u32x2{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3])};
+                    }
+                }
+            };
+            if (walk == 0) merge(std::integral_constant<int, 0>{});
+            else merge(std::integral_constant<int, HB>{});
+            if constexpr (!VARLEN) {
+                if (p.keep_neg_lse2 != nullptr && half == 0 && walk == 0 && qrow < L)
+                    p.keep_neg_lse2[(int64_t)bh * p.keep_rows + qrow] = l > 0.0f ? -m - __builtin_log2f(l) : -INFINITY;
+            }
+            __syncthreads();  // the next query tile's first DMA reuses the buffers
+            continue;
+        }
+
         // ---- normalise and store: lane holds, per 32-row block, 4 runs of 4 consecutive lanes of d ---
-        const float l = halves_sum(l_run);
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
         if constexpr (STATS) {
             // delta = dO . O over the elements this lane holds, then over the two lanes of the query
@@ -812,6 +882,11 @@ inline int flash_plan_launch(FlashParams& p, int64_t B, bool causal, int rows_pe
 template <typename T, int D, bool CAUSAL, bool VARLEN>
 __global__ __launch_bounds__(kFlashThreads, D == 256 ? 1 : 2) void flash_fwd_mfma_kernel(const FlashParams p) {
     flash_fwd_mfma_body<T, D, CAUSAL, VARLEN, false>(p, FlashStatsOut{});
+}
+
+template <typename T, int D, bool CAUSAL, bool VARLEN>
+__global__ __launch_bounds__(2 * kFlashThreads, 2) void flash_fwd_two_walks_kernel(const FlashParams p) {
+    flash_fwd_mfma_body<T, D, CAUSAL, VARLEN, false, 0, 2>(p, FlashStatsOut{});
 }
 
 // Dense launches with a mask [B,N,N]: MASK 1 reads the caller's fp32 mask, MASK 2 its packed copy.

@@ -152,3 +152,51 @@ def test_ragged(where, rows, dtype, lens, H, H_kv, d, causal):
         for w, x in zip(want, parts):
             w[a:b] = np.asarray(x).reshape(L, *w.shape[1:])
     check([where.get(x, dtype) for x in (o, gq, gk, gv)], want, dtype)
+
+
+# The 16-bit forward whose workgroups walk the keys in two sets of wavefronts (launches of few tiles, more than 512 keys): odd
+# and even numbers of key tiles, a last tile of one row, one that only the second set has, head dimensions below the kernel's.
+WALKS = [(1, 513, 2, 2, 64, True), (1, 577, 2, 1, 128, False), (2, 640, 2, 1, 96, True), (1, 769, 4, 2, 40, True), (1, 705, 1, 1, 128, True)]
+
+
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16])
+@pytest.mark.parametrize("B,N,H,H_kv,d,causal", WALKS)
+def test_two_walks_dense(where, dtype, B, N, H, H_kv, d, causal):
+    q = O.round_to(O.fill_normal((B, N, H, d), 53, 1), dtype)
+    k, v = (O.round_to(O.fill_normal((B, N, H_kv, d), 53, t), dtype) for t in (2, 3))
+    k[:, 64:128] *= 3.0  # the second set's first tile holds the largest scores, and the sets' maxima differ
+    (tq, pq), (tk, pk), (tv, pv) = (where.put(x, dtype) for x in (q, k, v))
+    scale, st, kst = 1.0 / np.sqrt(d), (N * H * d, H * d, d), (N * H_kv * d, H_kv * d, d)
+    n_st = where.hip.flash_row_stats_bytes(B, N, H)
+    got, stats = [], []
+    for rows in (0, 128):  # by shape (two walks), and the one-walk form
+        where.hip.set_tuning("flash_rows", rows)
+        (o, po), (ws, pws) = where.out(q.shape, dtype), where.scratch(n_st)
+        assert where.hip.flash_fwd_keep(pq, pk, pv, po, dtype, B, N, H, H_kv, d, st, kst, scale, causal, pws)
+        got.append(where.get(o, dtype))
+        stats.append((ws.cpu().numpy() if hasattr(ws, "cpu") else np.asarray(ws)).reshape(B * H, -1)[:, :N])
+    rep = H // H_kv
+    want = O.attention(q, np.repeat(k, rep, axis=2), np.repeat(v, rep, axis=2), B, N, H, d, scale, causal)
+    check(got[:1], [want], dtype)
+    check(got[1:], [want], dtype)
+    # log2 of sums of up to N fp32 terms in two orders (N * 2^-24 / ln 2), and the reference maxima's own rounding (|m| < 64: 2^-18)
+    assert np.abs(stats[0] - stats[1]).max() <= N * 2.0**-23 + 2.0**-16
+
+
+@pytest.mark.parametrize("lens,H,H_kv,d,causal", [((513, 0, 1, 65), 2, 1, 64, True), ((64, 600, 130), 2, 2, 128, False), ((300, 577, 16), 2, 1, 80, True)])
+def test_two_walks_ragged(where, lens, H, H_kv, d, causal):
+    dtype = O.BF16
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T, longest, n = int(cu[-1]), max(lens), len(lens)
+    q = O.round_to(O.fill_normal((T, H, d), 54, 1), dtype)
+    k, v = (O.round_to(O.fill_normal((T, H_kv, d), 54, t), dtype) for t in (2, 3))
+    (tq, pq), (tk, pk), (tv, pv), (tcu, pcu), (o, po) = *(where.put(x, dtype) for x in (q, k, v)), where.ints(cu), where.out(q.shape, dtype)
+    scale, rep = 1.0 / np.sqrt(d), H // H_kv
+    where.hip.flash_fwd_varlen_gqa(pq, pk, pv, po, dtype, pcu, n, longest, H, H_kv, d, H * d, d, H_kv * d, d, scale, causal)
+    want = np.zeros_like(q)
+    for a, b in zip(cu, cu[1:]):
+        if b > a:
+            qs, ks, vs = (x[None, a:b] for x in (q, k, v))
+            want[a:b] = np.asarray(O.attention(qs, np.repeat(ks, rep, axis=2), np.repeat(vs, rep, axis=2), 1, int(b - a), H, d, scale,
+                                               causal)).reshape(b - a, H, d)
+    check([where.get(o, dtype)], [want], dtype)
