@@ -1,6 +1,7 @@
 // Process-wide tuning values of the launchers.  Each starts from an environment variable that is read once,
 // when the first launcher asks; ahpc_hip_set_tuning changes it afterwards (tests use that to reach code paths
-// that ordinary problem sizes would need a large GPU job for).  None of them changes results.
+// that ordinary problem sizes would need a large GPU job for).  None of them changes results
+// by more than the order in which sums are taken.
 #pragma once
 
 #include <atomic>
