@@ -224,7 +224,7 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) oacc[mb] = neg_m;
     float l_run = 0.0f;
-    bool first = true;
+    bool seen = false;  // this lane's query has met a key of finite score in this wavefront's tiles
     constexpr float kRaise = 8.0f;  // the reference maximum is raised only when exceeded by 2^8 (flash_fwd_mfma.hpp)
 
     for (int t = wave_u; t < n_tiles; t += kSplitWaves) {
@@ -248,10 +248,13 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
 #pragma unroll
         for (int r = 3; r < 15; r += 2) mx = max3(mx, s[r], s[r + 1]);
         mx = max3(mx, s[15], s[15]);
-        if (first || __builtin_amdgcn_ballot_w64(mx > kRaise) != 0) {
+        if (__builtin_amdgcn_ballot_w64(seen ? mx > kRaise : mx > -INFINITY) != 0) {
             mx = halves_max(mx);  // both lanes of a query agree
-            const float delta = first ? mx : fmaxf(mx, 0.0f);
-            const float alpha = fast_exp2(-delta);
+            // the first maximum is set exactly and rescales nothing: 2^-delta of scores below -128 overflows, and times the empty
+            // accumulators that is not a number, in any of the four walks
+            const float delta = seen ? fmaxf(mx, 0.0f) : (mx > -INFINITY ? mx : 0.0f);
+            const float alpha = seen ? fast_exp2(-delta) : 1.0f;
+            seen = seen || mx > -INFINITY;
             l_run *= alpha;
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
@@ -263,7 +266,6 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
                 s[r] -= delta;
                 neg_m[r] = nm;
             }
-            first = false;
         }
         float sum = 0.0f;
 #pragma unroll
@@ -281,7 +283,7 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
     {
         const float l = halves_sum(l_run);
         if (half == 0) {
-            lds_m[wave][col] = first ? -INFINITY : -neg_m[0];  // (a wavefront without a tile)
+            lds_m[wave][col] = seen ? -neg_m[0] : -INFINITY;  // (a wavefront without a tile)
             lds_l[wave][col] = l;
         }
         X::put(lds, oacc, wave, lane);
