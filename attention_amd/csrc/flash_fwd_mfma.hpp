@@ -609,7 +609,7 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
                     seen = seen || mx > -INFINITY;
                 } else {
                     delta = first ? mx : fmaxf(mx, 0.0f);
-                    alpha = fast_exp2(-delta);
+                    alpha = first ? 1.0f : fast_exp2(-delta);  // (scores below -128 would make it infinite, times zeros)
                 }
                 l_run *= alpha;
 #pragma unroll

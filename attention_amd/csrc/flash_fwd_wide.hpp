@@ -254,7 +254,7 @@ __global__ __launch_bounds__(64 * kFlashWideWaves, 1) void flash_fwd_wide_kernel
             if (first || __builtin_amdgcn_ballot_w64(mx > kRaise) != 0) {
                 mx = halves_max(mx);  // both lanes of a query agree
                 const float delta = first ? mx : fmaxf(mx, 0.0f);
-                const float alpha = fast_exp2(-delta);
+                const float alpha = first ? 1.0f : fast_exp2(-delta);  // (scores below -128 would make it infinite, times zeros)
                 l_run *= alpha;
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
