@@ -414,27 +414,10 @@ static void launch_dkv(const FlashBwdParams& m, dim3 grid, dim3 block, hipStream
     }
 }
 
-// Launch geometry of the dQ and dK/dV kernels (tiles, pairing, the map from workgroups to tiles).
-static int plan_bwd(FlashBwdParams& m, int64_t B, int64_t H_kv, bool causal, bool ragged, int rows = kFlashRows) {
-    m.n_tiles = (m.N + rows - 1) / rows;
-    // causal launches: a workgroup takes a long and a short tile of its head, so that all (of a sequence) do the same work
-    m.paired = (causal && rows == kFlashRows && m.n_tiles >= 2 && tuning().bwd_pair.load() != 0) ? 1 : 0;
-    m.spread = ragged ? 1 : 0;
-    m.n_bh = (int32_t)(B * m.H);
-    const int64_t units = bwd_units(m), pairs_q = B * m.H, pairs_kv = B * H_kv;
-    const int64_t total_q = pairs_q * units, total_kv = pairs_kv * units;
-    const int64_t per_q = ragged ? (pairs_q + 7) / 8 * units : (total_q + 7) / 8;
-    const int64_t per_kv = ragged ? (pairs_kv + 7) / 8 * units : (total_kv + 7) / 8;
-    if (per_q * 8 > 0x7FFFFFF0ll || per_kv * 8 > 0x7FFFFFF0ll) return AHPC_ERR_BAD_SHAPE;
-    m.total_q = (int32_t)total_q; m.per_xcd_q = (int32_t)per_q;
-    m.total_kv = (int32_t)total_kv; m.per_xcd_kv = (int32_t)per_kv;
-    return AHPC_OK;
-}
-
 // Statistics, dQ, dK and dV.  pm: the packed copy of a dense mask (dense launches only), or null.
 template <typename T, int D, bool VARLEN>
 static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const void* o_kept, const float* stats_kept, int64_t B,
-                          int64_t H_kv, bool causal, float* lse2, float* delta, hipStream_t stream) {
+                          bool causal, float* lse2, float* delta, hipStream_t stream) {
     // 1. statistics: the forward kernel with its output kept in registers
     FlashParams f{};
     f.q = p.q; f.k = p.k; f.v = p.v; f.o = nullptr;
@@ -457,7 +440,7 @@ static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const v
     const FlashStatsOut st{p.d_out, lse2, delta, p.rows_padded};
     const dim3 block(kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));
-    if (int rc = plan_bwd(m, B, H_kv, causal, VARLEN)) return rc;
+    if (int rc = bwd_plan_launch(m, B, causal, VARLEN)) return rc;
     const dim3 grid_q((unsigned)(m.per_xcd_q * 8)), grid_kv((unsigned)(m.per_xcd_kv * 8));
     auto launch = [&](auto causal_c, auto masked_c) {
         constexpr bool C = decltype(causal_c)::value, M = decltype(masked_c)::value;
@@ -493,17 +476,17 @@ static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const v
 }
 
 template <typename T>
-static int launch_mfma(const FlashBwdParams& p, const PackedMask* pm, const void* o_kept, const float* stats_kept, int64_t B,
-                       int64_t H_kv, int d, bool causal, float* lse2, float* delta, hipStream_t stream) {
+static int launch_mfma(const FlashBwdParams& p, const PackedMask* pm, const void* o_kept, const float* stats_kept, int64_t B, int d,
+                       bool causal, float* lse2, float* delta, hipStream_t stream) {
     if (p.cu_seqlens) {
         if (pm) return AHPC_ERR_BAD_SHAPE;
-        if (d == 128) return launch_mfma_dv<T, 128, true>(p, nullptr, nullptr, nullptr, B, H_kv, causal, lse2, delta, stream);
-        if (d == 64) return launch_mfma_dv<T, 64, true>(p, nullptr, nullptr, nullptr, B, H_kv, causal, lse2, delta, stream);
-        if (d == 256) return launch_mfma_dv<T, 256, true>(p, nullptr, nullptr, nullptr, B, H_kv, causal, lse2, delta, stream);
+        if (d == 128) return launch_mfma_dv<T, 128, true>(p, nullptr, nullptr, nullptr, B, causal, lse2, delta, stream);
+        if (d == 64) return launch_mfma_dv<T, 64, true>(p, nullptr, nullptr, nullptr, B, causal, lse2, delta, stream);
+        if (d == 256) return launch_mfma_dv<T, 256, true>(p, nullptr, nullptr, nullptr, B, causal, lse2, delta, stream);
     } else {
-        if (d == 128) return launch_mfma_dv<T, 128, false>(p, pm, o_kept, stats_kept, B, H_kv, causal, lse2, delta, stream);
-        if (d == 64) return launch_mfma_dv<T, 64, false>(p, pm, o_kept, stats_kept, B, H_kv, causal, lse2, delta, stream);
-        if (d == 256) return launch_mfma_dv<T, 256, false>(p, pm, o_kept, stats_kept, B, H_kv, causal, lse2, delta, stream);
+        if (d == 128) return launch_mfma_dv<T, 128, false>(p, pm, o_kept, stats_kept, B, causal, lse2, delta, stream);
+        if (d == 64) return launch_mfma_dv<T, 64, false>(p, pm, o_kept, stats_kept, B, causal, lse2, delta, stream);
+        if (d == 256) return launch_mfma_dv<T, 256, false>(p, pm, o_kept, stats_kept, B, causal, lse2, delta, stream);
     }
     return AHPC_ERR_UNSUPPORTED_HEAD_DIM;
 }
@@ -518,7 +501,7 @@ static int64_t bwd_rows_wanted() {
 // fp32 tensors: the same three steps on the fp32 matrix instructions (flash_bwd_f32_mfma.hpp), dK and dV always in two walks;
 // launches too small for those: flash_f32_split.hpp, dK and dV in one
 template <int D, bool VARLEN>
-static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, int64_t H_kv, bool causal, float* lse2, float* delta,
+static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, bool causal, float* lse2, float* delta,
                               hipStream_t stream) {
     FlashParams f{};
     f.q = p.q; f.k = p.k; f.v = p.v; f.o = nullptr;
@@ -535,7 +518,7 @@ static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, int64_t H_kv, 
     const dim3 block(split ? kWave * kSplitWaves : kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));
     FlashBwdParams m = p;
-    if (int rc = plan_bwd(m, B, H_kv, causal, VARLEN, split ? kSplitRows : kFlashRows)) return rc;
+    if (int rc = bwd_plan_launch(m, B, causal, VARLEN, split ? kSplitRows : kFlashRows)) return rc;
     const dim3 grid_q((unsigned)(m.per_xcd_q * 8)), grid_kv((unsigned)(m.per_xcd_kv * 8));
     if (split) {
         auto launch = [&](auto causal_c) {
@@ -562,14 +545,14 @@ static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, int64_t H_kv, 
     return static_cast<int>(hipGetLastError());
 }
 
-static int launch_f32_mfma(const FlashBwdParams& p, int64_t B, int64_t H_kv, int d, bool causal, float* lse2, float* delta,
+static int launch_f32_mfma(const FlashBwdParams& p, int64_t B, int d, bool causal, float* lse2, float* delta,
                            hipStream_t stream) {
     if (p.cu_seqlens) {
-        if (d == 128) return launch_f32_mfma_dv<128, true>(p, B, H_kv, causal, lse2, delta, stream);
-        if (d == 64) return launch_f32_mfma_dv<64, true>(p, B, H_kv, causal, lse2, delta, stream);
+        if (d == 128) return launch_f32_mfma_dv<128, true>(p, B, causal, lse2, delta, stream);
+        if (d == 64) return launch_f32_mfma_dv<64, true>(p, B, causal, lse2, delta, stream);
     } else {
-        if (d == 128) return launch_f32_mfma_dv<128, false>(p, B, H_kv, causal, lse2, delta, stream);
-        if (d == 64) return launch_f32_mfma_dv<64, false>(p, B, H_kv, causal, lse2, delta, stream);
+        if (d == 128) return launch_f32_mfma_dv<128, false>(p, B, causal, lse2, delta, stream);
+        if (d == 64) return launch_f32_mfma_dv<64, false>(p, B, causal, lse2, delta, stream);
     }
     return AHPC_ERR_UNSUPPORTED_HEAD_DIM;
 }
@@ -647,16 +630,16 @@ static int flash_bwd_any(const void* d_out, const void* q, const void* k, const 
         m.scale_log2 = scale * kLog2e;
         m.d_real = (int32_t)d;
         if (!mask) {
-            if (dtype == AHPC_F32) return launch_f32_mfma(m, B, H_kv, kernel_d, causal != 0, p.lse, p.delta, st);
-            return dtype == AHPC_F16 ? launch_mfma<f16_t>(m, nullptr, o_kept, stats_kept, B, H_kv, kernel_d, causal != 0, p.lse, p.delta, st)
-                                     : launch_mfma<bf16_t>(m, nullptr, o_kept, stats_kept, B, H_kv, kernel_d, causal != 0, p.lse, p.delta, st);
+            if (dtype == AHPC_F32) return launch_f32_mfma(m, B, kernel_d, causal != 0, p.lse, p.delta, st);
+            return dtype == AHPC_F16 ? launch_mfma<f16_t>(m, nullptr, o_kept, stats_kept, B, kernel_d, causal != 0, p.lse, p.delta, st)
+                                     : launch_mfma<bf16_t>(m, nullptr, o_kept, stats_kept, B, kernel_d, causal != 0, p.lse, p.delta, st);
         }
         // a dense mask on 16-bit tensors: the matrix-core kernels on the mask's packed copy (both layouts), where that
         // can be made (not under graph capture, not beyond the library's buffer limit)
         bool launched = false;
         const int rc = with_packed_mask(mask, B, N, true, st, &launched, [&](const PackedMask& pm) {
-            return dtype == AHPC_F16 ? launch_mfma<f16_t>(m, &pm, o_kept, stats_kept, B, H_kv, kernel_d, causal != 0, p.lse, p.delta, st)
-                                     : launch_mfma<bf16_t>(m, &pm, o_kept, stats_kept, B, H_kv, kernel_d, causal != 0, p.lse, p.delta, st);
+            return dtype == AHPC_F16 ? launch_mfma<f16_t>(m, &pm, o_kept, stats_kept, B, kernel_d, causal != 0, p.lse, p.delta, st)
+                                     : launch_mfma<bf16_t>(m, &pm, o_kept, stats_kept, B, kernel_d, causal != 0, p.lse, p.delta, st);
         });
         if (launched || rc != AHPC_OK) return rc;
     }

@@ -77,7 +77,7 @@ __global__ __launch_bounds__(kFlashThreads, (D == 128 ? 1 : 2)) void flash_bwd_d
     const int lane = tid & 63;
     const int col = lane & 31;
     const int half = lane >> 5;
-    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_q, p.per_xcd_q, bwd_units(p), p.spread ? p.n_bh : 0);
+    const BwdWork work = bwd_work_q(blockIdx.x, p);
     if (!work.valid) return;
     const int b = work.bh / p.H, h = work.bh - b * p.H;
     const int hk = h / p.kv_group;
@@ -272,7 +272,7 @@ __global__ __launch_bounds__(kFlashThreads, (PART == 2 ? 1 : 2)) void flash_bwd_
     const int lane = tid & 63;
     const int col = lane & 31;
     const int half = lane >> 5;
-    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_kv, p.per_xcd_kv, bwd_units(p), p.spread ? p.n_bh / p.kv_group : 0);
+    const BwdWork work = bwd_work_kv(blockIdx.x, p);
     if (!work.valid) return;
     const int heads_kv = p.H / p.kv_group;
     const int b = work.bh / heads_kv, hk = work.bh - b * heads_kv;

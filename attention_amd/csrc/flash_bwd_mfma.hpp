@@ -51,12 +51,13 @@ struct FlashBwdParams {
     int32_t kv_group;           // query heads per key/value head
     int32_t n_tiles;            // 128-row tiles per sequence (of the longest one)
     int32_t n_bh;               // B * H
-    int32_t spread;             // ragged batches: 1 = the (sequence, head) pairs are dealt to the XCDs in turn (bwd_work_of_block)
+    int32_t slices_q, slices_kv;    // ragged batches: slices into which the tiles of a (sequence, head) pair are dealt to the XCDs
+                                // (bwd_work_of_block; dQ kernel, dK/dV kernel), 0 = equal shares of the id range
     int32_t paired;             // 1: a workgroup takes two tiles of a head, a long walk and a short one (causal launches:
                                 // tile i sees i + 1 tiles' worth of the other side, so i and n_tiles - 1 - i together are the
                                 // same work for every workgroup); total_q / total_kv count workgroups accordingly
-    int32_t total_q, per_xcd_q;     // dQ kernel: workgroups (B * H * n_tiles) and ceil(that / 8)
-    int32_t total_kv, per_xcd_kv;   // dK/dV kernel: workgroups (B * H_kv * n_tiles) and ceil(that / 8)
+    int32_t total_q, per_xcd_q;     // dQ kernel: workgroups (B * H * n_tiles) and ids per XCD
+    int32_t total_kv, per_xcd_kv;   // dK/dV kernel: workgroups (B * H_kv * n_tiles) and ids per XCD
     float scale;
     float scale_log2;           // scale * log2(e)
     int32_t d_real;             // head dimension of the tensors when smaller than the kernels' D, 0 = D (FlashParams::d_real)
@@ -65,10 +66,15 @@ struct FlashBwdParams {
 // Workgroup id -> (sequence * heads + head, tile).  Both kernels are launched on a 1-D grid of 8 * per_xcd
 // workgroups.  Hardware deals consecutive ids to the 8 XCDs in turn; `logical` undoes that, so that the tiles
 // of one head (consecutive logical ids) run on one XCD and find the head's K/V (Q/dO) in its L2.
-// Ragged batches (spread_groups = number of (sequence, head) pairs, 0 for dense ones): equal shares of the id range are not
-// equal shares of the work, so pair g runs on XCD g % 8, with as many ids as the longest sequence needs; a workgroup beyond
-// its own sequence's tiles exits.  (Forward and backward of 12 sequences of 100 to 2000 tokens, 16 heads over 4, d = 64: 444 us
-// in shares of the id range, 361 dealt, 332 dealt and paired: dQ 115 -> 75 us, dK/dV 218 -> 146.)
+// Ragged batches: equal shares of the id range are not equal shares of the work, so the pairs are dealt out.  A pair's tiles
+// (as many ids as the longest sequence needs; a workgroup beyond its own sequence's tiles exits) go in turn to `slices`
+// slices, and slice i runs on XCD i % 8.  heads * slices is a multiple of 8 (bwd_slices_for): every sequence, however long, is
+// spread evenly over the XCDs.  Which slice holds the pair's first tile rotates with the round of eight, so that sequences of
+// a tile or two don't meet on the same XCD.  Whole backward, us, in equal shares of the id range / a whole pair per XCD / this:
+//   12 sequences of 100 to 2000 tokens, 16 heads over 4, d = 64, causal   385 / 289 / 291    full 630 / 382 / 377
+//   one of 16384, 8 heads over 1, d = 128                                full 5518 / 16265 / 5598 (one XCD at work in the second)
+//   16384 and 700, 32 heads over 2, d = 64                             causal 10738 / 9884 / 6531
+//   9000, 800 and 5000, 4 heads, d = 128                               causal 1189 / 1039 / 691
 struct BwdWork {
     int bh, tile;
     bool valid;
@@ -76,17 +82,53 @@ struct BwdWork {
 // work units per head: tiles, or pairs of them
 __host__ __device__ inline int bwd_units(int paired, int n_tiles) { return paired ? (n_tiles + 1) >> 1 : n_tiles; }
 __host__ __device__ inline int bwd_units(const FlashBwdParams& p) { return bwd_units(p.paired, p.n_tiles); }
-__host__ __device__ inline BwdWork bwd_work_of_block(unsigned block_id, int total, int per_xcd, int n_tiles, int spread_groups) {
-    if (spread_groups) {
-        const int k = (int)(block_id >> 3);
-        const int round = k / n_tiles;
-        const int g = round * 8 + (int)(block_id & 7u);
-        return g < spread_groups ? BwdWork{g, k - round * n_tiles, true} : BwdWork{0, 0, false};
+inline int bwd_slices_for(int64_t heads) {
+    int slices = 1;
+    while ((heads * slices) % 8) slices *= 2;
+    return slices;
+}
+__host__ __device__ inline BwdWork bwd_work_of_block(unsigned block_id, int total, int per_xcd, int n_units, int n_pairs, int slices) {
+    if (slices) {
+        const int k = (int)(block_id >> 3), len = (n_units + slices - 1) / slices;  // ids per slice
+        const int round = k / len;
+        const int slice = round * 8 + (int)(block_id & 7u);
+        const int pair = slice / slices, tile = (k - round * len) * slices + ((slice + round) & (slices - 1));
+        return pair < n_pairs && tile < n_units ? BwdWork{pair, tile, true} : BwdWork{0, 0, false};
     }
     const int logical = (int)(block_id & 7u) * per_xcd + (int)(block_id >> 3);
     if (logical >= total) return BwdWork{0, 0, false};
-    const int bh = logical / n_tiles;
-    return BwdWork{bh, logical - bh * n_tiles, true};
+    const int pair = logical / n_units;
+    return BwdWork{pair, logical - pair * n_units, true};
+}
+__host__ __device__ inline BwdWork bwd_work_q(unsigned block_id, const FlashBwdParams& p) {
+    return bwd_work_of_block(block_id, p.total_q, p.per_xcd_q, bwd_units(p), p.n_bh, p.slices_q);
+}
+__host__ __device__ inline BwdWork bwd_work_kv(unsigned block_id, const FlashBwdParams& p) {
+    return bwd_work_of_block(block_id, p.total_kv, p.per_xcd_kv, bwd_units(p), p.n_bh / p.kv_group, p.slices_kv);
+}
+
+// Launch geometry of the dQ and dK/dV kernels (tiles, pairing, the map from workgroups to tiles); p.N, p.H and p.kv_group are set.
+inline int bwd_plan_launch(FlashBwdParams& p, int64_t B, bool causal, bool ragged, int rows = kFlashRows) {
+    p.n_tiles = (p.N + rows - 1) / rows;
+    // causal launches: a workgroup takes a long and a short tile of its head, so that all (of a sequence) do the same work
+    p.paired = (causal && rows == kFlashRows && p.n_tiles >= 2 && tuning().bwd_pair.load() != 0) ? 1 : 0;
+    p.n_bh = (int32_t)(B * p.H);
+    constexpr int64_t kMostIds = 0x7FFFFFF0ll;
+    auto plan = [&](int64_t heads, int32_t& total, int32_t& per_xcd, int32_t& slices) {
+        const int64_t units = bwd_units(p), all = B * heads * units;
+        slices = ragged ? bwd_slices_for(heads) : 0;
+        int64_t per = (all + 7) / 8;
+        if (slices) {
+            const int64_t dealt = (B * heads * slices + 7) / 8 * ((units + slices - 1) / slices);
+            if (dealt * 8 <= kMostIds) per = dealt;
+            else slices = 0;
+        }
+        total = (int32_t)all;
+        per_xcd = (int32_t)per;
+        return all <= kMostIds;
+    };
+    if (!plan(p.H, p.total_q, p.per_xcd_q, p.slices_q) || !plan(p.H / p.kv_group, p.total_kv, p.per_xcd_kv, p.slices_kv)) return AHPC_ERR_BAD_SHAPE;
+    return AHPC_OK;
 }
 
 // Byte offset inside a tile swizzled with FlashTile::fb of the 8 bytes a lane hands to a transposing read that fetches
@@ -159,7 +201,7 @@ __global__ __launch_bounds__(kFlashThreads, (D > 128 ? 1 : 2)) void flash_bwd_dq
     const int lane = tid & 63;
     const int col = lane & 31;
     const int half = lane >> 5;
-    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_q, p.per_xcd_q, bwd_units(p), p.spread ? p.n_bh : 0);
+    const BwdWork work = bwd_work_q(blockIdx.x, p);
     if (!work.valid) return;
     const int b = work.bh / p.H, h = work.bh - b * p.H;
     const int hk = h / p.kv_group;
@@ -405,7 +447,7 @@ __global__ __launch_bounds__(kFlashThreads, ((PART == 0 && D > 64) || D > 128 ? 
     const int lane = tid & 63;
     const int col = lane & 31;
     const int half = lane >> 5;
-    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_kv, p.per_xcd_kv, bwd_units(p), p.spread ? p.n_bh / p.kv_group : 0);
+    const BwdWork work = bwd_work_kv(blockIdx.x, p);
     if (!work.valid) return;
     const int heads_kv = p.H / p.kv_group;
     const int b = work.bh / heads_kv, hk = work.bh - b * heads_kv;

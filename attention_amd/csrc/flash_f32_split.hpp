@@ -392,7 +392,7 @@ __global__ __launch_bounds__(kWave * kSplitWaves, 1) void flash_bwd_dq_f32_split
     const int col = lane & 31;
     const int half = lane >> 5;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_q, p.per_xcd_q, p.n_tiles, p.spread ? p.n_bh : 0);
+    const BwdWork work = bwd_work_q(blockIdx.x, p);
     if (!work.valid) return;
     const int b = work.bh / p.H, h = work.bh - b * p.H;
     const int hk = h / p.kv_group;
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(kWave * kSplitWaves, 1) void flash_bwd_dkv_f32_spli
     const int half = lane >> 5;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const int heads_kv = p.H / p.kv_group;
-    const BwdWork work = bwd_work_of_block(blockIdx.x, p.total_kv, p.per_xcd_kv, p.n_tiles, p.spread ? p.n_bh / p.kv_group : 0);
+    const BwdWork work = bwd_work_kv(blockIdx.x, p);
     if (!work.valid) return;
     const int b = work.bh / heads_kv, hk = work.bh - b * heads_kv;
     int seq0 = 0;

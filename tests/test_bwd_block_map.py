@@ -1,0 +1,46 @@
+"""The backward kernels' workgroup -> work map (the launchers' own plan, on the host): every unit of every (sequence, head) pair
+exactly once, and in a ragged batch every sequence spread evenly over the 8 XCDs (consecutive workgroup ids run on them in
+turn), so that neither few heads nor unequal lengths leave XCDs idle."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from simt import simt as S
+
+
+def block_map(B, N, H, H_kv, causal, ragged, kv, capacity=1 << 20):
+    lib = S.load()
+    pair, unit, paired = np.empty(capacity, np.int32), np.empty(capacity, np.int32), C.c_int()
+    n = lib.simt_bwd_block_map(B, N, H, H_kv, int(causal), int(ragged), int(kv), capacity, C.c_void_p(pair.ctypes.data),
+                               C.c_void_p(unit.ctypes.data), C.byref(paired))
+    assert 0 <= n <= capacity
+    return pair[:n], unit[:n], paired.value
+
+
+SHAPES = [(1, 16384, 8, 1), (1, 4096, 8, 4), (3, 2048, 12, 3), (9, 3271, 8, 1), (12, 1783, 16, 4), (5, 7908, 32, 8), (32, 130, 5, 5),
+          (2, 100, 40, 40), (7, 1024, 6, 2)]
+
+
+@pytest.mark.parametrize("kv", [False, True])
+@pytest.mark.parametrize("ragged", [False, True])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("B,N,H,H_kv", SHAPES)
+def test_every_unit_once_and_sequences_spread_over_the_xcds(B, N, H, H_kv, causal, ragged, kv):
+    pair, unit, paired = block_map(B, N, H, H_kv, causal, ragged, kv)
+    heads, tiles = H_kv if kv else H, (N + 127) // 128
+    units = (tiles + 1) // 2 if paired else tiles
+    valid = pair >= 0
+    assert np.array_equal(np.sort(pair[valid].astype(np.int64) * units + unit[valid]), np.arange(B * heads * units))
+    if not ragged:
+        return
+    xcd = np.arange(len(pair)) % 8
+    for b in range(B):
+        for live in {1, units // 2, units}:  # a sequence as long as the longest one, and shorter ones
+            mine = valid & (pair // heads == b) & (unit < live)
+            share = np.bincount(xcd[mine], minlength=8)
+            # heads * live units; a slice holds one more than its part at most, and an XCD has at most `heads` slices of a sequence
+            assert share.max() <= heads * live / 8 + heads, (b, live, share)
+    # the first units of all sequences together (a batch of short sequences and one long one)
+    share = np.bincount(xcd[valid & (unit == 0)], minlength=8)
+    assert share.max() <= -(-B * heads // 8) + heads
