@@ -440,7 +440,7 @@ static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const v
     const FlashStatsOut st{p.d_out, lse2, delta, p.rows_padded};
     const dim3 block(kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));
-    if (int rc = bwd_plan_launch(m, B, causal, VARLEN)) return rc;
+    if (int rc = bwd_plan_launch(m, B, causal, VARLEN, D == 64)) return rc;
     const dim3 grid_q((unsigned)(m.per_xcd_q * 8)), grid_kv((unsigned)(m.per_xcd_kv * 8));
     auto launch = [&](auto causal_c, auto masked_c) {
         constexpr bool C = decltype(causal_c)::value, M = decltype(masked_c)::value;
@@ -518,7 +518,7 @@ static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, bool causal, f
     const dim3 block(split ? kWave * kSplitWaves : kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));
     FlashBwdParams m = p;
-    if (int rc = bwd_plan_launch(m, B, causal, VARLEN, split ? kSplitRows : kFlashRows)) return rc;
+    if (int rc = bwd_plan_launch(m, B, causal, VARLEN, false, split ? kSplitRows : kFlashRows)) return rc;
     const dim3 grid_q((unsigned)(m.per_xcd_q * 8)), grid_kv((unsigned)(m.per_xcd_kv * 8));
     if (split) {
         auto launch = [&](auto causal_c) {

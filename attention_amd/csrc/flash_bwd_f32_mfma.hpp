@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kFlashThreads, (D == 128 ? 1 : 2)) void flash_bwd_d
         kv_base = (int64_t)b * p.kv_stride_b + (int64_t)hk * p.kv_stride_h;
     }
     const int n_own = VARLEN ? (L + kFlashRows - 1) / kFlashRows : p.n_tiles;  // tiles of this sequence
-    if (VARLEN && work.tile >= bwd_units(p.paired, n_own)) return;
+    if (VARLEN && work.tile >= bwd_units(p.paired_q, n_own)) return;
     const float* const gq = static_cast<const float*>(p.q) + base;
     const float* const gdo = static_cast<const float*>(p.d_out) + base;
     const float* const gk = static_cast<const float*>(p.k) + kv_base;
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kFlashThreads, (D == 128 ? 1 : 2)) void flash_bwd_d
         // long tiles first: under a causal mask the late query tiles walk the most keys; a paired workgroup then takes the
         // early tile that completes its share
         const int tile = part == 0 ? work.tile : n_own - 1 - work.tile;
-        if (part == 1 && (!p.paired || tile == work.tile)) break;
+        if (part == 1 && (!p.paired_q || tile == work.tile)) break;
         const int q_tile0 = (n_own - 1 - tile) * kFlashRows;
         if (part == 1) __syncthreads();  // every wavefront is done with the first pass's last tile
         int k_end = L;
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(kFlashThreads, (PART == 2 ? 1 : 2)) void flash_bwd_
         L = p.cu_seqlens[b + 1] - seq0;
     }
     const int n_own = VARLEN ? (L + kFlashRows - 1) / kFlashRows : p.n_tiles;  // tiles of this sequence
-    if (VARLEN && work.tile >= bwd_units(p.paired, n_own)) return;
+    if (VARLEN && work.tile >= bwd_units(p.paired_kv, n_own)) return;
     const int64_t kv_base = VARLEN ? (int64_t)seq0 * p.kv_stride_n + (int64_t)hk * p.kv_stride_h
                                    : (int64_t)b * p.kv_stride_b + (int64_t)hk * p.kv_stride_h;
     const float* const gk = static_cast<const float*>(p.k) + kv_base;
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(kFlashThreads, (PART == 2 ? 1 : 2)) void flash_bwd_
         // under a causal mask the early key tiles see the most queries: they go first; a paired workgroup then takes the
         // late tile that completes its share
         const int tile = part == 0 ? work.tile : n_own - 1 - work.tile;
-        if (part == 1 && (!p.paired || tile == work.tile)) break;
+        if (part == 1 && (!p.paired_kv || tile == work.tile)) break;
         const int k_tile0 = tile * kFlashRows;
         const int kw = k_tile0 + wave * 32;  // first key of this wavefront
         const int key = kw + col;

@@ -53,7 +53,7 @@ struct FlashBwdParams {
     int32_t n_bh;               // B * H
     int32_t slices_q, slices_kv;    // ragged batches: slices into which the tiles of a (sequence, head) pair are dealt to the XCDs
                                 // (bwd_work_of_block; dQ kernel, dK/dV kernel), 0 = equal shares of the id range
-    int32_t paired;             // 1: a workgroup takes two tiles of a head, a long walk and a short one (causal launches:
+    int32_t paired_q, paired_kv;    // 1: a workgroup takes two tiles of a head, a long walk and a short one (causal launches:
                                 // tile i sees i + 1 tiles' worth of the other side, so i and n_tiles - 1 - i together are the
                                 // same work for every workgroup); total_q / total_kv count workgroups accordingly
     int32_t total_q, per_xcd_q;     // dQ kernel: workgroups (B * H * n_tiles) and ids per XCD
@@ -81,7 +81,6 @@ struct BwdWork {
 };
 // work units per head: tiles, or pairs of them
 __host__ __device__ inline int bwd_units(int paired, int n_tiles) { return paired ? (n_tiles + 1) >> 1 : n_tiles; }
-__host__ __device__ inline int bwd_units(const FlashBwdParams& p) { return bwd_units(p.paired, p.n_tiles); }
 inline int bwd_slices_for(int64_t heads) {
     int slices = 1;
     while ((heads * slices) % 8) slices *= 2;
@@ -101,21 +100,38 @@ __host__ __device__ inline BwdWork bwd_work_of_block(unsigned block_id, int tota
     return BwdWork{pair, logical - pair * n_units, true};
 }
 __host__ __device__ inline BwdWork bwd_work_q(unsigned block_id, const FlashBwdParams& p) {
-    return bwd_work_of_block(block_id, p.total_q, p.per_xcd_q, bwd_units(p), p.n_bh, p.slices_q);
+    return bwd_work_of_block(block_id, p.total_q, p.per_xcd_q, bwd_units(p.paired_q, p.n_tiles), p.n_bh, p.slices_q);
 }
 __host__ __device__ inline BwdWork bwd_work_kv(unsigned block_id, const FlashBwdParams& p) {
-    return bwd_work_of_block(block_id, p.total_kv, p.per_xcd_kv, bwd_units(p), p.n_bh / p.kv_group, p.slices_kv);
+    return bwd_work_of_block(block_id, p.total_kv, p.per_xcd_kv, bwd_units(p.paired_kv, p.n_tiles), p.n_bh / p.kv_group, p.slices_kv);
+}
+
+// Whether a causal launch takes tiles in pairs (FlashBwdParams::paired_q, paired_kv; `pairs` = (sequence, head) pairs of the
+// kernel in question).  Dense launches do.  A ragged batch whose tiles all find a place at once is done when its longest single
+// walk is, and a pair of tiles takes (n + 1) / n of that; beyond it pairs even out the second round.  The line lies a quarter
+// above a round of 256 CUs (tiles are counted from the longest sequence: some don't exist), or of 512 places for the 16-bit
+// kernels at d = 64, where two workgroups share a CU and long walks meet on one from 448 tiles on.  Whole backward, us, single ->
+// paired, by tiles:
+//   bf16, d = 128, 16 heads   256 (4 x 512) 59 -> 78      320 (4 of 500 to 1239, 8 heads) 106 -> 120     512 (4 x 1024) 147 -> 121
+//   bf16, d = 64, 16 heads    512 (16 x 256) 37 -> 43     512 (2 x 2048) 131 -> 116                    768 (12 x 512) 75 -> 70
+//   fp32, d = 64, 16 heads    256 (4 x 512) 208 -> 254    512 (4 x 1024) 706 -> 503
+inline bool bwd_pair_by_shape(bool narrow, bool ragged, int64_t pairs, int64_t n) {
+    if (!ragged) return true;
+    const int64_t tiles = pairs * n;
+    return narrow ? tiles > 640 || (tiles > 448 && n >= 16) : tiles > 320;
 }
 
 // Launch geometry of the dQ and dK/dV kernels (tiles, pairing, the map from workgroups to tiles); p.N, p.H and p.kv_group are set.
-inline int bwd_plan_launch(FlashBwdParams& p, int64_t B, bool causal, bool ragged, int rows = kFlashRows) {
+// narrow: 16-bit tensors at d = 64.
+inline int bwd_plan_launch(FlashBwdParams& p, int64_t B, bool causal, bool ragged, bool narrow, int rows = kFlashRows) {
     p.n_tiles = (p.N + rows - 1) / rows;
-    // causal launches: a workgroup takes a long and a short tile of its head, so that all (of a sequence) do the same work
-    p.paired = (causal && rows == kFlashRows && p.n_tiles >= 2 && tuning().bwd_pair.load() != 0) ? 1 : 0;
     p.n_bh = (int32_t)(B * p.H);
     constexpr int64_t kMostIds = 0x7FFFFFF0ll;
-    auto plan = [&](int64_t heads, int32_t& total, int32_t& per_xcd, int32_t& slices) {
-        const int64_t units = bwd_units(p), all = B * heads * units;
+    auto plan = [&](int64_t heads, int32_t& paired, int32_t& total, int32_t& per_xcd, int32_t& slices) {
+        const int64_t wanted = tuning().bwd_pair.load();
+        const bool two = causal && rows == kFlashRows && p.n_tiles >= 2 && wanted != 0;
+        paired = two && (wanted == 1 || bwd_pair_by_shape(narrow, ragged, B * heads, p.n_tiles)) ? 1 : 0;
+        const int64_t units = bwd_units(paired, p.n_tiles), all = B * heads * units;
         slices = ragged ? bwd_slices_for(heads) : 0;
         int64_t per = (all + 7) / 8;
         if (slices) {
@@ -127,7 +143,8 @@ inline int bwd_plan_launch(FlashBwdParams& p, int64_t B, bool causal, bool ragge
         per_xcd = (int32_t)per;
         return all <= kMostIds;
     };
-    if (!plan(p.H, p.total_q, p.per_xcd_q, p.slices_q) || !plan(p.H / p.kv_group, p.total_kv, p.per_xcd_kv, p.slices_kv)) return AHPC_ERR_BAD_SHAPE;
+    if (!plan(p.H, p.paired_q, p.total_q, p.per_xcd_q, p.slices_q)) return AHPC_ERR_BAD_SHAPE;
+    if (!plan(p.H / p.kv_group, p.paired_kv, p.total_kv, p.per_xcd_kv, p.slices_kv)) return AHPC_ERR_BAD_SHAPE;
     return AHPC_OK;
 }
 
@@ -219,7 +236,7 @@ __global__ __launch_bounds__(kFlashThreads, (D > 128 ? 1 : 2)) void flash_bwd_dq
     }
     // tiles of this sequence (a ragged batch hands every sequence as many units as the longest one needs)
     const int n_own = VARLEN ? (L + kFlashRows - 1) / kFlashRows : p.n_tiles;
-    if (VARLEN && work.tile >= bwd_units(p.paired, n_own)) return;
+    if (VARLEN && work.tile >= bwd_units(p.paired_q, n_own)) return;
     const T* const gq = static_cast<const T*>(p.q) + base;
     const T* const gdo = static_cast<const T*>(p.d_out) + base;
     const T* const gk = static_cast<const T*>(p.k) + kv_base;
@@ -271,7 +288,7 @@ __global__ __launch_bounds__(kFlashThreads, (D > 128 ? 1 : 2)) void flash_bwd_dq
         // long tiles first: under a causal mask the late query tiles walk the most keys; a paired workgroup then takes the
         // early tile that completes its share
         const int tile = part == 0 ? work.tile : n_own - 1 - work.tile;
-        if (part == 1 && (!p.paired || tile == work.tile)) break;
+        if (part == 1 && (!p.paired_q || tile == work.tile)) break;
         const int q_tile0 = (n_own - 1 - tile) * kFlashRows;
         if (part == 1) __syncthreads();  // every wavefront is done with the first pass's last tile
         int k_end = L;
@@ -458,7 +475,7 @@ __global__ __launch_bounds__(kFlashThreads, ((PART == 0 && D > 64) || D > 128 ? 
         L = p.cu_seqlens[b + 1] - seq0;
     }
     const int n_own = VARLEN ? (L + kFlashRows - 1) / kFlashRows : p.n_tiles;  // tiles of this sequence
-    if (VARLEN && work.tile >= bwd_units(p.paired, n_own)) return;
+    if (VARLEN && work.tile >= bwd_units(p.paired_kv, n_own)) return;
     const int64_t kv_base = VARLEN ? (int64_t)seq0 * p.kv_stride_n + (int64_t)hk * p.kv_stride_h
                                    : (int64_t)b * p.kv_stride_b + (int64_t)hk * p.kv_stride_h;
     const T* const gk = static_cast<const T*>(p.k) + kv_base;
@@ -489,7 +506,7 @@ __global__ __launch_bounds__(kFlashThreads, ((PART == 0 && D > 64) || D > 128 ? 
         // under a causal mask the early key tiles see the most queries: they go first; a paired workgroup then takes the
         // late tile that completes its share
         const int tile = part == 0 ? work.tile : n_own - 1 - work.tile;
-        if (part == 1 && (!p.paired || tile == work.tile)) break;
+        if (part == 1 && (!p.paired_kv || tile == work.tile)) break;
         const int k_tile0 = tile * kFlashRows;
         const int kw = k_tile0 + wave * 32;  // first key of this wavefront
         const int key = kw + col;

@@ -24,7 +24,7 @@ Tuning::Tuning()
       decode_matrix_min_group(env_value("AHPC_DECODE_MFMA_MIN_GROUP", 2)),
       bwd_split(env_value("AHPC_BWD_SPLIT", 0)),
       mask_pack(env_value("AHPC_MASK_PACK", 1)),
-      bwd_pair(env_value("AHPC_BWD_PAIR", 1)),
+      bwd_pair(env_value("AHPC_BWD_PAIR", 2)),
       flash_rows(env_value("AHPC_FLASH_ROWS", 0)),
       pool_in_place(env_value("AHPC_POOL_IN_PLACE", 1)) {
     if (flash_pair_min_tiles.load() < 1) flash_pair_min_tiles = kPairDefault;

@@ -31,8 +31,8 @@ struct Tuning {
     // front of the launch, into device memory the library keeps; 0 = the kernel reads the caller's fp32 mask in place
     // (what a stream under graph capture gets in any case).  (AHPC_MASK_PACK)
     std::atomic<int64_t> mask_pack;
-    // backward, causal launches: 1 (default) = the dQ and dK/dV workgroups take a long and a short tile of their
-    // head each (equal work for all), 0 = one tile per workgroup, long tiles first.  (AHPC_BWD_PAIR)
+    // backward, causal launches: 1 = the dQ and dK/dV workgroups take a long and a short tile of their head each (equal work
+    // for all), 0 = one tile per workgroup, long tiles first, 2 (default) = by shape (bwd_pair_by_shape).  (AHPC_BWD_PAIR)
     std::atomic<int64_t> bwd_pair;
     // forward on the 16-bit matrix-core kernel: query rows per workgroup, 128 (4 wavefronts, two workgroups per CU) or
     // 256 (8 wavefronts, one workgroup per CU: one stream of K/V tiles feeds twice the rows); fp32 forward: 128, or 32 (the

@@ -106,12 +106,12 @@ __global__ void dpp_sums(const float* in, float* out) {
 extern "C" {
 // The map of the backward's dQ (kv = 0) or dK/dV kernel: (sequence * heads + head, work unit) of every workgroup id, -1 for those
 // without work.  Returns the number of ids.
-int simt_bwd_block_map(int B, int N, int H, int H_kv, int causal, int ragged, int kv, int capacity, int* pair, int* unit, int* paired) {
+int simt_bwd_block_map(int B, int N, int H, int H_kv, int causal, int ragged, int narrow, int kv, int capacity, int* pair, int* unit, int* paired) {
     ahpc::FlashBwdParams p{};
     p.N = N; p.H = H; p.kv_group = H / H_kv;
-    if (ahpc::bwd_plan_launch(p, B, causal != 0, ragged != 0)) return -1;
+    if (ahpc::bwd_plan_launch(p, B, causal != 0, ragged != 0, narrow != 0)) return -1;
     const int n = 8 * (kv ? p.per_xcd_kv : p.per_xcd_q);
-    *paired = p.paired;
+    *paired = kv ? p.paired_kv : p.paired_q;
     for (int i = 0; i < n && n <= capacity; ++i) {
         const ahpc::BwdWork w = kv ? ahpc::bwd_work_kv((unsigned)i, p) : ahpc::bwd_work_q((unsigned)i, p);
         pair[i] = w.valid ? w.bh : -1;

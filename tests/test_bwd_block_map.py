@@ -9,10 +9,10 @@ import pytest
 from simt import simt as S
 
 
-def block_map(B, N, H, H_kv, causal, ragged, kv, capacity=1 << 20):
+def block_map(B, N, H, H_kv, causal, ragged, kv, narrow=False, capacity=1 << 20):
     lib = S.load()
     pair, unit, paired = np.empty(capacity, np.int32), np.empty(capacity, np.int32), C.c_int()
-    n = lib.simt_bwd_block_map(B, N, H, H_kv, int(causal), int(ragged), int(kv), capacity, C.c_void_p(pair.ctypes.data),
+    n = lib.simt_bwd_block_map(B, N, H, H_kv, int(causal), int(ragged), int(narrow), int(kv), capacity, C.c_void_p(pair.ctypes.data),
                                C.c_void_p(unit.ctypes.data), C.byref(paired))
     assert 0 <= n <= capacity
     return pair[:n], unit[:n], paired.value
@@ -22,12 +22,12 @@ SHAPES = [(1, 16384, 8, 1), (1, 4096, 8, 4), (3, 2048, 12, 3), (9, 3271, 8, 1), 
           (2, 100, 40, 40), (7, 1024, 6, 2)]
 
 
-@pytest.mark.parametrize("kv", [False, True])
+@pytest.mark.parametrize("kv,narrow", [(False, False), (True, False), (True, True)])
 @pytest.mark.parametrize("ragged", [False, True])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("B,N,H,H_kv", SHAPES)
-def test_every_unit_once_and_sequences_spread_over_the_xcds(B, N, H, H_kv, causal, ragged, kv):
-    pair, unit, paired = block_map(B, N, H, H_kv, causal, ragged, kv)
+def test_every_unit_once_and_sequences_spread_over_the_xcds(B, N, H, H_kv, causal, ragged, kv, narrow):
+    pair, unit, paired = block_map(B, N, H, H_kv, causal, ragged, kv, narrow)
     heads, tiles = H_kv if kv else H, (N + 127) // 128
     units = (tiles + 1) // 2 if paired else tiles
     valid = pair >= 0
@@ -44,3 +44,16 @@ def test_every_unit_once_and_sequences_spread_over_the_xcds(B, N, H, H_kv, causa
     # the first units of all sequences together (a batch of short sequences and one long one)
     share = np.bincount(xcd[valid & (unit == 0)], minlength=8)
     assert share.max() <= -(-B * heads // 8) + heads
+
+
+@pytest.mark.parametrize("B,N,H,narrow,ragged,paired", [
+    (1, 2048, 16, False, True, 0),   # 256 tiles: a CU for each
+    (5, 1024, 8, False, True, 0), (5, 1024, 8, False, False, 1), (4, 1024, 16, False, True, 1),
+    (16, 256, 16, True, True, 0), (2, 2048, 16, True, True, 1), (12, 512, 16, True, True, 1), (12, 512, 16, True, False, 1)])
+def test_small_ragged_launches_take_their_tiles_singly(B, N, H, narrow, ragged, paired):
+    for kv in (False, True):
+        assert block_map(B, N, H, H, True, ragged, kv, narrow)[2] == paired
+        assert block_map(B, N, H, H, False, ragged, kv, narrow)[2] == 0
+    # grouped heads: dQ and dK/dV count their own tiles
+    assert block_map(B, N, 8 * H, H, True, ragged, True, narrow)[2] == paired
+    assert block_map(B, N, 8 * H, H, True, ragged, False, narrow)[2] == 1

@@ -126,6 +126,10 @@ def test_dense(where, rows, dtype, B, N, H, H_kv, d, causal):
 @pytest.mark.parametrize("lens,H,H_kv,d,causal", RAGGED)
 def test_ragged(where, rows, dtype, lens, H, H_kv, d, causal):
     force(where, rows)
+    ragged_forward_and_backward(where, dtype, lens, H, H_kv, d, causal)
+
+
+def ragged_forward_and_backward(where, dtype, lens, H, H_kv, d, causal):
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     T, longest, n = int(cu[-1]), max(lens), len(lens)
     q, do = (O.round_to(O.fill_normal((T, H, d), 52, t), dtype) for t in (1, 7))
@@ -152,6 +156,21 @@ def test_ragged(where, rows, dtype, lens, H, H_kv, d, causal):
         for w, x in zip(want, parts):
             w[a:b] = np.asarray(x).reshape(L, *w.shape[1:])
     check([where.get(x, dtype) for x in (o, gq, gk, gv)], want, dtype)
+
+
+# The 16-bit backward of a ragged batch, tiles singly and in pairs: odd and even numbers of tiles, sequences of fewer than the
+# longest one's, an empty one; head counts whose pairs are dealt to the XCDs whole, in 2 and in 8 slices.
+@pytest.mark.parametrize("pair", [0, 1])
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16])
+@pytest.mark.parametrize("lens,H,H_kv,d,causal", [((130, 0, 1, 33), 2, 1, 64, True), ((300, 129, 0, 257), 4, 4, 128, True),
+                                                  ((31, 160), 8, 8, 96, True), ((200, 385), 3, 3, 64, False)])
+def test_ragged_backward_16_bit(where, pair, dtype, lens, H, H_kv, d, causal):
+    before = where.hip.get_tuning("bwd_pair")
+    where.hip.set_tuning("bwd_pair", pair)
+    try:
+        ragged_forward_and_backward(where, dtype, lens, H, H_kv, d, causal)
+    finally:
+        where.hip.set_tuning("bwd_pair", before)
 
 
 # The 16-bit forward whose workgroups walk the keys in two sets of wavefronts (launches of few tiles, more than 512 keys): odd
