@@ -511,7 +511,7 @@ static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, bool causal, f
     f.cu_seqlens = p.cu_seqlens;
     f.scale_log2 = p.scale_log2;
     f.d_real = p.d_real;
-    const bool split = f32_split_for(bwd_rows_wanted(), kSharedBackward, causal, VARLEN, B * p.H, p.kv_group, p.N);
+    const bool split = f32_split_backward(bwd_rows_wanted(), D, causal, VARLEN, B * p.H, p.kv_group, p.N);
     if (int rc = split ? flash_plan_launch(f, B, causal, kSplitRows, kNeverPair, VARLEN)
                        : flash_plan_launch(f, B, causal, kFlashRows, rows_128_pair_threshold(D, true, VARLEN, B, f), VARLEN)) return rc;
     const FlashStatsOut st{p.d_out, lse2, delta, p.rows_padded};

@@ -29,31 +29,51 @@ constexpr int kSplitWaves = 4;   // wavefronts that share its walk
 // Which fp32 launches run here.  Times in units of one 128-row tile's whole walk on a CU of its own, n = 128-row tiles of a
 // sequence, 256 CUs that hold the 128-row kernels' workgroups one at a time (two share the matrix cores and take twice as
 // long): the 128-row form takes a round per 256 workgroups, a causal pair (a long and a short tile) (n + 1) / n of a round;
-// the grouped heads of a dK/dV workgroup are walked one after the other.  This form spreads evenly, at `kShared` times the
-// work: it reads every operand from the caches.  Measured at H = 8 to 16, d = 64 (forward / backward, us, 128-row form ->
-// this one), where the model draws its line:
+// the grouped heads of a dK/dV workgroup are walked one after the other.  This form spreads evenly, at SplitCost::shared times
+// the work, since it reads every operand from the caches, plus per tile SplitCost::fixed steps of a walk (n steps) for the first loads
+// and the exchange, which short sequences feel; at d = 128 the forward has one workgroup per CU and nothing beside it hides them.
+// Ragged batches: tiles are counted from the longest sequence, lengths are not known here.  Where some tiles don't exist this
+// form gains evenly and the other by whole rounds; in the backward, where the other form's long walks weigh most, that is worth a fifth.
+// Measured at d = 64 (forward / backward, us, 128-row form -> this one), where the model draws its line:
 //     tiles  64 (2 x 512 x 8)     causal 38.7 -> 14.7 / 247 -> 60    not causal 38.3 -> 14.7 / 196 -> 60
 //     tiles 128 (2 x 1024 x 8)    causal 74 -> 47 / 432 -> 143       not causal 72 -> 49 / 372 -> 206
 //     tiles 256 (1 x 2048 x 16)   causal 144 -> 105 / 804 -> 434     not causal 139 -> 175 / 732 -> 751
 //     tiles 512 (2 x 2048 x 16)   causal 157 -> 206 / 923 -> 861     not causal 257 -> 341 / 1364 -> 1492
+// d = 128, forward:
+//     tiles 256                   causal 262 -> 190 (1 x 2048 x 16), 72 -> 86 (4 x 512 x 16)     not causal 73 -> 107 (4 x 512 x 16)
+//     ragged, 576 (12 of 100 to 400, 16 heads)     causal 86 -> 138     not causal 103 -> 191
+// Over 260 ragged and 236 dense shapes with 24 to 1500 tiles the form taken is 0.2 to 2 % slower than the better of the two
+// (geometric means by direction and d); on single ragged shapes, with half of the tiles missing or none, by up to 1.7 times.
 // `rows`: 32 or 128 forces a form (the tuning values flash_rows and bwd_split), anything else = by shape.  `group`: query heads
-// per K/V head where they are walked serially (backward), 1 otherwise.
-constexpr double kSharedForward = 1.35, kSharedBackward = 1.07;
-inline bool f32_split_for(int64_t rows, double shared, bool causal, bool ragged, int64_t pairs, int64_t group, int64_t N) {
+// per K/V head where they are walked serially (backward), 1 otherwise.  `pairs_tiles`: whether the 128-row form may pair tiles.
+struct SplitCost {
+    double shared, fixed;
+};
+inline SplitCost f32_split_forward_cost(int D) { return D > 64 ? SplitCost{1.25, 1.5} : SplitCost{1.45, 0.25}; }
+inline SplitCost f32_split_backward_cost(int D, bool ragged) { return ragged ? SplitCost{0.8, 1.0} : D > 64 ? SplitCost{1.07, 1.0} : SplitCost{1.0, 0.5}; }
+inline bool f32_split_for(int64_t rows, SplitCost cost, bool causal, bool pairs_tiles, int64_t pairs, int64_t group, int64_t N) {
     if (rows == kSplitRows) return true;
     if (rows == kFlashRows || rows == kFlashWideRows) return false;
     const int64_t n = (N + kFlashRows - 1) / kFlashRows, tiles = pairs * n;
-    if (ragged) return tiles <= 768;  // counted from the longest sequence: about half of them exist
     auto rounds = [](int64_t workgroups) { return (double)((workgroups + 255) / 256); };
     auto tile_form = [&](int64_t heads) {  // `heads` (sequence, head) pairs own the tiles
         const double single = rounds(heads * n);
-        if (!causal || n == 1) return single;
+        if (!causal || n == 1 || !pairs_tiles) return single;
         const double paired = rounds(heads * ((n + 1) / 2)) * (double)(n + 1) / (double)n;
         return single < paired ? single : paired;
     };
     const double there = group == 1 ? tile_form(pairs) : 0.5 * (tile_form(pairs) + (double)group * tile_form(pairs / group));
     const double walk = causal ? (double)(n + 1) / (double)(2 * n) : 1.0;
-    return shared * walk * (double)tiles / 256.0 < there;
+    return cost.shared * (walk + cost.fixed / (double)n) * (double)tiles / 256.0 < there;
+}
+// The forward of `pairs` (sequence, head) pairs (a ragged batch's 128-row launch pairs tiles from flash_pair_min_tiles of them on)
+// and the backward.
+inline bool f32_split_forward(int64_t rows, int D, bool causal, bool ragged, int64_t pairs, int64_t N) {
+    const bool pairs_tiles = !ragged || pairs * ((N + kFlashRows - 1) / kFlashRows) >= tuning().flash_pair_min_tiles.load();
+    return f32_split_for(rows, f32_split_forward_cost(D), causal, pairs_tiles, pairs, 1, N);
+}
+inline bool f32_split_backward(int64_t rows, int D, bool causal, bool ragged, int64_t pairs, int64_t group, int64_t N) {
+    return f32_split_for(rows, f32_split_backward_cost(D, ragged), causal, true, pairs, group, N);
 }
 
 // Loads of one tile of 32 rows of a [rows][d] tensor, first row `t0`, rows at or beyond L as zeros (columns from d_real on: see

@@ -450,7 +450,7 @@ static int launch_f32_split(FlashParams p, int64_t B, bool causal, hipStream_t s
 template <bool VARLEN, bool MASKED>
 static int launch_f32_mfma(FlashParams p, int64_t B, int d, bool causal, hipStream_t stream) {
     if constexpr (!MASKED) {
-        if (d <= 128 && f32_split_for(tuning().flash_rows.load(), kSharedForward, causal, VARLEN, B * p.H, 1, p.N))
+        if (d <= 128 && f32_split_forward(tuning().flash_rows.load(), d, causal, VARLEN, B * p.H, p.N))
             return d == 128 ? launch_f32_split<128, VARLEN>(p, B, causal, stream) : launch_f32_split<64, VARLEN>(p, B, causal, stream);
     }
     if (int rc = flash_plan_launch(p, B, causal, kFlashRows, rows_128_pair_threshold(d, true, VARLEN, B, p), VARLEN)) return rc;

@@ -6,6 +6,7 @@
 
 #include "ahpc_hip.h"
 #include "flash_bwd_mfma.hpp"
+#include "flash_f32_split.hpp"
 #include "flash_fwd_mfma.hpp"
 
 namespace {
@@ -104,6 +105,11 @@ __global__ void dpp_sums(const float* in, float* out) {
 }  // namespace
 
 extern "C" {
+// Whether an fp32 launch left to its shape takes the kernels of 32 rows (d: the kernels' head dimension, 64 or 128).
+int simt_f32_split(int backward, int d, int causal, int ragged, int B, int N, int H, int H_kv) {
+    return backward ? ahpc::f32_split_backward(0, d, causal != 0, ragged != 0, (int64_t)B * H, H / H_kv, N)
+                    : ahpc::f32_split_forward(0, d, causal != 0, ragged != 0, (int64_t)B * H, N);
+}
 // The map of the backward's dQ (kv = 0) or dK/dV kernel: (sequence * heads + head, work unit) of every workgroup id, -1 for those
 // without work.  Returns the number of ids.
 int simt_bwd_block_map(int B, int N, int H, int H_kv, int causal, int ragged, int narrow, int kv, int capacity, int* pair, int* unit, int* paired) {
