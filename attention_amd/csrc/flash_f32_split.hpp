@@ -69,7 +69,7 @@ inline bool f32_split_for(int64_t rows, SplitCost cost, bool causal, bool pairs_
 // The forward of `pairs` (sequence, head) pairs (a ragged batch's 128-row launch pairs tiles from flash_pair_min_tiles of them on)
 // and the backward.
 inline bool f32_split_forward(int64_t rows, int D, bool causal, bool ragged, int64_t pairs, int64_t N) {
-    const bool pairs_tiles = !ragged || pairs * ((N + kFlashRows - 1) / kFlashRows) >= tuning().flash_pair_min_tiles.load();
+    const bool pairs_tiles = !ragged || pairs * ((N + kFlashRows - 1) / kFlashRows) >= ragged_pair_threshold();
     return f32_split_for(rows, f32_split_forward_cost(D), causal, pairs_tiles, pairs, 1, N);
 }
 inline bool f32_split_backward(int64_t rows, int D, bool causal, bool ragged, int64_t pairs, int64_t group, int64_t N) {

@@ -580,7 +580,7 @@ int ahpc_hip_flash_block_map(int64_t B, int64_t N, int64_t H, int causal, int64_
     FlashParams p{};
     p.N = (int32_t)N; p.H = (int32_t)H; p.kv_group = 1;
     const int rows = tuning().flash_rows.load() == kFlashWideRows ? kFlashWideRows : kFlashRows;
-    if (int rc = flash_plan_launch(p, B, causal != 0, rows, tuning().flash_pair_min_tiles.load())) return rc;
+    if (int rc = flash_plan_launch(p, B, causal != 0, rows, ragged_pair_threshold())) return rc;
     const int64_t grid = (int64_t)p.blocks_per_xcd * 8;
     *n_blocks = grid;
     if (!seq_head && !first_tile && !second_tile) return AHPC_OK;

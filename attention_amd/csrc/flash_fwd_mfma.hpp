@@ -851,7 +851,7 @@ inline bool flash_pair_by_shape(int D, bool f32, int64_t seq_heads, int64_t n) {
 
 // The threshold the launchers of the 128-row kernels hand to flash_plan_launch (p.N and p.H are set).
 inline int64_t rows_128_pair_threshold(int D, bool f32, bool ragged, int64_t B, const FlashParams& p) {
-    if (ragged) return tuning().flash_pair_min_tiles.load();
+    if (ragged) return ragged_pair_threshold();
     return pair_threshold(flash_pair_by_shape(D, f32, B * p.H, (p.N + kFlashRows - 1) / kFlashRows));
 }
 

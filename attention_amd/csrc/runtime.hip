@@ -18,7 +18,7 @@ static int64_t env_value(const char* name, int64_t dflt) {
 }
 
 Tuning::Tuning()
-    : flash_pair_min_tiles(env_value("AHPC_FLASH_PAIR_MIN", kPairDefault)),
+    : flash_pair_min_tiles(env_value("AHPC_FLASH_PAIR_MIN", 0)),
       decode_waves(env_value("AHPC_DECODE_WAVES", 0)),
       decode_chunk(env_value("AHPC_DECODE_CHUNK", 0)),
       decode_matrix_min_group(env_value("AHPC_DECODE_MFMA_MIN_GROUP", 2)),
@@ -27,7 +27,7 @@ Tuning::Tuning()
       bwd_pair(env_value("AHPC_BWD_PAIR", 2)),
       flash_rows(env_value("AHPC_FLASH_ROWS", 0)),
       pool_in_place(env_value("AHPC_POOL_IN_PLACE", 1)) {
-    if (flash_pair_min_tiles.load() < 1) flash_pair_min_tiles = kPairDefault;
+    if (flash_pair_min_tiles.load() < 0) flash_pair_min_tiles = 0;
 }
 
 Tuning& tuning() {

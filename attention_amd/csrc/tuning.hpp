@@ -11,7 +11,8 @@ namespace ahpc {
 
 struct Tuning {
     // forward, causal: a workgroup takes a late query tile and then an early one once the launch has at least
-    // this many query tiles (AHPC_FLASH_PAIR_MIN; the default, 1024, leaves dense launches to their shape)
+    // this many query tiles; 0 (default) = by shape in dense launches, from 1024 tiles on in ragged ones.  The kernels that
+    // share a workgroup's walk out (two walks, fp32 with 32 rows) never pair.  (AHPC_FLASH_PAIR_MIN)
     std::atomic<int64_t> flash_pair_min_tiles;
     // decode: wavefronts per workgroup, 1..8 (AHPC_DECODE_WAVES, default 0 = the launcher's choice)
     std::atomic<int64_t> decode_waves;
@@ -48,11 +49,16 @@ struct Tuning {
 Tuning& tuning();
 
 // Thresholds of query tiles for flash_plan_launch.
-constexpr int64_t kPairDefault = 1024, kAlwaysPair = 1, kNeverPair = int64_t(1) << 40;
+constexpr int64_t kAlwaysPair = 1, kNeverPair = int64_t(1) << 40;
 // The threshold of a dense launch: the tuning value when it was set, else what the launch's shape asks for.
 inline int64_t pair_threshold(bool paired_by_shape) {
     const int64_t t = tuning().flash_pair_min_tiles.load();
-    return t != kPairDefault ? t : paired_by_shape ? kAlwaysPair : kNeverPair;
+    return t > 0 ? t : paired_by_shape ? kAlwaysPair : kNeverPair;
+}
+// Of a ragged batch: two rounds of two workgroups on each of 256 CUs (its own shape is not known on the host).
+inline int64_t ragged_pair_threshold() {
+    const int64_t t = tuning().flash_pair_min_tiles.load();
+    return t > 0 ? t : 1024;
 }
 
 }  // namespace ahpc

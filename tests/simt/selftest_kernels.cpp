@@ -105,6 +105,13 @@ __global__ void dpp_sums(const float* in, float* out) {
 }  // namespace
 
 extern "C" {
+// Whether a causal forward launch of the 128-row kernels takes its tiles in pairs (d: the kernels' head dimension).
+int simt_flash_paired(int d, int f32, int ragged, int B, int N, int H) {
+    ahpc::FlashParams p{};
+    p.N = N; p.H = H; p.kv_group = 1;
+    if (ahpc::flash_plan_launch(p, B, true, ahpc::kFlashRows, ahpc::rows_128_pair_threshold(d, f32 != 0, ragged != 0, B, p), ragged != 0)) return -1;
+    return p.paired;
+}
 // Whether an fp32 launch left to its shape takes the kernels of 32 rows (d: the kernels' head dimension, 64 or 128).
 int simt_f32_split(int backward, int d, int causal, int ragged, int B, int N, int H, int H_kv) {
     return backward ? ahpc::f32_split_backward(0, d, causal != 0, ragged != 0, (int64_t)B * H, H / H_kv, N)

@@ -66,3 +66,23 @@ def test_rejects_bad_shapes_without_a_gpu():
     assert hip.load().ahpc_hip_flash_block_map(1, 16, 4, 0, 0, None, None, None, None) == -1
     buf = np.empty(4, np.int32)
     assert hip.load().ahpc_hip_flash_block_map(4, 4096, 32, 1, 4, C.byref(n), buf.ctypes.data, buf.ctypes.data, buf.ctypes.data) == -2
+
+
+@pytest.fixture
+def pair_line():
+    from simt import simt as S
+    lib = S.load()
+    hip = S.EmulatedHip()
+    before = hip.get_tuning("flash_pair_min_tiles")
+    yield lambda n, *shape: (hip.set_tuning("flash_pair_min_tiles", n), lib.simt_flash_paired(*shape))[1]
+    hip.set_tuning("flash_pair_min_tiles", before)
+
+
+def test_every_pairing_line_that_is_named_holds(pair_line):
+    """512 tiles, which the shape would pair, and 1152: the default's old value, 1024, is a line like any other."""
+    assert pair_line(0, 128, 0, 0, 4, 2048, 8) == 1 and pair_line(0, 128, 0, 1, 4, 2048, 8) == 0
+    for line in (1023, 1024, 1025):
+        for f32, ragged in ((0, 0), (1, 0), (0, 1), (1, 1)):
+            assert pair_line(line, 128, f32, ragged, 4, 2048, 8) == 0
+            assert pair_line(line, 128, f32, ragged, 9, 2048, 8) == 1
+    assert pair_line(1, 128, 0, 1, 1, 129, 1) == 1
