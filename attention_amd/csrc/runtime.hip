@@ -26,6 +26,7 @@ Tuning::Tuning()
       mask_pack(env_value("AHPC_MASK_PACK", 1)),
       bwd_pair(env_value("AHPC_BWD_PAIR", 2)),
       flash_rows(env_value("AHPC_FLASH_ROWS", 0)),
+      flash_walks(env_value("AHPC_FLASH_WALKS", 0)),
       pool_in_place(env_value("AHPC_POOL_IN_PLACE", 1)) {
     if (flash_pair_min_tiles.load() < 0) flash_pair_min_tiles = 0;
 }
@@ -46,6 +47,7 @@ static std::atomic<int64_t>* tuning_slot(const char* name) {
     if (!std::strcmp(name, "mask_pack")) return &t.mask_pack;
     if (!std::strcmp(name, "bwd_pair")) return &t.bwd_pair;
     if (!std::strcmp(name, "flash_rows")) return &t.flash_rows;
+    if (!std::strcmp(name, "flash_walks")) return &t.flash_walks;
     if (!std::strcmp(name, "pool_in_place")) return &t.pool_in_place;
     return nullptr;
 }

@@ -39,6 +39,9 @@ struct Tuning {
     // 256 (8 wavefronts, one workgroup per CU: one stream of K/V tiles feeds twice the rows); fp32 forward: 128, or 32 (the
     // wavefronts of a workgroup share the walk over the keys); 0 (default) = by shape.  (AHPC_FLASH_ROWS)
     std::atomic<int64_t> flash_rows;
+    // forward on the 16-bit matrix-core kernel with 128 rows, no mask, d <= 128: 1 = one set of wavefronts per workgroup, 2 = two that
+    // share the walk over the keys, 0 (default) = by shape.  (AHPC_FLASH_WALKS)
+    std::atomic<int64_t> flash_walks;
     // KV block pool (host class): 1 (default) = slabs are address ranges that grow in place where the device has virtual
     // memory management; 0 = plain allocations that grow by reallocation and a device copy.  Read when a pool is
     // created.  (AHPC_POOL_IN_PLACE)

@@ -71,6 +71,7 @@ def test_fp32(where, rows, low, causal):  # noqa: F811
 @pytest.mark.parametrize("dtype", [O.BF16])
 def test_16_bit(where, dtype, low, rows, N, d, causal):  # noqa: F811
     where.hip.set_tuning("flash_rows", rows)
+    where.hip.set_tuning("flash_walks", 2 if rows == 0 else 1)
     H = 1
     x = inputs(dtype, N, H, d, low)
     check(run(where, dtype, N, H, d, causal, *x), *x, dtype, N, H, d, causal)

@@ -79,7 +79,7 @@ def where(request):
         w = Gpu(request.getfixturevalue("gpu"))
     else:
         w = Executor()
-    before = {n: w.hip.get_tuning(n) for n in ("flash_rows", "bwd_split", "flash_pair_min_tiles")}
+    before = {n: w.hip.get_tuning(n) for n in ("flash_rows", "flash_walks", "bwd_split", "flash_pair_min_tiles")}
     yield w
     for n, v in before.items():
         w.hip.set_tuning(n, v)
@@ -173,9 +173,10 @@ def test_ragged_backward_16_bit(where, pair, dtype, lens, H, H_kv, d, causal):
         where.hip.set_tuning("bwd_pair", before)
 
 
-# The 16-bit forward whose workgroups walk the keys in two sets of wavefronts (launches of few tiles, more than 512 keys): odd
-# and even numbers of key tiles, a last tile of one row, one that only the second set has, head dimensions below the kernel's.
-WALKS = [(1, 513, 2, 2, 64, True), (1, 577, 2, 1, 128, False), (2, 640, 2, 1, 96, True), (1, 769, 4, 2, 40, True), (1, 705, 1, 1, 128, True)]
+# The 16-bit forward whose workgroups walk the keys in two sets of wavefronts (by itself in launches of few tiles, more than 512
+# keys; named here): odd and even numbers of key tiles, one tile, a last tile of one row, one that only the second set has, head
+# dimensions below the kernel's.
+WALKS = [(1, 50, 2, 1, 64, True), (2, 65, 1, 1, 128, False), (1, 129, 2, 2, 64, True), (1, 513, 2, 2, 64, True), (1, 577, 2, 1, 128, False), (2, 640, 2, 1, 96, True), (1, 769, 4, 2, 40, True), (1, 705, 1, 1, 128, True)]
 
 
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16])
@@ -188,8 +189,8 @@ def test_two_walks_dense(where, dtype, B, N, H, H_kv, d, causal):
     scale, st, kst = 1.0 / np.sqrt(d), (N * H * d, H * d, d), (N * H_kv * d, H_kv * d, d)
     n_st = where.hip.flash_row_stats_bytes(B, N, H)
     got, stats = [], []
-    for rows in (0, 128):  # by shape (two walks), and the one-walk form
-        where.hip.set_tuning("flash_rows", rows)
+    for walks in (2, 1):
+        where.hip.set_tuning("flash_walks", walks)
         (o, po), (ws, pws) = where.out(q.shape, dtype), where.scratch(n_st)
         assert where.hip.flash_fwd_keep(pq, pk, pv, po, dtype, B, N, H, H_kv, d, st, kst, scale, causal, pws)
         got.append(where.get(o, dtype))
@@ -198,13 +199,16 @@ def test_two_walks_dense(where, dtype, B, N, H, H_kv, d, causal):
     want = O.attention(q, np.repeat(k, rep, axis=2), np.repeat(v, rep, axis=2), B, N, H, d, scale, causal)
     check(got[:1], [want], dtype)
     check(got[1:], [want], dtype)
+    if N > 512:
+        assert not np.array_equal(got[0], got[1])  # two forms ran: their weights are rounded against different maxima
     # log2 of sums of up to N fp32 terms in two orders (N * 2^-24 / ln 2), and the reference maxima's own rounding (|m| < 64: 2^-18)
     assert np.abs(stats[0] - stats[1]).max() <= N * 2.0**-23 + 2.0**-16
 
 
-@pytest.mark.parametrize("lens,H,H_kv,d,causal", [((513, 0, 1, 65), 2, 1, 64, True), ((64, 600, 130), 2, 2, 128, False), ((300, 577, 16), 2, 1, 80, True)])
+@pytest.mark.parametrize("lens,H,H_kv,d,causal", [((513, 0, 1, 65), 2, 1, 64, True), ((64, 2, 128), 2, 2, 64, False), ((64, 600, 130), 2, 2, 128, False), ((300, 577, 16), 2, 1, 80, True)])
 def test_two_walks_ragged(where, lens, H, H_kv, d, causal):
     dtype = O.BF16
+    where.hip.set_tuning("flash_walks", 2)
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     T, longest, n = int(cu[-1]), max(lens), len(lens)
     q = O.round_to(O.fill_normal((T, H, d), 54, 1), dtype)
