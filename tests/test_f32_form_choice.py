@@ -24,6 +24,8 @@ TIMED = [
     (BACKWARD, 64, False, RAGGED, 12, 512, 16, 16, False),  # 561        656
     (BACKWARD, 64, True, RAGGED, 8, 904, 8, 8, True),       # 417        201
     (BACKWARD, 128, True, RAGGED, 4, 1024, 8, 2, True),     # 1885       574
+    (BACKWARD, 128, False, RAGGED, 9, 1024, 16, 16, False),  # 3135       3536
+    (BACKWARD, 128, True, RAGGED, 25, 512, 12, 12, False),  # 1327       1788
 ]
 
 
