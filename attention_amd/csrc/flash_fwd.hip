@@ -272,7 +272,7 @@ static int dispatch_mfma_masked(const FlashParams& p, int64_t B, int d, bool cau
 // With bits_t given the same pass also writes the transposed layout the backward's dK/dV kernels read: word
 // [(b * n_rb + query block) * N + key] holds the block's 64 queries, bit r set = mask[b][64 * block + r][key] != 0
 // (lane = key collects its wavefront's 16 bits of that word from the values it loads).
-// live: one byte per wavefront's share of a tile, whether anything of it stays (PackedMask::live).
+// live: each wavefront writes its byte of the tile's word, whether anything of its share stays (PackedMask::live).
 // Bound by the read of the mask, hence 16 rows per wavefront and no condition around a load (rows and keys behind the end
 // re-read the last ones): all 16 are in flight together, and a launch has four times the wavefronts of one that takes 64 rows
 // in turn with each load under its condition.  Mask [4,1001,1001]: 30.8 -> 6.1 us (16 MB).

@@ -838,7 +838,7 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
 //   16-bit, d = 256    256 (1 x 2048 x 16) 91.6 -> 102     384 (2 x 1024 x 24) 79.9 -> 64.2    512 (16 x 256 x 16) 43.6 -> 40.5
 //   16-bit, d = 64 (three workgroups to a CU even out by themselves)    512 (4 x 1024 x 16) 18.8 -> 19.1    768 (3 x 1024 x 32) 27.2 -> 24.7
 // Just above a full round of pairs (512 for two workgroups per CU) single tiles fill the second round better: d = 128,
-// 2048 tokens x 72 heads (576 pairs) 106.5 -> 95.5 us.
+// 2048 tokens x 72 heads (576 pairs) 106.5 -> 95.5 us, the one launch timed between 512 and 620 pairs.
 inline bool flash_pair_by_shape(int D, bool f32, int64_t seq_heads, int64_t n) {
     const int64_t tiles = seq_heads * n, pairs = seq_heads * ((n + 1) / 2);
     if (n < 2) return false;

@@ -12,8 +12,8 @@ namespace ahpc {
 //   bits   [(b * tiles + key tile) * N + query]    the tile's 64 keys of one query   (bit j = key 64 * tile + j stays)
 //   bits_t [(b * tiles + query block) * N + key]   the block's 64 queries of one key (bit r = query 64 * block + r sees the key);
 //          null unless asked for
-//   live   [(b * tiles + query block) * tiles + key tile] byte w: the tile's keys and queries 16 * w .. 16 * w + 15 of the
-//          block share a pair that stays (0: a kernel may pass the tile by for them)
+//   live   [(b * tiles + query block) * tiles + key tile] nonzero: some pair of the tile's 64 keys and the block's 64 queries
+//          stays (0: a kernel may pass the tile by).  The bytes are the four packing wavefronts' shares.
 struct PackedMask {
     const uint64_t* bits;
     const uint64_t* bits_t;

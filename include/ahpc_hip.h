@@ -188,9 +188,11 @@ int ahpc_hip_flash_fwd_varlen_gqa(const void* q, const void* k, const void* v, v
  * uses (no GPU needed): for a dense fp16/bf16 launch of B sequences, N tokens, H heads it reports the grid
  * size in *n_blocks and, when the three arrays (capacity entries each) are given, for every workgroup id
  * its (sequence * H + head), the query tile it handles first and the one it handles second (-1 = none; all -1
- * for padding workgroups).  Tiles are 128 query rows, or 256 while the tuning value "flash_rows" is 256 (the
- * launcher itself takes 256 rows at d = 128 for dense launches of at least 2048 tokens that fill the chip).  Lets a test check that every query tile of every head is
- * handled exactly once, whatever the pairing and interleaving in force.  No counterpart in the reference
+ * for padding workgroups).  Tiles are 128 query rows, or 256 while the tuning value "flash_rows" is 256, and causal
+ * launches pair tiles from "flash_pair_min_tiles" of them on (0: from 1024).  A launch is one of these maps: which rows
+ * it takes and whether it pairs, where the tuning values leave that open, depends on d, the type and the shape, which
+ * this function is not told.  Lets a test check that every query tile of every head is
+ * handled exactly once, in either row count, paired or not.  No counterpart in the reference
  * (its kernels are launched one tile per block, src/backends/cuda/cuda_kernels.cu:125-127). */
 int ahpc_hip_flash_block_map(int64_t B, int64_t N, int64_t H, int causal, int64_t capacity, int64_t* n_blocks,
                              int32_t* seq_head, int32_t* first_tile, int32_t* second_tile);

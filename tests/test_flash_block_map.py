@@ -58,6 +58,23 @@ def test_map_of_256_row_workgroups_covers_every_tile_once(B, N, H, causal):
         hip.set_tuning("flash_rows", before)
 
 
+@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("line", [1, 1 << 40])
+@pytest.mark.parametrize("B,N,H", SHAPES + [(2, 2048, 12), (4, 1024, 16), (9, 1152, 8), (3, 1000, 32)])
+def test_map_covers_every_tile_once_paired_and_single(B, N, H, line, rows):
+    """Every map a causal launch can take: which of them it takes is a matter of d, type and shape."""
+    from attention_amd import hip
+    before = {n: hip.get_tuning(n) for n in ("flash_rows", "flash_pair_min_tiles")}
+    hip.set_tuning("flash_rows", rows)
+    hip.set_tuning("flash_pair_min_tiles", line)
+    try:
+        _, _, second = check_exact_cover(B, N, H, True, ROWS=rows)
+        assert (second >= 0).any() == (line == 1 and N > rows)
+    finally:
+        for n, v in before.items():
+            hip.set_tuning(n, v)
+
+
 def test_rejects_bad_shapes_without_a_gpu():
     from attention_amd import hip
     import ctypes as C
