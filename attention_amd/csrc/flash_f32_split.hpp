@@ -249,8 +249,8 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) oacc[mb] = neg_m;
     float l_run = 0.0f;
-    bool seen = false;  // this lane's query has met a key of finite score in this wavefront's tiles
     constexpr float kRaise = 8.0f;  // the reference maximum is raised only when exceeded by 2^8 (flash_fwd_mfma.hpp)
+    float raise = -INFINITY;        // kRaise once this lane's query has met a key of finite score in this wavefront's tiles
 
     for (int t = wave_u; t < n_tiles; t += kSplitWaves) {
         const int k0 = t * kF32Keys;
@@ -273,13 +273,14 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
 #pragma unroll
         for (int r = 3; r < 15; r += 2) mx = max3(mx, s[r], s[r + 1]);
         mx = max3(mx, s[15], s[15]);
-        if (__builtin_amdgcn_ballot_w64(seen ? mx > kRaise : mx > -INFINITY) != 0) {
+        if (__builtin_amdgcn_ballot_w64(mx > raise) != 0) {
             mx = halves_max(mx);  // both lanes of a query agree
             // the first maximum is set exactly and rescales nothing: 2^-delta of scores below -128 overflows, and times the empty
             // accumulators that is not a number, in any of the four walks
+            const bool seen = raise > 0.0f;
             const float delta = seen ? fmaxf(mx, 0.0f) : (mx > -INFINITY ? mx : 0.0f);
             const float alpha = seen ? fast_exp2(-delta) : 1.0f;
-            seen = seen || mx > -INFINITY;
+            raise = seen || mx > -INFINITY ? kRaise : raise;
             l_run *= alpha;
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
@@ -308,7 +309,7 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
     {
         const float l = halves_sum(l_run);
         if (half == 0) {
-            lds_m[wave][col] = seen ? -neg_m[0] : -INFINITY;  // (a wavefront without a tile)
+            lds_m[wave][col] = raise > 0.0f ? -neg_m[0] : -INFINITY;  // (a wavefront without a tile)
             lds_l[wave][col] = l;
         }
         X::put(lds, oacc, wave, lane);

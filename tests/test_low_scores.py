@@ -75,3 +75,24 @@ def test_16_bit(where, dtype, low, rows, N, d, causal):  # noqa: F811
     H = 1
     x = inputs(dtype, N, H, d, low)
     check(run(where, dtype, N, H, d, causal, *x), *x, dtype, N, H, d, causal)
+
+
+@pytest.mark.parametrize("dtype,rows,N,d,tile", [(O.F32, 32, 130, 64, 0), (O.F32, 32, 130, 64, 1), (O.F32, 32, 130, 128, 3), (O.F32, 128, 130, 64, 1),
+                                                 (O.BF16, 0, 577, 64, 0), (O.BF16, 0, 577, 128, 1), (O.BF16, 128, 130, 64, 1)])
+def test_a_tile_of_infinitely_low_scores(where, dtype, rows, N, d, tile):  # noqa: F811
+    """Keys that an infinity in K takes out altogether: a tile of them, also as the first one a set of wavefronts meets."""
+    where.hip.set_tuning("flash_rows", rows)
+    where.hip.set_tuning("flash_walks", 2 if rows == 0 else 1)
+    q, k, v, _ = inputs(dtype, N, 1, d, None)
+    k[..., 0] = 0.0
+    k[:, TILE[dtype] * tile:TILE[dtype] * (tile + 1), :, 0] = -np.inf
+    (tq, pq), (tk, pk), (tv, pv), (o, po) = *(where.put(x, dtype) for x in (q, k, v)), where.out(q.shape, dtype)
+    scale, st = 1.0 / np.sqrt(d), (N * d, d, d)
+    where.hip.flash_fwd_gqa(pq, pk, pv, po, dtype, 1, N, 1, 1, d, st, st, scale, False)
+    keep = np.r_[0:TILE[dtype] * tile, min(N, TILE[dtype] * (tile + 1)):N]
+    s = q[0, :, 0].astype(np.float64) @ k[0, keep, 0].astype(np.float64).T * scale
+    w = np.exp(s - s.max(1, keepdims=True))
+    want = (w / w.sum(1, keepdims=True)) @ v[0, keep, 0].astype(np.float64)
+    got = where.get(o, dtype)[0, :, 0]
+    assert np.isfinite(got).all()
+    assert np.abs(got - want).max() <= TOL[dtype] * max(1.0, np.abs(want).max())
