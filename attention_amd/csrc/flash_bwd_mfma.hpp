@@ -68,22 +68,25 @@ struct FlashBwdParams {
 // of one head (consecutive logical ids) run on one XCD and find the head's K/V (Q/dO) in its L2.
 // Ragged batches: equal shares of the id range are not equal shares of the work, so the pairs are dealt out.  A pair's tiles
 // (as many ids as the longest sequence needs; a workgroup beyond its own sequence's tiles exits) go in turn to `slices`
-// slices, and slice i runs on XCD i % 8.  heads * slices is a multiple of 8 (bwd_slices_for): every sequence, however long, is
-// spread evenly over the XCDs.  Which slice holds the pair's first tile rotates with the round of eight, so that sequences of
-// a tile or two don't meet on the same XCD.  Whole backward, us, in equal shares of the id range / a whole pair per XCD / this:
-//   12 sequences of 100 to 2000 tokens, 16 heads over 4, d = 64, causal   385 / 289 / 291    full 630 / 382 / 377
-//   one of 16384, 8 heads over 1, d = 128                                full 5518 / 16265 / 5598 (one XCD at work in the second)
-//   16384 and 700, 32 heads over 2, d = 64                             causal 10738 / 9884 / 6531
-//   9000, 800 and 5000, 4 heads, d = 128                               causal 1189 / 1039 / 691
+// slices, and slice i runs on XCD i % 8.  Which slice holds the pair's first tile rotates with the round of eight, so that
+// sequences of a tile or two don't meet on the same XCD.
 struct BwdWork {
     int bh, tile;
     bool valid;
 };
 // work units per head: tiles, or pairs of them
 __host__ __device__ inline int bwd_units(int paired, int n_tiles) { return paired ? (n_tiles + 1) >> 1 : n_tiles; }
-inline int bwd_slices_for(int64_t heads) {
+// A whole pair per XCD shares its other side's tiles in one L2, and short sequences have few tiles to deal out (sequences of up to 340
+// tokens, 12 heads: 660 us whole, 735 in two slices), so a pair is cut only as far as it takes to keep three quarters of the XCDs
+// busy: launches of fewer than 6 and of 9 to 11 pairs.  Up to three sequences of 24 tiles and more are taken one by one: any of them
+// may be most of the work.  Over 150 ragged batches never slower than whole pairs by more than 2 %.  Whole backward, us, in equal
+// shares of the id range / a whole pair per XCD / this:
+//   12 sequences of 100 to 2000 tokens, 16 heads over 4, d = 64, causal   385 / 289 / 289    full 630 / 382 / 382
+//   one of 16384, 8 heads over 1, d = 128                                full 5518 / 16265 / 5598 (one XCD at work in the second)
+inline int bwd_slices_for(int64_t B, int64_t heads, int64_t N) {
+    const int64_t pairs = B <= 3 && N > 23 * kFlashRows ? heads : B * heads;
     int slices = 1;
-    while ((heads * slices) % 8) slices *= 2;
+    while (slices < 8 && (pairs * slices + 7) / 8 * 8 * 3 > pairs * slices * 4) slices *= 2;
     return slices;
 }
 __host__ __device__ inline BwdWork bwd_work_of_block(unsigned block_id, int total, int per_xcd, int n_units, int n_pairs, int slices) {
@@ -132,7 +135,7 @@ inline int bwd_plan_launch(FlashBwdParams& p, int64_t B, bool causal, bool ragge
         const bool two = causal && rows == kFlashRows && p.n_tiles >= 2 && wanted != 0;
         paired = two && (wanted == 1 || bwd_pair_by_shape(narrow, ragged, B * heads, p.n_tiles)) ? 1 : 0;
         const int64_t units = bwd_units(paired, p.n_tiles), all = B * heads * units;
-        slices = ragged ? bwd_slices_for(heads) : 0;
+        slices = ragged ? bwd_slices_for(B, heads, p.N) : 0;
         int64_t per = (all + 7) / 8;
         if (slices) {
             const int64_t dealt = (B * heads * slices + 7) / 8 * ((units + slices - 1) / slices);
