@@ -34,7 +34,8 @@ constexpr int kSplitWaves = 4;   // wavefronts that share its walk
 // and the exchange, which short sequences feel; at d = 128 the forward has one workgroup per CU and nothing beside it hides them.
 // Ragged batches: tiles are counted from the longest sequence, lengths are not known here.  Where some tiles don't exist this
 // form gains evenly and the other by whole rounds; in the backward, where the other form's long walks weigh most, that is worth a fifth
-// up to 1024 tiles.
+// up to 1024 tiles (768 for sequences of at most three tiles, whose walks aren't long: 11 of up to 264 tokens, 24 heads over 12, d = 128,
+// 792 tiles, 482 -> 628).
 // Measured at d = 64 (forward / backward, us, 128-row form -> this one), where the model draws its line:
 //     tiles  64 (2 x 512 x 8)     causal 38.7 -> 14.7 / 247 -> 60    not causal 38.3 -> 14.7 / 196 -> 60
 //     tiles 128 (2 x 1024 x 8)    causal 74 -> 47 / 432 -> 143       not causal 72 -> 49 / 372 -> 206
@@ -51,8 +52,8 @@ struct SplitCost {
     double shared, fixed;
 };
 inline SplitCost f32_split_forward_cost(int D) { return D > 64 ? SplitCost{1.25, 1.5} : SplitCost{1.45, 0.25}; }
-inline SplitCost f32_split_backward_cost(int D, bool ragged, int64_t tiles) {
-    if (ragged && tiles <= 1024) return SplitCost{0.8, 1.0};
+inline SplitCost f32_split_backward_cost(int D, bool ragged, int64_t n, int64_t tiles) {
+    if (ragged && tiles <= (n > 3 ? 1024 : 768)) return SplitCost{0.8, 1.0};
     return D > 64 ? SplitCost{1.07, 1.0} : SplitCost{1.0, 0.5};
 }
 inline bool f32_split_for(int64_t rows, SplitCost cost, bool causal, bool pairs_tiles, int64_t pairs, int64_t group, int64_t N) {
@@ -77,8 +78,8 @@ inline bool f32_split_forward(int64_t rows, int D, bool causal, bool ragged, int
     return f32_split_for(rows, f32_split_forward_cost(D), causal, pairs_tiles, pairs, 1, N);
 }
 inline bool f32_split_backward(int64_t rows, int D, bool causal, bool ragged, int64_t pairs, int64_t group, int64_t N) {
-    const int64_t tiles = pairs * ((N + kFlashRows - 1) / kFlashRows);
-    return f32_split_for(rows, f32_split_backward_cost(D, ragged, tiles), causal, true, pairs, group, N);
+    const int64_t n = (N + kFlashRows - 1) / kFlashRows;
+    return f32_split_for(rows, f32_split_backward_cost(D, ragged, n, pairs * n), causal, true, pairs, group, N);
 }
 
 // Loads of one tile of 32 rows of a [rows][d] tensor, first row `t0`, rows at or beyond L as zeros (columns from d_real on: see

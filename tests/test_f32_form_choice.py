@@ -26,6 +26,7 @@ TIMED = [
     (BACKWARD, 128, True, RAGGED, 4, 1024, 8, 2, True),     # 1885       574
     (BACKWARD, 128, False, RAGGED, 9, 1024, 16, 16, False),  # 3135       3536
     (BACKWARD, 128, True, RAGGED, 25, 512, 12, 12, False),  # 1327       1788
+    (BACKWARD, 128, False, RAGGED, 11, 264, 24, 12, False),  # 482        628
 ]
 
 
