@@ -48,6 +48,8 @@ constexpr int kSplitWaves = 4;   // wavefronts that share its walk
 // (geometric means by direction and d); on single ragged shapes, with half of the tiles missing or none, by up to 1.7 times.
 // `rows`: 32 or 128 forces a form (the tuning values flash_rows and bwd_split), anything else = by shape.  `group`: query heads
 // per K/V head where they are walked serially (backward), 1 otherwise.  `pairs_tiles`: whether the 128-row form may pair tiles.
+// `single`: what rounds of single causal tiles take of whole ones; 2/3 in the dense forward from 257 to 400 pairs, where single tiles are what
+// flash_pair_by_shape leaves and their short walks fill the second round (d = 64, 432 tiles, 3 per sequence: 47 us, 65 here).
 struct SplitCost {
     double shared, fixed;
 };
@@ -56,16 +58,16 @@ inline SplitCost f32_split_backward_cost(int D, bool ragged, int64_t n, int64_t 
     if (ragged && tiles <= (n > 3 ? 1024 : 768)) return SplitCost{0.8, 1.0};
     return D > 64 ? SplitCost{1.07, 1.0} : SplitCost{1.0, 0.5};
 }
-inline bool f32_split_for(int64_t rows, SplitCost cost, bool causal, bool pairs_tiles, int64_t pairs, int64_t group, int64_t N) {
+inline bool f32_split_for(int64_t rows, SplitCost cost, bool causal, bool pairs_tiles, double single, int64_t pairs, int64_t group, int64_t N) {
     if (rows == kSplitRows) return true;
     if (rows == kFlashRows || rows == kFlashWideRows) return false;
     const int64_t n = (N + kFlashRows - 1) / kFlashRows, tiles = pairs * n;
     auto rounds = [](int64_t workgroups) { return (double)((workgroups + 255) / 256); };
     auto tile_form = [&](int64_t heads) {  // `heads` (sequence, head) pairs own the tiles
-        const double single = rounds(heads * n);
-        if (!causal || n == 1 || !pairs_tiles) return single;
+        const double whole = rounds(heads * n);
+        if (!causal || n == 1 || !pairs_tiles) return whole;
         const double paired = rounds(heads * ((n + 1) / 2)) * (double)(n + 1) / (double)n;
-        return single < paired ? single : paired;
+        return single * whole < paired ? single * whole : paired;
     };
     const double there = group == 1 ? tile_form(pairs) : 0.5 * (tile_form(pairs) + (double)group * tile_form(pairs / group));
     const double walk = causal ? (double)(n + 1) / (double)(2 * n) : 1.0;
@@ -74,12 +76,14 @@ inline bool f32_split_for(int64_t rows, SplitCost cost, bool causal, bool pairs_
 // The forward of `pairs` (sequence, head) pairs (a ragged batch's 128-row launch pairs tiles from flash_pair_min_tiles of them on)
 // and the backward.
 inline bool f32_split_forward(int64_t rows, int D, bool causal, bool ragged, int64_t pairs, int64_t N) {
-    const bool pairs_tiles = !ragged || pairs * ((N + kFlashRows - 1) / kFlashRows) >= ragged_pair_threshold();
-    return f32_split_for(rows, f32_split_forward_cost(D), causal, pairs_tiles, pairs, 1, N);
+    const int64_t n = (N + kFlashRows - 1) / kFlashRows, paired = pairs * ((n + 1) / 2);
+    const bool pairs_tiles = !ragged || pairs * n >= ragged_pair_threshold();
+    const double single = !ragged && paired > 256 && paired <= 400 && pairs * n < 1024 ? 2.0 / 3.0 : 1.0;
+    return f32_split_for(rows, f32_split_forward_cost(D), causal, pairs_tiles, single, pairs, 1, N);
 }
 inline bool f32_split_backward(int64_t rows, int D, bool causal, bool ragged, int64_t pairs, int64_t group, int64_t N) {
     const int64_t n = (N + kFlashRows - 1) / kFlashRows;
-    return f32_split_for(rows, f32_split_backward_cost(D, ragged, n, pairs * n), causal, true, pairs, group, N);
+    return f32_split_for(rows, f32_split_backward_cost(D, ragged, n, pairs * n), causal, true, 1.0, pairs, group, N);
 }
 
 // Loads of one tile of 32 rows of a [rows][d] tensor, first row `t0`, rows at or beyond L as zeros (columns from d_real on: see

@@ -831,22 +831,26 @@ __device__ __forceinline__ void flash_fwd_mfma_body(const FlashParams& p, const 
 
 // Whether a causal dense launch of the 128-row kernels pairs a late query tile with an early one in a workgroup (every
 // workgroup then has the same walk, (n + 1) / n times the longest single one for n tiles of a sequence), by shape.  Up to 256
-// tiles every tile has a CU of its own and single ones are done first; from about 350 on CUs get two, and where ids land two
-// long walks meet on one CU.  Measured, single -> paired, us:
-//   fp32 (MFMA-bound from the first workgroup)   384 tiles (2 x 1024 x 24, d = 64) 131 -> 86    512 (16 x 256 x 16) 39 -> 35
-//   16-bit, d = 128    256 (1 x 2048 x 16) 37.8 -> 42.7    384 (2 x 2048 x 12) 49.6 -> 43.5    512 (16 x 256 x 16) 17.6 -> 19.4
-//   16-bit, d = 256    256 (1 x 2048 x 16) 91.6 -> 102     384 (2 x 1024 x 24) 79.9 -> 64.2    512 (16 x 256 x 16) 43.6 -> 40.5
-//   16-bit, d = 64 (three workgroups to a CU even out by themselves)    512 (4 x 1024 x 16) 18.8 -> 19.1    768 (3 x 1024 x 32) 27.2 -> 24.7
-// Just above a full round of pairs (512 for two workgroups per CU) single tiles fill the second round better: d = 128,
-// 2048 tokens x 72 heads (576 pairs) 106.5 -> 95.5 us, the one launch timed between 512 and 620 pairs.
+// tiles every tile has a CU of its own and single ones are done first.  Beyond that CUs get two, long walks may meet on
+// one, and pairs help while they fit a round: 256 CUs that work on one workgroup at a time (fp32, MFMA-bound; d = 256) or twice as
+// many places (d = 128; d = 64 has three, which even out by themselves).  Just beyond a round of pairs single tiles fill the
+// second one better, until it is about half full; sequences of two to four tiles, and odd n, whose middle tile has no partner, gain least.
+// Timed on 380 shapes of 240 to 1700 tiles; single -> paired, us:
+//   fp32, d = 128   384 tiles (24 per sequence) 594 -> 410    576 (9, 320 pairs) 224 -> 308    768 (8, 384 pairs) 354 -> 281
+//   fp32, d = 64    352 (11) 165 -> 113     432 (3, 288 pairs) 47 -> 69    600 (5, 360 pairs) 93 -> 100    912 (2) 62 -> 53
+//   d = 256         512 (16) 155 -> 105     532 (7, 304 pairs) 83 -> 112   800 (4, 400 pairs) 114 -> 84
+//   d = 128         372 (31) 86 -> 72       400 (5, 240 pairs) 19 -> 23    600 (25, 312 pairs) 77 -> 89    720 (12, 360 pairs) 60 -> 52
+//   d = 64          480 (30) 53 -> 49       672 (7, 384 pairs) 20 -> 23    832 (4, 416 pairs) 22 -> 19
+// Against 1024 tiles for all: 3 to 9 % faster by type and d, 1.10 times at most on any of the shapes.
 inline bool flash_pair_by_shape(int D, bool f32, int64_t seq_heads, int64_t n) {
     const int64_t tiles = seq_heads * n, pairs = seq_heads * ((n + 1) / 2);
     if (n < 2) return false;
-    if (f32) return tiles >= 352;
-    if (D == 128 && pairs > 512 && pairs <= 620) return false;
+    if (D == 128 && !f32 && pairs > 512 && pairs <= 620) return false;
     if (tiles >= 1024) return true;
-    if (D == 64) return tiles >= 640 || (tiles >= 448 && n >= 16);
-    return tiles >= 352 && n >= 4;
+    if (f32) return pairs <= 256 ? tiles >= 352 : (pairs >= 400 && n != 3) || (pairs >= 320 && n >= 8 && n % 2 == 0);
+    if (D == 256) return n >= 4 && (pairs <= 256 ? tiles >= 352 : pairs >= 400);
+    if (D == 128) return pairs <= 256 ? tiles >= 352 && n >= 9 : pairs >= 350 && n >= 4;
+    return pairs <= 264 ? tiles >= 448 && n >= 16 : (pairs >= 330 && n >= 16) || (pairs >= 416 && (n % 2 == 0 || n >= 9));
 }
 
 // The threshold the launchers of the 128-row kernels hand to flash_plan_launch (p.N and p.H are set).

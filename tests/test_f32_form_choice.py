@@ -10,6 +10,8 @@ TIMED = [
     (FORWARD, 64, True, DENSE, 2, 512, 8, 8, True),         # 38.7       14.8
     (FORWARD, 64, False, DENSE, 1, 2048, 16, 16, False),    # 139        176
     (FORWARD, 128, False, DENSE, 2, 512, 8, 8, True),       # 68.5       27.2
+    (FORWARD, 64, True, DENSE, 6, 376, 24, 24, False),      # 47         65
+    (FORWARD, 128, True, DENSE, 2, 1106, 32, 32, False),    # 224        277
     (BACKWARD, 64, True, DENSE, 1, 2048, 16, 16, True),     # 807        436
     (BACKWARD, 128, False, DENSE, 2, 2048, 16, 16, False),  # 2594       2813
     (BACKWARD, 64, False, DENSE, 1, 2048, 16, 4, True),     # 1817       738

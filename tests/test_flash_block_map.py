@@ -103,3 +103,24 @@ def test_every_pairing_line_that_is_named_holds(pair_line):
             assert pair_line(line, 128, f32, ragged, 4, 2048, 8) == 0
             assert pair_line(line, 128, f32, ragged, 9, 2048, 8) == 1
     assert pair_line(1, 128, 0, 1, 1, 129, 1) == 1
+
+
+# d, fp32?, B, N, H -> are tiles paired?       single    paired, us
+PAIRED = [(128, 1, 1, 2958, 16, 1),          # 594       410
+          (128, 1, 2, 1106, 32, 0),          # 224       308
+          (64, 1, 2, 1337, 16, 1),           # 165       113
+          (64, 1, 6, 376, 24, 0),            # 47        69
+          (256, 0, 8, 1930, 4, 1),           # 155       105
+          (256, 0, 19, 814, 4, 0),           # 83        112
+          (128, 0, 2, 3894, 6, 1),           # 86        72
+          (128, 0, 2, 552, 40, 0),           # 19        23
+          (128, 0, 3, 3101, 8, 0),           # 77        89
+          (64, 0, 2, 3779, 8, 1),            # 53        49
+          (64, 0, 3, 794, 32, 0),            # 20        23
+          (64, 0, 13, 469, 16, 1)]           # 22        19
+
+
+@pytest.mark.parametrize("d,f32,B,N,H,paired", PAIRED)
+def test_the_faster_of_single_and_paired_tiles_is_taken(pair_line, d, f32, B, N, H, paired):
+    """Causal launches of the 128-row kernels that were timed both ways."""
+    assert pair_line(0, d, f32, 0, B, N, H) == paired
