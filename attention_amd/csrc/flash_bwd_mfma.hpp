@@ -113,14 +113,15 @@ __host__ __device__ inline BwdWork bwd_work_kv(unsigned block_id, const FlashBwd
 // kernel in question).  Dense launches do.  A ragged batch whose tiles all find a place at once is done when its longest single
 // walk is, and a pair of tiles takes (n + 1) / n of that; beyond it pairs even out the second round.  The line lies a quarter
 // above a round of 256 CUs (tiles are counted from the longest sequence: some don't exist), or of 512 places for the 16-bit
-// kernels at d = 64, where two workgroups share a CU and long walks meet on one from 448 tiles on.  Whole backward, us, single ->
-// paired, by tiles:
+// kernels at d = 64, where two workgroups share a CU and long walks meet on one from 448 tiles on; and not just beyond a round
+// of pairs, where the second round of them is nearly empty.  Whole backward, us, single -> paired, by tiles:
 //   bf16, d = 128, 16 heads   256 (4 x 512) 59 -> 78      320 (4 of 500 to 1239, 8 heads) 106 -> 120     512 (4 x 1024) 147 -> 121
 //   bf16, d = 64, 16 heads    512 (16 x 256) 37 -> 43     512 (2 x 2048) 131 -> 116                    768 (12 x 512) 75 -> 70
 //   fp32, d = 64, 16 heads    256 (4 x 512) 208 -> 254    512 (4 x 1024) 706 -> 503
 inline bool bwd_pair_by_shape(bool narrow, bool ragged, int64_t pairs, int64_t n) {
     if (!ragged) return true;
-    const int64_t tiles = pairs * n;
+    const int64_t tiles = pairs * n, pairs_of_tiles = pairs * ((n + 1) / 2);
+    if (pairs_of_tiles > 256 && pairs_of_tiles <= 350) return false;
     return narrow ? tiles > 640 || (tiles > 448 && n >= 16) : tiles > 320;
 }
 

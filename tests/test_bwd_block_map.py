@@ -47,6 +47,7 @@ def test_every_unit_once_and_all_xcds_at_work(B, N, H, H_kv, causal, ragged, kv,
 
 @pytest.mark.parametrize("B,N,H,narrow,ragged,paired", [
     (1, 2048, 16, False, True, 0),   # 256 tiles: a CU for each
+    (4, 1170, 15, False, True, 0),   # 600 tiles, 300 pairs: the second round of pairs would be nearly empty
     (5, 1024, 8, False, True, 0), (5, 1024, 8, False, False, 1), (4, 1024, 16, False, True, 1),
     (16, 256, 16, True, True, 0), (2, 2048, 16, True, True, 1), (12, 512, 16, True, True, 1), (12, 512, 16, True, False, 1)])
 def test_small_ragged_launches_take_their_tiles_singly(B, N, H, narrow, ragged, paired):
