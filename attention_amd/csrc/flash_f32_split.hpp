@@ -74,14 +74,18 @@ inline bool f32_split_for(int64_t rows, SplitCost cost, bool causal, bool pairs_
     return cost.shared * (walk + cost.fixed / (double)n) * (double)tiles / 256.0 < there;
 }
 // The forward of `pairs` (sequence, head) pairs (a ragged batch's 128-row launch pairs tiles from flash_pair_min_tiles of them on)
-// and the backward.
+// and the backward.  Below two key tiles there is no walk to share, only the exchange to pay for: forward, 8 heads, 16 tokens 7.5 (128
+// rows) / 8.4 us at d = 64, 8.1 / 13.8 at d = 128, 48 tokens 12.4 / 14.2, 64 tokens 12.7 / 10.1; backward at d = 128, 16 tokens 39 / 51,
+// 32 tokens 41 / 37 (at d = 64 the two are equal there).
 inline bool f32_split_forward(int64_t rows, int D, bool causal, bool ragged, int64_t pairs, int64_t N) {
+    if (rows != kSplitRows && N < 2 * kF32Keys) return false;
     const int64_t n = (N + kFlashRows - 1) / kFlashRows, paired = pairs * ((n + 1) / 2);
     const bool pairs_tiles = !ragged || pairs * n >= ragged_pair_threshold();
     const double single = !ragged && paired > 256 && paired <= 400 && pairs * n < 1024 ? 2.0 / 3.0 : 1.0;
     return f32_split_for(rows, f32_split_forward_cost(D), causal, pairs_tiles, single, pairs, 1, N);
 }
 inline bool f32_split_backward(int64_t rows, int D, bool causal, bool ragged, int64_t pairs, int64_t group, int64_t N) {
+    if (rows != kSplitRows && D > 64 && N < kF32Keys) return false;
     const int64_t n = (N + kFlashRows - 1) / kFlashRows;
     return f32_split_for(rows, f32_split_backward_cost(D, ragged, n, pairs * n), causal, true, 1.0, pairs, group, N);
 }

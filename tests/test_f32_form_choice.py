@@ -12,6 +12,11 @@ TIMED = [
     (FORWARD, 128, False, DENSE, 2, 512, 8, 8, True),       # 68.5       27.2
     (FORWARD, 64, True, DENSE, 6, 376, 24, 24, False),      # 47         65
     (FORWARD, 128, True, DENSE, 2, 1106, 32, 32, False),    # 224        277
+    (FORWARD, 128, True, DENSE, 1, 16, 8, 8, False),        # 8.1        13.8
+    (FORWARD, 64, True, RAGGED, 4, 48, 8, 8, False),        # 8.0        8.6
+    (FORWARD, 64, False, DENSE, 1, 64, 8, 8, True),         # 8.3        7.5
+    (BACKWARD, 128, False, DENSE, 4, 16, 8, 8, False),      # 40         51
+    (BACKWARD, 128, False, DENSE, 4, 32, 8, 8, True),       # 41         37
     (BACKWARD, 64, True, DENSE, 1, 2048, 16, 16, True),     # 807        436
     (BACKWARD, 128, False, DENSE, 2, 2048, 16, 16, False),  # 2594       2813
     (BACKWARD, 64, False, DENSE, 1, 2048, 16, 4, True),     # 1817       738
