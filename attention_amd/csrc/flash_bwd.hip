@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kDeltaThreads) void flash_bwd_delta_kernel(const T*
 
 // dK and dV: in one walk over the query tiles (four matrix products per tile) up to d = 128, in two walks (dV, then dK:
 // five products) at d = 256, where one walk would need more registers than a wavefront has.  At d = 128 the one walk
-// runs at one wavefront per SIMD (324 registers) and takes 5 % more cycles than the two walks at two per SIMD; on
+// runs at one wavefront per SIMD (400 registers) and takes 5 % more cycles than the two walks at two per SIMD; on
 // N(0,1) inputs, where the board sits at its power limit and the clock follows the energy spent, it is the faster of
 // the two by 4-15 % at every shape timed (fewer products), and it is one launch less.  The tuning value bwd_split
 // (0 = this choice, 1 = one walk, 2 = two) overrides.

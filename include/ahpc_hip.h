@@ -71,7 +71,7 @@ typedef struct ahpc_device_info {
  * "bwd_split", "bwd_pair", "mask_pack", "pool_in_place"): process-wide, each starts from its environment variable
  * (AHPC_FLASH_PAIR_MIN, AHPC_FLASH_ROWS, AHPC_FLASH_WALKS, AHPC_DECODE_WAVES, AHPC_DECODE_CHUNK, AHPC_DECODE_MFMA_MIN_GROUP, AHPC_BWD_SPLIT,
  * AHPC_BWD_PAIR, AHPC_MASK_PACK, AHPC_POOL_IN_PLACE), which is read once.  No value
- * changes results; unknown names and negative values are refused.  The reference has no counterpart: its tile sizes
+ * changes results by more than the order in which sums are taken; unknown names and negative values are refused.  The reference has no counterpart: its tile sizes
  * sit in PerformanceConfig (src/api/attention_interface.hpp:29-53), which the host classes still honour. */
 int ahpc_hip_set_tuning(const char* name, int64_t value);
 int ahpc_hip_get_tuning(const char* name, int64_t* value);
