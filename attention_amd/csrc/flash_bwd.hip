@@ -523,7 +523,7 @@ static int launch_f32_mfma_dv(const FlashBwdParams& p, int64_t B, bool causal, f
     if (split) {
         auto launch = [&](auto causal_c) {
             constexpr bool C = decltype(causal_c)::value;
-            hipLaunchKernelGGL((flash_bwd_stats_f32_split_kernel<D, C, VARLEN>), grid_stats, block, 0, stream, f, st);
+            hipLaunchKernelGGL((flash_bwd_stats_f32_split_kernel<D, C, VARLEN>), grid_stats, dim3(kWave * SplitFwd<D>::W), 0, stream, f, st);
             hipLaunchKernelGGL((flash_bwd_dq_f32_split_kernel<D, C, VARLEN>), grid_q, block, 0, stream, m);
             hipLaunchKernelGGL((flash_bwd_dkv_f32_split_kernel<D, C, VARLEN>), grid_kv, block, 0, stream, m);
         };

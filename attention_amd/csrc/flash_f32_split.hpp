@@ -6,6 +6,8 @@
 // its own, and the four partial results meet in LDS once at the end, in a fixed order (no atomics; results do not depend on
 // which wavefront is faster).  Four times the workgroups, a quarter of the walk.
 //
+// The forward and the statistics multiply with bf16 pieces (f32_x3.hpp) and, at d = 64, share a walk among eight wavefronts, two to a
+// SIMD; the backward multiplies with the fp32 instructions, as does a forward whose inputs have no such pieces.
 // Same products, layouts and contraction order within a tile as those kernels (see there).  The operands come straight from
 // memory: a v_mfma_f32_32x32x2_f32 takes 64 cycles, a tile's two products 4096 (d = 64), and its operands are 16 KB, so one
 // load instruction in flight per few matrix instructions keeps up and there is nothing to stage, swizzle or synchronise:
@@ -13,10 +15,10 @@
 //   columns operand (A of the products over rows)  a lane reads one float per instruction, 128 bytes of a row per half
 // Each operand is requested one product (2048 cycles at d = 64) ahead of the product that uses it, so that two or three operand
 // sets are in registers at a time; the workgroup's own 32 rows, the B operands of the products over d, are the same for all
-// its wavefronts and wait in LDS.  With that the forward at d = 64 leaves two
-// workgroups to a CU; everything else takes one with up to 512 registers and no scratch.
-// Bound: the fp32 matrix rate where the launch fills the chip (2 x 512 x 8, d = 64: 1024 wavefronts of four tiles each, 14.6 us of
-// which 7 are matrix instructions and the rest the launch, the first loads, the exchange), the length of one walk below that.
+// its wavefronts and wait in LDS.  The backward takes a CU per workgroup with up to 512 registers and no scratch.
+// Bound: 2 x 512 x 8, d = 64, forward: 14.7 us on the fp32 instructions with four wavefronts of four tiles, of which 7 were matrix instructions;
+// 13.6 on pieces, 13.1 on pieces with eight wavefronts: the launch, the first loads and the exchange, then splitting and addressing (vector
+// instructions).  2 x 1024 x 8 causal 46.9 -> 26.5, 1 x 2048 x 16 causal 105 -> 83.
 #pragma once
 
 #include "flash_bwd_f32_mfma.hpp"
@@ -37,13 +39,13 @@ constexpr int kSplitWaves = 4;   // wavefronts that share its walk
 // up to 1024 tiles (768 for sequences of at most three tiles, whose walks aren't long: 11 of up to 264 tokens, 24 heads over 12, d = 128,
 // 792 tiles, 482 -> 628).
 // Measured at d = 64 (forward / backward, us, 128-row form -> this one), where the model draws its line:
-//     tiles  64 (2 x 512 x 8)     causal 38.7 -> 14.7 / 247 -> 60    not causal 38.3 -> 14.7 / 196 -> 60
-//     tiles 128 (2 x 1024 x 8)    causal 74 -> 47 / 432 -> 143       not causal 72 -> 49 / 372 -> 206
-//     tiles 256 (1 x 2048 x 16)   causal 144 -> 105 / 804 -> 434     not causal 139 -> 175 / 732 -> 751
-//     tiles 512 (2 x 2048 x 16)   causal 157 -> 206 / 923 -> 861     not causal 257 -> 341 / 1364 -> 1492
+//     tiles  64 (2 x 512 x 8)     causal 33 -> 13 / 247 -> 60        not causal 34 -> 14 / 196 -> 60
+//     tiles 128 (2 x 1024 x 8)    causal 62 -> 27 / 432 -> 143       not causal 63 -> 42 / 372 -> 206
+//     tiles 256 (1 x 2048 x 16)   causal 120 -> 83 / 804 -> 434      not causal 125 -> 148 / 732 -> 751
+//     tiles 512 (2 x 2048 x 16)   causal 132 -> 164 / 923 -> 861     not causal 194 -> 290 / 1364 -> 1492
 // d = 128, forward:
-//     tiles 256                   causal 262 -> 190 (1 x 2048 x 16), 72 -> 86 (4 x 512 x 16)     not causal 73 -> 107 (4 x 512 x 16)
-//     ragged, 576 (12 of 100 to 400, 16 heads)     causal 86 -> 138     not causal 103 -> 191
+//     tiles 256                   causal 216 -> 183 (1 x 2048 x 16), 65 -> 79 (4 x 512 x 16)     not causal 69 -> 101 (4 x 512 x 16)
+// The costs were fitted when both forms used the fp32 instructions; both forms' walks have become shorter by about as much.
 // Over 260 ragged and 236 dense shapes with 24 to 1500 tiles the form taken is 0.2 to 2 % slower than the better of the two
 // (geometric means by direction and d); on single ragged shapes, with half of the tiles missing or none, by up to 1.7 times.
 // `rows`: 32 or 128 forces a form (the tuning values flash_rows and bwd_split), anything else = by shape.  `group`: query heads
@@ -172,10 +174,10 @@ template <int D> struct F32SplitTile {
     // The workgroup's own rows as B operands in LDS, multiplied by c (zeros from d_real on): piece m of lane `lane` at
     // own + (m * 64 + lane) * 4.  The wavefronts share the pieces out; the caller's barrier follows.
     static constexpr int kOwnFloats = MS * kWave * 4;
-    __device__ static void put_own(float* own, const float* row_ptr, int wave, int lane, float c, int d_real) {
+    template <int W = kSplitWaves> __device__ static void put_own(float* own, const float* row_ptr, int wave, int lane, float c, int d_real) {
 #pragma unroll
-        for (int i = 0; i < MS / kSplitWaves; ++i) {
-            const int m = i * kSplitWaves + wave;
+        for (int i = 0; i < MS / W; ++i) {
+            const int m = i * W + wave;
             const int at = 8 * m + 4 * (lane >> 5);
             const f32x4 raw = at < d_real ? *reinterpret_cast<const f32x4*>(row_ptr + at) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             *reinterpret_cast<f32x4*>(own + (m * kWave + lane) * 4) = f32x4{raw[0] * c, raw[1] * c, raw[2] * c, raw[3] * c};
@@ -183,10 +185,126 @@ template <int D> struct F32SplitTile {
     }
 };
 
-// Partial accumulators of the workgroup's wavefronts in LDS: [wavefront][32-row block][group of 4 registers][lane] 16 bytes each.
-// Wavefront w collects register group w of every block: elements 32 mb + 8 w + 4 half .. + 3 of row `col`.
-template <int MB> struct SplitExchange {
-    static constexpr int kFloats = kSplitWaves * MB * 4 * kWave * 4;
+// The same on the bf16 matrix instructions (f32_x3.hpp): every wavefront splits the operands of its own tiles in registers.
+template <int D> struct X3SplitTile {
+    static constexpr int KS = D / 16, MB = D / 32;
+
+    // rows operand: rows[ks] = 8 floats from d = 16 ks + 8 half of row t0 + col (rows behind the last one: zeros).  Straight from
+    // memory: as whole cache lines and through LDS the forward took 13.2 us where this takes 13.0, 609 where it takes 573
+    // (4 x 2048 x 16, d = 64).
+    __device__ static void load_rows(float (&rows)[KS][8], const float* base, int64_t stride, int t0, int L, int col, int half, int d_real) {
+        const int row = t0 + col;
+        const float* const src = base + (int64_t)(row < L ? row : L - 1) * stride;
+        const int last = d_real - 4;  // the last quad the row has
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                const int at = 16 * ks + 8 * half + 4 * v;
+                const f32x4 x = *reinterpret_cast<const f32x4*>(src + (at < last ? at : last));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rows[ks][4 * v + e] = x[e];
+            }
+        if (t0 + kF32Keys > L) {  // (uniform)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) rows[ks][e] = row < L ? rows[ks][e] : 0.0f;
+        }
+    }
+
+    // c + (rows . own) over d.  own: put_own's.
+    __device__ static f32x16 product_over_d(const float (&rows)[KS][8], const unsigned char* own, int lane, const f32x16& c, Magnitudes& seen) {
+        f32x16 hi = c, lo;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) lo[r] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const unsigned char* const at = own + (3 * ks * kWave + lane) * 16;
+            seen.see(rows[ks]);
+            mfma_x3(split_f32(rows[ks]), F32x3{lds_read_b128(at), lds_read_b128(at + kWave * 16), lds_read_b128(at + 2 * kWave * 16)}, hi, lo);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) hi[r] += lo[r];
+        return hi;
+    }
+
+    // acc += A^T B over the 32 rows of the tile; cols: F32SplitTile::load_cols, b: one 8-register group per 16 rows, split
+    __device__ static void product_over_rows(f32x16 (&acc)[MB], const float (&cols)[16][MB], const F32x3 (&b)[2], Magnitudes& seen) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            f32x16 t;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) t[r] = 0.0f;
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = cols[8 * g + e][mb];
+                seen.see(x);
+                mfma_x3(split_f32(x), b[g], t, t);
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mb][r] += t[r];
+        }
+    }
+    __device__ static void split_groups(F32x3 (&out)[2], const f32x16& w) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = w[8 * g + e];
+            out[g] = split_f32(x);
+        }
+    }
+
+    // The workgroup's own rows as B operands in LDS, multiplied by c and split: piece i of step ks of lane `lane` at own +
+    // ((3 ks + i) 64 + lane) 16 bytes.  The wavefronts share the steps out; the caller's barrier follows.
+    static constexpr int kOwnBytes = 3 * KS * kWave * 16;
+    template <int W = kSplitWaves>
+    __device__ static void put_own(unsigned char* own, const float* row_ptr, int wave, int lane, float c, int d_real, Magnitudes& seen) {
+#pragma unroll
+        for (int i = 0; i < (KS + W - 1) / W; ++i) {
+            const int ks = i * W + wave;
+            if (W > KS && ks >= KS) break;  // (uniform)
+            float x[8];
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                const int at = 16 * ks + 8 * (lane >> 5) + 4 * v;
+                const bool there = at < d_real;
+                const f32x4 raw = *reinterpret_cast<const f32x4*>(row_ptr + (there ? at : 0));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[4 * v + e] = there ? raw[e] * c : 0.0f;
+            }
+            seen.see(x);
+            const F32x3 piece = split_f32(x);
+            unsigned char* const dst = own + (3 * ks * kWave + lane) * 16;
+            *reinterpret_cast<u32x4*>(dst) = piece.h;
+            *reinterpret_cast<u32x4*>(dst + kWave * 16) = piece.m;
+            *reinterpret_cast<u32x4*>(dst + 2 * kWave * 16) = piece.l;
+        }
+    }
+};
+
+// Whether any wavefront of the workgroup met a value that cannot be split.  (Uniform; everyone is done with `lds`.)
+__device__ inline bool split_again(const Magnitudes& seen, unsigned char* lds) {
+    int* const flag = reinterpret_cast<int*>(lds);
+    __syncthreads();
+    if (threadIdx.x == 0) *flag = 0;
+    __syncthreads();
+    if (!seen.in_range()) *flag = 1;
+    __syncthreads();
+    const bool again = *flag != 0;
+    __syncthreads();
+    return again;
+}
+
+// Partial accumulators of the workgroup's W wavefronts in LDS: [wavefront][32-row block][group of 4 registers][lane] 16 bytes each.
+// Wavefront w collects the pieces w, w + W, ... of the 4 MB (block, group) pairs: piece u is group u % 4 of block u / 4, elements
+// 32 (u / 4) + 8 (u % 4) + 4 half .. + 3 of row `col`.
+template <int MB, int W = kSplitWaves> struct SplitExchange {
+    static constexpr int kFloats = W * MB * 4 * kWave * 4;
+    static constexpr int kPieces = MB * 4 / W;  // per wavefront
     __device__ static void put(float* lds, const f32x16 (&acc)[MB], int wave, int lane) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -195,20 +313,31 @@ template <int MB> struct SplitExchange {
                 *reinterpret_cast<f32x4*>(lds + (((wave * MB + mb) * 4 + g4) * kWave + lane) * 4) =
                     f32x4{acc[mb][4 * g4], acc[mb][4 * g4 + 1], acc[mb][4 * g4 + 2], acc[mb][4 * g4 + 3]};
     }
-    __device__ static f32x4 get(const float* lds, int from, int mb, int wave, int lane) {
-        return *reinterpret_cast<const f32x4*>(lds + (((from * MB + mb) * 4 + wave) * kWave + lane) * 4);
+    __device__ static f32x4 get(const float* lds, int from, int piece, int lane) {
+        return *reinterpret_cast<const f32x4*>(lds + ((from * MB * 4 + piece) * kWave + lane) * 4);
     }
+    __device__ static int element(int piece, int half) { return 32 * (piece >> 2) + 8 * (piece & 3) + 4 * half; }
 };
 
 // Work map: flash_work_of_block over blocks of 32 query rows (flash_plan_launch with 32 rows per workgroup, never paired).
-template <int D, bool CAUSAL, bool VARLEN, bool STATS>
-__device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, const FlashStatsOut& st) {
+// X3: on the bf16 instructions; returns whether the workgroup met a value that cannot be split, in which case what it wrote is
+// void.  (Uniform.)
+template <int D> struct SplitFwd {
+    static constexpr int W = D == 64 ? 8 : 4;
+    static constexpr int kLdsBytes = 4 * SplitExchange<D / 32, W>::kFloats;
+    struct Lds {
+        float m[W][kSplitRows], l[W][kSplitRows], part[W][kSplitRows];
+    };
+};
+template <int D, bool CAUSAL, bool VARLEN, bool STATS, bool X3>
+__device__ __forceinline__ bool flash_fwd_f32_split_body(const FlashParams& p, const FlashStatsOut& st, float* lds, typename SplitFwd<D>::Lds& ex) {
     typedef F32SplitTile<D> TL;
+    typedef X3SplitTile<D> TX;
     constexpr int MS = TL::MS, MB = TL::MB;
-    typedef SplitExchange<MB> X;
-    static_assert(TL::kOwnFloats <= X::kFloats, "the own rows and the exchange share their LDS");
-    __shared__ __attribute__((aligned(1024))) float lds[X::kFloats];
-    __shared__ float lds_m[kSplitWaves][kSplitRows], lds_l[kSplitWaves][kSplitRows], lds_part[kSplitWaves][kSplitRows];
+    constexpr int W = SplitFwd<D>::W;
+    typedef SplitExchange<MB, W> X;
+    static_assert(TL::kOwnFloats <= X::kFloats && TX::kOwnBytes <= 4 * X::kFloats, "the own rows and the exchange share their LDS");
+    Magnitudes seen_values;
 
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
@@ -216,8 +345,8 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
     const int half = lane >> 5;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const FlashWork work = flash_work_of_block(blockIdx.x, p);
-    if (!work.valid) return;
-    if (work.bh < 0 || work.bh >= p.n_bh || work.slot < 0 || work.slot >= flash_per_head(p)) return;
+    if (!work.valid) return false;
+    if (work.bh < 0 || work.bh >= p.n_bh || work.slot < 0 || work.slot >= flash_per_head(p)) return false;
     const int b = work.bh / p.H;
     const int h = work.bh - b * p.H;
     const int hk = h / p.kv_group;
@@ -234,7 +363,7 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
         kv_base = (int64_t)b * p.kv_stride_b + (int64_t)hk * p.kv_stride_h;
     }
     const int n_q = VARLEN ? (L + kSplitRows - 1) / kSplitRows : p.n_qtiles;
-    if (work.slot >= n_q) return;
+    if (work.slot >= n_q) return false;
     const int q0 = (n_q - 1 - work.slot) * kSplitRows;  // long walks first
     const float* const gk = static_cast<const float*>(p.k) + kv_base;
     const float* const gv = static_cast<const float*>(p.v) + kv_base;
@@ -246,10 +375,17 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
     if (CAUSAL) k_end = q0 + kSplitRows < L ? q0 + kSplitRows : L;
     const int n_tiles = (k_end + kF32Keys - 1) / kF32Keys;
 
-    f32x4 kq[MS];
+    typename std::conditional<X3, float[TX::KS][8], f32x4[MS]>::type kq;
     float vc[16][MB];
-    if (wave_u < n_tiles) TL::load_rows(kq, gk, skv, wave_u * kF32Keys, L, col, half, d_real);
-    TL::put_own(lds, static_cast<const float*>(p.q) + base + (int64_t)(qrow < L ? qrow : L - 1) * sn, wave, lane, p.scale_log2, d_real);
+    const float* const own = static_cast<const float*>(p.q) + base + (int64_t)(qrow < L ? qrow : L - 1) * sn;
+    unsigned char* const lds_own = reinterpret_cast<unsigned char*>(lds);
+    auto load_keys = [&](int k0) __attribute__((always_inline)) {
+        if constexpr (X3) TX::load_rows(kq, gk, skv, k0, L, col, half, d_real);
+        else TL::load_rows(kq, gk, skv, k0, L, col, half, d_real);
+    };
+    if (wave_u < n_tiles) load_keys(wave_u * kF32Keys);
+    if constexpr (X3) TX::template put_own<W>(lds_own, own, wave, lane, p.scale_log2, d_real, seen_values);
+    else TL::template put_own<W>(lds, own, wave, lane, p.scale_log2, d_real);
     __syncthreads();
 
     f32x16 oacc[MB], neg_m;
@@ -261,14 +397,16 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
     constexpr float kRaise = 8.0f;  // the reference maximum is raised only when exceeded by 2^8 (flash_fwd_mfma.hpp)
     float raise = -INFINITY;        // kRaise once this lane's query has met a key of finite score in this wavefront's tiles
 
-    for (int t = wave_u; t < n_tiles; t += kSplitWaves) {
+    for (int t = wave_u; t < n_tiles; t += W) {
         const int k0 = t * kF32Keys;
-        const bool more = t + kSplitWaves < n_tiles;
+        const bool more = t + W < n_tiles;
         TL::load_cols(vc, gv, skv, k0, L, col, half, d_real);
         __builtin_amdgcn_sched_barrier(0);
-        f32x16 s = TL::product_over_d(kq, lds, lane, neg_m);
+        f32x16 s;
+        if constexpr (X3) s = TX::product_over_d(kq, lds_own, lane, neg_m, seen_values);
+        else s = TL::product_over_d(kq, lds, lane, neg_m);
         __builtin_amdgcn_sched_barrier(0);
-        if (more) TL::load_rows(kq, gk, skv, k0 + kSplitWaves * kF32Keys, L, col, half, d_real);
+        if (more) load_keys(k0 + W * kF32Keys);
         __builtin_amdgcn_sched_barrier(0);
         // key of register r: k0 + 8 (r / 4) + 4 half + r % 4; visible iff key <= min(qrow, L - 1)
         if ((k0 + kF32Keys > L) || (CAUSAL && (k0 + kF32Keys - 1 > q0))) {
@@ -309,7 +447,13 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
             sum += s[r];
         }
         l_run += sum;
-        TL::product_over_rows(oacc, vc, s);
+        if constexpr (X3) {
+            F32x3 w[2];
+            TX::split_groups(w, s);
+            TX::product_over_rows(oacc, vc, w, seen_values);
+        } else {
+            TL::product_over_rows(oacc, vc, s);
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();  // the own rows' LDS is the exchange's
@@ -318,53 +462,55 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
     {
         const float l = halves_sum(l_run);
         if (half == 0) {
-            lds_m[wave][col] = raise > 0.0f ? -neg_m[0] : -INFINITY;  // (a wavefront without a tile)
-            lds_l[wave][col] = l;
+            ex.m[wave][col] = raise > 0.0f ? -neg_m[0] : -INFINITY;  // (a wavefront without a tile)
+            ex.l[wave][col] = l;
         }
         X::put(lds, oacc, wave, lane);
     }
     __syncthreads();
-    float m = -INFINITY, l = 0.0f, f[kSplitWaves];
+    float m = -INFINITY, l = 0.0f, f[W];
 #pragma unroll
-    for (int w = 0; w < kSplitWaves; ++w) m = fmaxf(m, lds_m[w][col]);
+    for (int w = 0; w < W; ++w) m = fmaxf(m, ex.m[w][col]);
 #pragma unroll
-    for (int w = 0; w < kSplitWaves; ++w) {
-        f[w] = m > -INFINITY ? fast_exp2(lds_m[w][col] - m) : 0.0f;
-        l = __builtin_fmaf(lds_l[w][col], f[w], l);
+    for (int w = 0; w < W; ++w) {
+        f[w] = m > -INFINITY ? fast_exp2(ex.m[w][col] - m) : 0.0f;
+        l = __builtin_fmaf(ex.l[w][col], f[w], l);
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    f32x4 out[MB];
+    f32x4 out[X::kPieces];
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
+    for (int i = 0; i < X::kPieces; ++i) {
         f32x4 a = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int w = 0; w < kSplitWaves; ++w) {
-            const f32x4 x = X::get(lds, w, mb, wave, lane);
+        for (int w = 0; w < W; ++w) {
+            const f32x4 x = X::get(lds, w, wave + W * i, lane);
 #pragma unroll
             for (int e = 0; e < 4; ++e) a[e] = __builtin_fmaf(x[e], f[w], a[e]);
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) out[mb][e] = a[e] * inv;
+        for (int e = 0; e < 4; ++e) out[i][e] = a[e] * inv;
     }
-    const int at = 8 * wave + 4 * half;  // this lane's elements of a 32-element block
     if constexpr (STATS) {
         float part = 0.0f;
         if (qrow < L) {
-            const float* src = static_cast<const float*>(st.d_out) + base + (int64_t)qrow * sn + at;
+            const float* src = static_cast<const float*>(st.d_out) + base + (int64_t)qrow * sn;
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb) {
-                if (32 * mb + at >= d_real) continue;  // columns the tensors do not have
-                const f32x4 w = *reinterpret_cast<const f32x4*>(src + 32 * mb);
-                part += out[mb][0] * w[0] + out[mb][1] * w[1] + out[mb][2] * w[2] + out[mb][3] * w[3];
+            for (int i = 0; i < X::kPieces; ++i) {
+                const int at = X::element(wave + W * i, half);
+                if (at >= d_real) continue;  // columns the tensors do not have
+                const f32x4 w = *reinterpret_cast<const f32x4*>(src + at);
+                part += out[i][0] * w[0] + out[i][1] * w[1] + out[i][2] * w[2] + out[i][3] * w[3];
             }
         }
         part = halves_sum(part);
-        if (half == 0) lds_part[wave][col] = part;
+        if (half == 0) ex.part[wave][col] = part;
         __syncthreads();
         if (wave == 0) {
             const int64_t row0 = (int64_t)work.bh * st.rows_padded;
             if (half == 0) {
-                const float delta = (lds_part[0][col] + lds_part[1][col]) + (lds_part[2][col] + lds_part[3][col]);
+                float delta = 0.0f;
+#pragma unroll
+                for (int w = 0; w < W; ++w) delta += ex.part[w][col];
                 const bool live = qrow < L && l > 0.0f;
                 st.neg_lse2[row0 + qrow] = live ? -m - __builtin_log2f(l) : -INFINITY;
                 st.neg_delta[row0 + qrow] = live ? -delta : 0.0f;
@@ -379,36 +525,46 @@ __device__ __forceinline__ void flash_fwd_f32_split_body(const FlashParams& p, c
             }
         }
     } else if (qrow < L) {
-        float* dst = static_cast<float*>(p.o) + base + (int64_t)qrow * sn + at;
+        float* dst = static_cast<float*>(p.o) + base + (int64_t)qrow * sn;
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-            if (32 * mb + at < d_real) *reinterpret_cast<f32x4*>(dst + 32 * mb) = out[mb];
+        for (int i = 0; i < X::kPieces; ++i) {
+            const int at = X::element(wave + W * i, half);
+            if (at < d_real) *reinterpret_cast<f32x4*>(dst + at) = out[i];
+        }
     }
+    return X3 ? split_again(seen_values, lds_own) : false;
 }
 
 template <int D, bool CAUSAL, bool VARLEN>
-__global__ __launch_bounds__(kWave * kSplitWaves, D > 64 ? 1 : 2) void flash_fwd_f32_split_kernel(const FlashParams p) {
-    flash_fwd_f32_split_body<D, CAUSAL, VARLEN, false>(p, FlashStatsOut{});
+__global__ __launch_bounds__(kWave * SplitFwd<D>::W, SplitFwd<D>::W == 8 ? 2 : 1) void flash_fwd_f32_split_kernel(const FlashParams p) {
+    __shared__ __attribute__((aligned(1024))) float lds[SplitFwd<D>::kLdsBytes / 4];
+    __shared__ typename SplitFwd<D>::Lds ex;
+    if (flash_fwd_f32_split_body<D, CAUSAL, VARLEN, false, true>(p, FlashStatsOut{}, lds, ex))
+        flash_fwd_f32_split_body<D, CAUSAL, VARLEN, false, false>(p, FlashStatsOut{}, lds, ex);
 }
 template <int D, bool CAUSAL, bool VARLEN>
-__global__ __launch_bounds__(kWave * kSplitWaves, D > 64 ? 1 : 2) void flash_bwd_stats_f32_split_kernel(const FlashParams p, const FlashStatsOut st) {
-    flash_fwd_f32_split_body<D, CAUSAL, VARLEN, true>(p, st);
+__global__ __launch_bounds__(kWave * SplitFwd<D>::W, SplitFwd<D>::W == 8 ? 2 : 1) void flash_bwd_stats_f32_split_kernel(const FlashParams p, const FlashStatsOut st) {
+    __shared__ __attribute__((aligned(1024))) float lds[SplitFwd<D>::kLdsBytes / 4];
+    __shared__ typename SplitFwd<D>::Lds ex;
+    if (flash_fwd_f32_split_body<D, CAUSAL, VARLEN, true, true>(p, st, lds, ex))
+        flash_fwd_f32_split_body<D, CAUSAL, VARLEN, true, false>(p, st, lds, ex);
 }
 
 // Stores the sum of the wavefronts' partial accumulators, times f, at dst_row (row `col` of the block).
 template <int MB>
 __device__ inline void split_store_sum(float* dst_row, const float* lds, int wave, int lane, float f, int d_real) {
-    const int at = 8 * wave + 4 * (lane >> 5);
+    typedef SplitExchange<MB> X;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-        f32x4 a = SplitExchange<MB>::get(lds, 0, mb, wave, lane);
+    for (int i = 0; i < X::kPieces; ++i) {
+        const int piece = wave + kSplitWaves * i, at = X::element(piece, lane >> 5);
+        f32x4 a = X::get(lds, 0, piece, lane);
 #pragma unroll
         for (int w = 1; w < kSplitWaves; ++w) {
-            const f32x4 x = SplitExchange<MB>::get(lds, w, mb, wave, lane);
+            const f32x4 x = X::get(lds, w, piece, lane);
 #pragma unroll
             for (int e = 0; e < 4; ++e) a[e] += x[e];
         }
-        if (32 * mb + at < d_real) *reinterpret_cast<f32x4*>(dst_row + 32 * mb + at) = f32x4{a[0] * f, a[1] * f, a[2] * f, a[3] * f};
+        if (at < d_real) *reinterpret_cast<f32x4*>(dst_row + at) = f32x4{a[0] * f, a[1] * f, a[2] * f, a[3] * f};
     }
 }
 

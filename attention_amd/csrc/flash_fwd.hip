@@ -446,7 +446,7 @@ static bool f32_mfma_eligible(int dtype, int64_t d, const void* q, const void* k
 template <int D, bool VARLEN>
 static int launch_f32_split(FlashParams p, int64_t B, bool causal, hipStream_t stream) {
     if (int rc = flash_plan_launch(p, B, causal, kSplitRows, kNeverPair, VARLEN)) return rc;
-    dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(kWave * kSplitWaves);
+    dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(kWave * SplitFwd<D>::W);
     if (causal) hipLaunchKernelGGL((flash_fwd_f32_split_kernel<D, true, VARLEN>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((flash_fwd_f32_split_kernel<D, false, VARLEN>), grid, block, 0, stream, p);
     return static_cast<int>(hipGetLastError());

@@ -1,5 +1,6 @@
-// FlashAttention forward for fp32 tensors on the gfx950 matrix cores (v_mfma_f32_32x32x2_f32: fp32 operands, fp32
-// products and sums, so the result keeps the fp32 kernel's accuracy).  fp32 is the reference's default data type
+// FlashAttention forward for fp32 tensors on the gfx950 matrix cores: up to d = 128 as products of bf16 pieces (f32_x3.hpp and the
+// second half of this file), beyond that and for inputs that have no such pieces with v_mfma_f32_32x32x2_f32, which is what
+// comes first (fp32 operands, products and sums).  fp32 is the reference's default data type
 // (DataType::FLOAT32, src/api/attention_interface.hpp:13-19; every case of tests/test_flash_attention.cpp uses it);
 // the block it replaces is FlashAttention::compute_attention_block, src/algorithms/flash_attention.cpp:277-350.
 //
@@ -26,6 +27,7 @@
 //   V: f = 8 * ((r / 4) % 2): the two halves of a 4-byte read (rows 4 apart, same 32 floats) hit different banks.
 #pragma once
 
+#include "f32_x3.hpp"
 #include "flash_fwd_mfma.hpp"
 
 namespace ahpc {
@@ -43,7 +45,8 @@ __device__ inline f32x16 mfma_32x32x2_f32(float a, float b, f32x16 c) {
 // STATS: the first step of the backward.  The output stays in registers; per query row the kernel writes what
 // FlashStatsOut describes (flash_fwd_mfma.hpp): -lse2 and -(dO . O), padding rows -inf and 0.
 template <int D, bool CAUSAL, bool VARLEN, bool MASKED, bool STATS>
-__device__ __forceinline__ void flash_fwd_f32_mfma_body(const FlashParams& p, const FlashStatsOut& st) {
+__device__ __forceinline__ void flash_fwd_f32_mfma_body(const FlashParams& p, const FlashStatsOut& st, unsigned char* lds_k0,
+                                                        unsigned char* lds_v0, unsigned char* lds_k1, unsigned char* lds_v1) {
     static_assert(D == 64 || D == 128 || D == 256, "head dimensions of the fp32 matrix-core kernel");
     static_assert(!(MASKED && (VARLEN || STATS)), "the mask belongs to dense forward launches");
     constexpr int RB = 4 * D;                 // row bytes
@@ -52,12 +55,6 @@ __device__ __forceinline__ void flash_fwd_f32_mfma_body(const FlashParams& p, co
     constexpr int IPW = kF32Keys / RPI / 4;   // load instructions per wavefront and tile (K or V)
     constexpr int MS = D / 8;                 // 16-byte K reads (= register quads of Q) per lane
     constexpr int MB = D / 32;                // 32-row blocks of O^T
-    constexpr int kTileBytes = kF32Keys * RB;
-
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_k0[kTileBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_v0[kTileBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_k1[kTileBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_v1[kTileBytes];
 
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
@@ -340,14 +337,404 @@ __device__ __forceinline__ void flash_fwd_f32_mfma_body(const FlashParams& p, co
     }
 }
 
+// ---- the same on the bf16 matrix instructions (f32_x3.hpp), d <= 128 ---------------------------------------------------
+// Tiles, wavefronts, work map and softmax are the fp32 kernel's; what differs is how a tile gets to its operands.  A thread
+// takes 8 consecutive floats at a time into registers, splits them and writes the three pieces into the planes of the tile,
+// whose layouts and swizzles are the 16-bit kernel's: K read by rows, V by transposing reads.  Four wavefronts share that
+// work, so that it is 6 vector instructions per float and a quarter of a wavefront's tile.  Weights are split in the
+// registers they are computed in.  Every tile's V^T P^T starts from zero and is added to O^T (see f32_x3.hpp).
+// One tile of K and one of V are in LDS.  While S^T is computed the next K is on its way to registers, and goes to LDS behind
+// the barrier that ends S^T; V likewise while O^T is computed: half a tile's registers, and the two workgroups of a CU fill
+// each other's barriers.  (Both at once left d = 128 with values in scratch; a reload inside the loop waits for the tile in
+// flight, since loads answer in order: 1010 us where this takes 706, 4 x 2048 x 16, not causal.)
+// Bound: vector arithmetic beside the matrix cores (8.4 vector instructions per matrix instruction at d = 64, each worth about
+// 1.8 cycles of a SIMD that has matrix instructions as well; matrix pipes busy for 55 % of the launch) at the power limit (1.94 GHz).
+// fp32 instructions -> this, us: 4 x 2048 x 16, d = 64 507 -> 377, d = 128 976 -> 706 (194 TFLOP/s, 1.24 of the fp32 peak); causal
+// 4 x 2048 x 32, d = 128 1052 -> 778; 8 x 1000 x 12, d = 96 280 -> 186; 4 x 512 x 16, d = 128 (one workgroup per CU) 73 -> 69.
+//
+// Returns whether the workgroup met a value that cannot be split, in which case what it wrote is void.  (Uniform.)
+template <int D> struct F32Fwd {
+    typedef X3Tile<D> XT;
+    static constexpr int kX3Bytes = 2 * XT::kBytes;
+    // d = 128: the queries' last pieces wait in LDS (80 KiB with them, half of a CU's); with all three in registers the
+    // 256 that two workgroups per CU have would not do
+    static constexpr bool kLowQueriesInLds = D == 128;
+    static constexpr int kLowBytes = kLowQueriesInLds ? kFlashRows * 2 * D : 0;
+    static constexpr int kF32Bytes = 4 * kF32Keys * 4 * D;  // two stages of K and V as floats
+    static constexpr int kLdsBytes = kX3Bytes + kLowBytes > kF32Bytes ? kX3Bytes + kLowBytes : kF32Bytes;
+};
+
+template <int D, bool CAUSAL, bool VARLEN, bool MASKED, bool STATS>
+__device__ __forceinline__ bool flash_fwd_f32_x3_body(const FlashParams& p, const FlashStatsOut& st, unsigned char* lds) {
+    static_assert(D == 64 || D == 128, "head dimensions of this form");
+    static_assert(!(MASKED && (VARLEN || STATS)), "the mask belongs to dense forward launches");
+    typedef X3Tile<D> XT;
+    typedef FlashTile<D> TL;
+    constexpr int KS = D / 16;                       // k-steps of the first product
+    constexpr int MB = D / 32;                       // 32-row blocks of O^T
+    constexpr int RB = XT::RB;
+    constexpr int UPT = 32 * XT::CH / kFlashThreads;  // groups of 8 floats per thread, K and V each
+
+    const int tid = threadIdx.x;
+    const int wave = tid >> 6;
+    const int lane = tid & 63;
+    const int col = lane & 31;   // query column / operand row owned by this lane
+    const int half = lane >> 5;
+    const FlashWork work = flash_work_of_block(blockIdx.x, p);
+    if (!work.valid) return false;
+    // whatever the map says, nothing outside the tensors is ever addressed (uniform per workgroup)
+    if (work.bh < 0 || work.bh >= p.n_bh || work.slot < 0 || work.slot >= flash_per_head(p)) return false;
+    const int slot = work.slot;
+    const int b = work.bh / p.H;
+    const int h = work.bh - b * p.H;
+    const int hk = h / p.kv_group;
+    int L;
+    int64_t base, kv_base;
+    if (VARLEN) {
+        const int s0 = p.cu_seqlens[b];
+        L = p.cu_seqlens[b + 1] - s0;
+        base = (int64_t)s0 * p.stride_n + (int64_t)h * p.stride_h;
+        kv_base = (int64_t)s0 * p.kv_stride_n + (int64_t)hk * p.kv_stride_h;
+    } else {
+        L = p.N;
+        base = (int64_t)b * p.stride_b + (int64_t)h * p.stride_h;
+        kv_base = (int64_t)b * p.kv_stride_b + (int64_t)hk * p.kv_stride_h;
+    }
+    const int n_q = VARLEN ? (L + kFlashRows - 1) / kFlashRows : p.n_qtiles;
+    if (VARLEN && slot >= (p.paired ? (n_q + 1) >> 1 : n_q)) return false;
+    const float* const gq = static_cast<const float*>(p.q) + base;
+    const float* const gk = static_cast<const float*>(p.k) + kv_base;
+    const float* const gv = static_cast<const float*>(p.v) + kv_base;
+    float* const go = STATS ? nullptr : static_cast<float*>(p.o) + base;
+    const int64_t sn = p.stride_n;
+    const int64_t skv = p.kv_stride_n;
+    const int d_real = (p.d_real > 0 && p.d_real < D) ? p.d_real : D;
+    Magnitudes seen_values;
+
+    // ---- a tile's way into LDS: thread t takes group t + 256 i, row (group / groups per row)
+    float raw[UPT][8];
+    const int unit_row = tid / XT::CH, unit_chunk = tid % XT::CH;
+    constexpr int kRowStep = kFlashThreads / XT::CH;  // rows between a thread's groups
+    // (a head dimension below D, FlashParams::d_real: quads from d_real on are the row's first quad again)
+    const uint32_t quad0 = 8 * unit_chunk < d_real ? 8 * unit_chunk : 0, quad1 = 8 * unit_chunk + 4 < d_real ? 8 * unit_chunk + 4 : 0;
+    auto request = [&](const float* from, int k0) __attribute__((always_inline)) {
+        const float* const tile = from + (int64_t)k0 * skv;
+        const int left = L - 1 - k0;  // (rows behind the last one: the last one again)
+#pragma unroll
+        for (int i = 0; i < UPT; ++i) {
+            const int row = unit_row + i * kRowStep;
+            const uint32_t at = (uint32_t)(row < left ? row : left) * (uint32_t)skv;  // rows of a tile: below 2^31 bytes apart
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(tile + (at + quad0)), hi = *reinterpret_cast<const f32x4*>(tile + (at + quad1));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                raw[i][e] = lo[e];
+                raw[i][4 + e] = hi[e];
+            }
+        }
+    };
+    unsigned char* const tile_k = lds;
+    unsigned char* const tile_v = lds + XT::kBytes;
+    auto deliver_k = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < UPT; ++i) {
+            const int r = unit_row + i * kRowStep;
+            seen_values.see(raw[i]);
+            XT::put(tile_k, r, unit_chunk ^ TL::fk(r), split_f32(raw[i]));
+        }
+    };
+    auto deliver_v = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < UPT; ++i) {
+            const int r = unit_row + i * kRowStep;
+            // (rows behind the sequence: their scores are removed, and zeros keep 0 * x finite)
+            if (k0 + kF32Keys > L) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) raw[i][e] = k0 + r < L ? raw[i][e] : 0.0f;
+            }
+            seen_values.see(raw[i]);
+            XT::put(tile_v, r, unit_chunk ^ TL::fv(r), split_f32(raw[i]));
+        }
+    };
+
+    // ---- operand addresses inside a plane (the 16-bit kernel's; step ks and block mb exchange chunk bits of the first's)
+    const int k_off = col * RB + ((half ^ TL::fk(col)) << 4);  // chunk 2 ks + half of row col: ^ ks << 5
+    const int vi = lane & 15;
+    const int vkey = 4 * half + (vi >> 2);
+    const int v_off = vkey * RB + (((2 * ((lane >> 4) & 1) + ((vi & 3) >> 1)) ^ TL::fv(vkey)) << 4) + 8 * (vi & 1);  // ^ mb << 6
+    auto v_operand = [&](const unsigned char* plane, int mb, int g) __attribute__((always_inline)) {
+        const u32x2 a = TrRead<bf16_t>::load(plane + (v_off ^ (mb << 6)) + (16 * g) * RB);
+        const u32x2 c = TrRead<bf16_t>::load(plane + (v_off ^ (mb << 6)) + (16 * g + 8) * RB);
+        return u32x4{a[0], a[1], c[0], c[1]};
+    };
+
+    for (int part = 0; part < 2; ++part) {
+        const int qt = flash_qtile_of_part(p, n_q, slot, part);
+        if (qt < 0) break;
+        const int q_tile0 = qt * kFlashRows;
+        if (q_tile0 >= L) continue;
+        request(gk, 0);
+        // ---- Q^T as B operands: step ks holds d = 16 ks + 8 half .. + 7 of this lane's query, pre-scaled
+        const int qw = q_tile0 + wave * 32;
+        const int qrow = qw + col;
+        u32x4 q_h[KS], q_m[KS], q_l[F32Fwd<D>::kLowQueriesInLds ? 1 : KS];
+        unsigned char* const low = lds + F32Fwd<D>::kX3Bytes + wave * (KS * 1024) + lane * 16;  // this wavefront's own
+        {
+            const float c = p.scale_log2;
+            const float* src = gq + (int64_t)(qrow < L ? qrow : L - 1) * sn;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                if (ks % (D == 128 ? 2 : 4) == 0) __builtin_amdgcn_sched_barrier(0);  // (all of them in flight would push finished ones out of the registers)
+                float x[8];
+#pragma unroll
+                for (int v = 0; v < 2; ++v) {
+                    // (columns the tensors do not have: the row's first quad, then zeros; a load under a condition would be
+                    // waited for before the next one is requested)
+                    const bool there = 16 * ks + 8 * half + 4 * v < d_real;
+                    const f32x4 raw = *reinterpret_cast<const f32x4*>(src + (there ? 16 * ks + 8 * half + 4 * v : 0));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[4 * v + e] = there ? raw[e] * c : 0.0f;
+                }
+                seen_values.see(x);
+                const F32x3 piece = split_f32(x);
+                q_h[ks] = piece.h;
+                q_m[ks] = piece.m;
+                if constexpr (F32Fwd<D>::kLowQueriesInLds) *reinterpret_cast<u32x4*>(low + ks * 1024) = piece.l;
+                else q_l[ks] = piece.l;
+            }
+        }
+
+        f32x16 oacc[MB];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) oacc[mb][r] = 0.0f;
+        float neg_m = 0.0f;
+        float l_run = 0.0f;
+        bool first = true;
+        bool seen = false;  // masked launches: this lane's query has met a key it may attend to
+        constexpr float kRaise = 8.0f;  // raise the reference maximum only when exceeded by 2^8
+        const uint64_t* const mword = MASKED ? p.mask_bits + (int64_t)b * p.mask_kt * p.N + (qrow < L ? qrow : L - 1) : nullptr;
+
+        int k_end = L;
+        if (CAUSAL) k_end = (q_tile0 + kFlashRows) < L ? (q_tile0 + kFlashRows) : L;
+        const int n_tiles = (k_end + kF32Keys - 1) / kF32Keys;
+
+        // ---- S^T = c K Q^T - m, the small products in a sum of their own
+        auto scores = [&](f32x16& s) __attribute__((always_inline)) {
+            f32x16 s_low;
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s_low[r] = 0.0f;
+            s = s_low;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                F32x3 own{q_h[ks], q_m[ks], u32x4{}};
+                if constexpr (F32Fwd<D>::kLowQueriesInLds) own.l = lds_read_b128(low + ks * 1024);
+                else own.l = q_l[ks];
+                mfma_x3(XT::row_operand(tile_k + (k_off ^ (ks << 5))), own, s, s_low);
+            }
+            // the operands of a step are requested in front of the products of the step before it
+            constexpr int kReads = F32Fwd<D>::kLowQueriesInLds ? 4 : 3;
+            __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);  // LDS reads
+#pragma unroll
+            for (int ks = 1; ks < KS; ++ks) {
+                __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);  // matrix instructions
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+            __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = (s[r] + neg_m) + s_low[r];
+        };
+        auto weights_and_output = [&](f32x16 s, int k0, uint64_t mw) __attribute__((always_inline)) {
+            // key of register r: k0 + 8 (r / 4) + 4 half + r % 4; visible iff key <= min(qrow, L - 1)
+            const bool need_mask = (k0 + kF32Keys > L) || (CAUSAL && (k0 + kF32Keys - 1 > qw));
+            if (need_mask) {
+                int lim = L - 1;
+                if (CAUSAL) lim = qrow < lim ? qrow : lim;
+                lim -= k0 + 4 * half;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] = (8 * (r >> 2) + (r & 3)) <= lim ? s[r] : -INFINITY;
+            }
+            if constexpr (MASKED) {
+                // the word holds 64 keys, the tile is its lower or upper half; the lane's keys are 4 half + 8 (r / 4) + r % 4
+                const uint32_t word = (uint32_t)(mw >> ((k0 & 32) + 4 * half));
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int pos = 8 * (r >> 2) + (r & 3);
+                    const uint32_t keep = (uint32_t)((int32_t)(word << (31 - pos)) >> 31);
+                    s[r] = as_f32((as_u32(s[r]) & keep) | (0xFF800000u & ~keep));
+                }
+            }
+            float mx = s[0];
+#pragma unroll
+            for (int r = 1; r < 16; r += 2) mx = r + 1 < 16 ? max3(mx, s[r], s[r + 1]) : max3(mx, s[r], s[r]);
+            bool adjust;
+            if constexpr (MASKED) adjust = __builtin_amdgcn_ballot_w64(seen ? mx > kRaise : mx > -INFINITY) != 0;
+            else adjust = first || __builtin_amdgcn_ballot_w64(mx > kRaise) != 0;
+            if (adjust) {
+                mx = halves_max(mx);  // both lanes of a query agree
+                float delta, alpha;
+                if constexpr (MASKED) {
+                    // a query without a visible key so far has accumulated nothing: its maximum is set exactly, nothing
+                    // is rescaled; one that still sees none stays as it is
+                    delta = seen ? fmaxf(mx, 0.0f) : (mx > -INFINITY ? mx : 0.0f);
+                    alpha = seen ? fast_exp2(-delta) : 1.0f;
+                    seen = seen || mx > -INFINITY;
+                } else {
+                    delta = first ? mx : fmaxf(mx, 0.0f);
+                    alpha = first ? 1.0f : fast_exp2(-delta);  // (scores below -128 would make it infinite, times zeros)
+                }
+                l_run *= alpha;
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) oacc[mb][r] *= alpha;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] -= delta;
+                neg_m -= delta;
+                first = false;
+            }
+            float sum = 0.0f;
+            F32x3 pw[2];  // B operands: registers 8 g .. 8 g + 7 are the keys of k-step g in the order V's operand has them
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    x[e] = fast_exp2(s[8 * g + e]);
+                    sum += x[e];
+                }
+                pw[g] = split_f32(x);
+            }
+            l_run += sum;
+            // ---- O^T += V^T P^T
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                f32x16 t;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) t[r] = 0.0f;
+#pragma unroll
+                for (int g = 0; g < 2; ++g)
+                    mfma_x3(F32x3{v_operand(tile_v, mb, g), v_operand(tile_v + XT::kPlane, mb, g), v_operand(tile_v + 2 * XT::kPlane, mb, g)}, pw[g], t, t);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[mb][r] += t[r];
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+            for (int i = 1; i < 2 * MB; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+            __builtin_amdgcn_s_setprio(0);
+        };
+
+        // (not causal: always, which the compiler must not know: with the two products in one block it schedules them into
+        // each other, and at d = 128 values go to scratch inside the loop)
+        int last_active = CAUSAL ? __builtin_amdgcn_readfirstlane(qw) + 31 : 0x7FFFFFFF;
+#if !defined(AHPC_TRACED_LDS_READ_B128) && defined(__HIP_DEVICE_COMPILE__)
+        if (!CAUSAL) asm volatile("" : "+s"(last_active));
+#endif
+        deliver_k();
+        request(gv, 0);
+        deliver_v(0);
+        __syncthreads();
+        for (int t = 0; t < n_tiles; ++t) {
+            const int k0 = t * kF32Keys;
+            const bool more = t + 1 < n_tiles;
+            // a wavefront whose queries all precede this tile has nothing to add
+            const bool active = k0 <= last_active;
+            uint64_t mw = 0;
+            if constexpr (MASKED) mw = mword[(int64_t)(k0 >> 6) * p.N];
+            if (more) request(gk, k0 + kF32Keys);
+            __builtin_amdgcn_sched_barrier(0);
+            f32x16 s;
+            if (active) scores(s);
+            __syncthreads();  // everyone is done with the tile's K, and its V is there
+            if (more) {
+                deliver_k();
+                request(gv, k0 + kF32Keys);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (active) weights_and_output(s, k0, mw);
+            __syncthreads();  // everyone is done with the tile's V, and the next tile's K is there
+            if (more) deliver_v(k0 + kF32Keys);
+        }
+
+        // ---- normalise and store: per 32-row block a lane holds 4 runs of 4 consecutive d of its query
+        const float l = halves_sum(l_run);
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        if constexpr (STATS) {
+            // delta = dO . O over the elements this lane holds, then over the two lanes of the query
+            float part_sum = 0.0f;
+            if (qrow < L) {
+                const float* src = static_cast<const float*>(st.d_out) + base + (int64_t)qrow * sn + 4 * half;
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                    for (int g4 = 0; g4 < 4; ++g4) {
+                        if (32 * mb + 8 * g4 + 4 * half >= d_real) continue;  // columns the tensors do not have
+                        const f32x4 w = *reinterpret_cast<const f32x4*>(src + 32 * mb + 8 * g4);
+                        part_sum += oacc[mb][4 * g4] * w[0] + oacc[mb][4 * g4 + 1] * w[1] + oacc[mb][4 * g4 + 2] * w[2] +
+                                    oacc[mb][4 * g4 + 3] * w[3];
+                    }
+            }
+            const float delta = halves_sum(part_sum) * inv;
+            if (half == 0) {  // every row of the 128-row tile gets a value: the statistics arrays are padded to whole tiles
+                const int64_t row = (int64_t)work.bh * st.rows_padded + qrow;
+                const bool live = qrow < L && l > 0.0f;
+                st.neg_lse2[row] = live ? neg_m - __builtin_log2f(l) : -INFINITY;
+                st.neg_delta[row] = live ? -delta : 0.0f;
+            }
+        } else if (qrow < L) {
+            float* dst = go + (int64_t)qrow * sn + 4 * half;
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int g4 = 0; g4 < 4; ++g4)
+                    if (32 * mb + 8 * g4 + 4 * half < d_real)
+                        *reinterpret_cast<f32x4*>(dst + 32 * mb + 8 * g4) =
+                            f32x4{oacc[mb][4 * g4] * inv, oacc[mb][4 * g4 + 1] * inv, oacc[mb][4 * g4 + 2] * inv, oacc[mb][4 * g4 + 3] * inv};
+        }
+    }
+    int* const flag = reinterpret_cast<int*>(lds);  // (every pass ends with a barrier behind its last tile)
+    if (tid == 0) *flag = 0;
+    __syncthreads();
+    if (!seen_values.in_range()) *flag = 1;
+    __syncthreads();
+    const bool again = *flag != 0;
+    __syncthreads();  // (before anyone reuses the memory)
+    return again;
+}
+
+// d = 256: the fp32 instructions, its operands as three pieces would not fit the registers.
+template <int D, bool CAUSAL, bool VARLEN, bool MASKED, bool STATS>
+__device__ __forceinline__ void flash_fwd_f32_kernel_body(const FlashParams& p, const FlashStatsOut& st) {
+    if constexpr (D == 256) {
+        constexpr int kTileBytes = kF32Keys * 4 * D;
+        __shared__ __attribute__((aligned(1024))) unsigned char lds_k0[kTileBytes];
+        __shared__ __attribute__((aligned(1024))) unsigned char lds_v0[kTileBytes];
+        __shared__ __attribute__((aligned(1024))) unsigned char lds_k1[kTileBytes];
+        __shared__ __attribute__((aligned(1024))) unsigned char lds_v1[kTileBytes];
+        flash_fwd_f32_mfma_body<D, CAUSAL, VARLEN, MASKED, STATS>(p, st, lds_k0, lds_v0, lds_k1, lds_v1);
+    } else {
+        constexpr int kTileBytes = kF32Keys * 4 * D;
+        __shared__ __attribute__((aligned(1024))) unsigned char lds[F32Fwd<D>::kLdsBytes];
+        if (flash_fwd_f32_x3_body<D, CAUSAL, VARLEN, MASKED, STATS>(p, st, lds))
+            flash_fwd_f32_mfma_body<D, CAUSAL, VARLEN, MASKED, STATS>(p, st, lds, lds + kTileBytes, lds + 2 * kTileBytes, lds + 3 * kTileBytes);
+    }
+}
+
 template <int D, bool CAUSAL, bool VARLEN, bool MASKED = false>
 __global__ __launch_bounds__(kFlashThreads, D == 256 ? 1 : 2) void flash_fwd_f32_mfma_kernel(const FlashParams p) {
-    flash_fwd_f32_mfma_body<D, CAUSAL, VARLEN, MASKED, false>(p, FlashStatsOut{});
+    flash_fwd_f32_kernel_body<D, CAUSAL, VARLEN, MASKED, false>(p, FlashStatsOut{});
 }
 
 template <int D, bool CAUSAL, bool VARLEN>
 __global__ __launch_bounds__(kFlashThreads, 2) void flash_bwd_stats_f32_mfma_kernel(const FlashParams p, const FlashStatsOut st) {
-    flash_fwd_f32_mfma_body<D, CAUSAL, VARLEN, false, true>(p, st);
+    flash_fwd_f32_kernel_body<D, CAUSAL, VARLEN, false, true>(p, st);
 }
 
 }  // namespace ahpc
