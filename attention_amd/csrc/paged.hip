@@ -359,7 +359,11 @@ template <int LPH> __device__ __forceinline__ float head_allreduce(float x) {
 // DUMP: nothing is loaded or computed; instead the lane that owns (pool head 0, element 0) stores, for every token
 // row the kernel would read, the element offset of that row in the pool - taken from the very expression the loads
 // use - and -1 for the tokens of its chunk it would not read.  This is what the bit-exact index test compares.
-template <typename T, int D, int PT, int G, bool DUMP = false>
+//
+// SHARE: the wavefronts of a workgroup work on the same heads and share the chunk's batches of tokens out (wavefront w takes batches
+// w, w + waves, ..); their results become one in LDS at the end (decode_share_for).
+constexpr int lane_share_waves(int group) { return group >= 8 ? 4 : 8; }  // most that share: their results fit 80 KiB of LDS
+template <typename T, int D, int PT, int G, bool DUMP = false, bool SHARE = false>
 __global__ __launch_bounds__(512) void paged_decode_kernel(const DecodeParams p) {
     constexpr int kDecodeBatch = G >= 4 ? 4 : 8;  // tokens whose K and V rows are in flight together, per lane
     constexpr int EPL = 16 / (int)sizeof(T);
@@ -375,7 +379,7 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(const DecodeParams p)
     // token row are dispatched side by side and stream whole pages between them
     const int chunk = blockIdx.y;
     const int b = blockIdx.z;
-    const int h_raw = (blockIdx.x * waves + wave) * HPW + lane / LPH;  // pool head
+    const int h_raw = (SHARE ? blockIdx.x : blockIdx.x * waves + wave) * HPW + lane / LPH;  // pool head
     const bool head_ok = h_raw < p.H_kv;
     const int h = head_ok ? h_raw : p.H_kv - 1;
     const int e0 = (lane % LPH) * EPL;
@@ -456,6 +460,7 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(const DecodeParams p)
 
     const int n_tok = t1 - t0;            // 0 when the chunk's first page is missing
     const int n_batches = (n_tok + kDecodeBatch - 1) / kDecodeBatch;
+    const int first_batch = SHARE ? wave : 0, batch_step = SHARE ? waves : 1;
 
     // Requests the K and V rows of batch `bi` (tokens 8*bi .. 8*bi+7 of the chunk).  Tokens past the
     // end of the chunk re-read the last valid one; their scores are masked when the batch is consumed.
@@ -558,20 +563,50 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(const DecodeParams p)
         for (int bi = 0; bi < n_batches; ++bi) issue(ka, va, bi);
         return;
     }
-    if (n_batches > 0) issue(ka, va, 0);
-    for (int bi = 0; bi < n_batches; bi += 2) {
-        if (bi + 1 < n_batches) issue(kb2, vb2, bi + 1);
+    if (first_batch < n_batches) issue(ka, va, first_batch);
+    for (int bi = first_batch; bi < n_batches; bi += 2 * batch_step) {
+        if (bi + batch_step < n_batches) issue(kb2, vb2, bi + batch_step);
         consume(ka, va, bi);
-        if (bi + 1 < n_batches) {
-            if (bi + 2 < n_batches) issue(ka, va, bi + 2);
-            consume(kb2, vb2, bi + 1);
+        if (bi + batch_step < n_batches) {
+            if (bi + 2 * batch_step < n_batches) issue(ka, va, bi + 2 * batch_step);
+            consume(kb2, vb2, bi + batch_step);
         }
     }
 
+    if constexpr (SHARE) {
+        // every wavefront's m, l and accumulators, [wavefront][value][lane]; wavefront w merges the query heads w, w + waves, ..
+        constexpr int kValues = EPL + 2;
+        __shared__ float share[lane_share_waves(G)][G * kValues][kWave];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            share[wave][g * kValues][lane] = m[g];
+            share[wave][g * kValues + 1][lane] = l[g];
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) share[wave][g * kValues + 2 + e][lane] = acc[g][e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            if (g % waves != wave) continue;  // (uniform; not stored below)
+            float top = -INFINITY;
+            for (int w = 0; w < waves; ++w) top = fmaxf(top, share[w][g * kValues][lane]);
+            l[g] = 0.0f;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) acc[g][e] = 0.0f;
+            for (int w = 0; w < waves; ++w) {
+                const float f = top > -INFINITY ? fast_exp2(share[w][g * kValues][lane] - top) : 0.0f;
+                l[g] = __builtin_fmaf(share[w][g * kValues + 1][lane], f, l[g]);
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) acc[g][e] = __builtin_fmaf(share[w][g * kValues + 2 + e][lane], f, acc[g][e]);
+            }
+            m[g] = top;
+        }
+    }
     if (!head_ok) return;
 #pragma unroll
     for (int g = 0; g < G; ++g) {
         if (g >= gr) break;
+        if (SHARE && g % waves != wave) continue;
         const int hq = h * group + g0 + g;
         if (p.n_chunks == 1) {
             const float inv = l[g] > 0.0f ? 1.0f / l[g] : 0.0f;
@@ -700,9 +735,46 @@ static int64_t fit_chunk(int64_t chunk, int64_t P) {
 
 // Tokens per chunk and wavefronts per workgroup of one decode launch.  row_waves = wavefronts that cover the
 // pool heads of one token (each wave works alone; waves only sets how many heads travel together).
-struct DecodePlan { int64_t chunk; int waves; };
+// share: wavefronts that share a chunk (1: none do; the kernel for the widest groups has its own sharing, `waves`).
+struct DecodePlan { int64_t chunk; int waves; int share = 1; };
 
-static DecodePlan plan_decode(int64_t B, int64_t H_kv, int64_t group, int64_t row_waves, int64_t max_len, int64_t P,
+// How many wavefronts share a chunk.  A wavefront on its own walks a chunk in steps that are a round trip to memory each (a page, or a
+// batch of 4 or 8 tokens of the lane-per-element kernel), about 1 us: 128 tokens took 8 to 16 us however little a launch had to read.
+//   lane-per-element kernel: always.  Eight where there are few chunks (`combinations`: batch entries x chunks x wavefronts' worth of
+//   heads) or they are long; four otherwise, whose workgroups share a CU better.  us, alone -> shared: 1 x 777, 32 heads 19.6 -> 11.0;
+//   1 x 200, 8 heads 18.8 -> 10.7; 13 x 94, 32 heads, d = 96 14.8 -> 7.5; 8 x 1000..8000, 24 heads over 6, d = 96 72.8 -> 42.6;
+//   64 x 512..4096, 32 heads 434 -> 414; 8 x 16384..32768 513 -> 494.
+//   matrix-core kernel: eight (four at d = 256: 128 KiB of page slots) up to a workgroup per CU, half as many up to two while chunks are short, none beyond,
+//   where the stream is the bound and neighbouring heads side by side read whole token rows (16 x 512..4096, 32 heads over 8: 32.6 us alone, 37
+//   with two, 43 with eight) - unless the heads do not fill their workgroups (12 pool heads in workgroups of 8: 57 x 2048 102 -> 85).
+//   1 x 777, 32 heads over 8 11.6 -> 9.7; 1 x 30000 over 2 28.1 -> 18.5; 100 x 16..64, 8 heads over 4 7.3 -> 6.2.
+static int decode_share_for(bool matrix_kernel, int64_t combinations, int64_t H_kv, int64_t group, int64_t d, int64_t chunk, int64_t max_len) {
+    const int most = matrix_kernel ? (d <= 128 ? 8 : 4) : lane_share_waves((int)(group < 8 ? group : 8));
+    int64_t share = tuning().decode_share.load();
+    if (share <= 0) {
+        if (tuning().decode_waves.load() > 0) share = 1;
+        else if (matrix_kernel) {
+            const int64_t side_by_side = H_kv >= 8 && d <= 128 ? 8 : H_kv >= 4 ? 4 : H_kv >= 2 ? 2 : 1;
+            share = combinations <= 256 ? most : combinations <= 512 && chunk <= 512 ? most / 2 : H_kv % side_by_side && d <= 128 ? 4 : 1;
+        } else {
+            share = combinations <= 256 || (group == 1 && chunk >= 1024 && max_len >= 1024) ? 8 : 4;
+        }
+    }
+    share = share >= 8 ? 8 : share >= 4 ? 4 : share >= 2 ? 2 : 1;
+    return (int)(share < most ? share : most);
+}
+
+// Contexts that one chunk holds with no longer a walk than the launch and the partials of a merge cost (4 to 5 us): up to 256 tokens, and up
+// to six pages for each of the wavefronts that share it where every sequence and head has a CU.  Two or three chunks of 128 and a merge
+// took, us: 2 x 136, 16 heads 11.3, now 7.8; 2 x 129, 64 heads over 8 10.2 -> 6.0; 20 x 173, 64 over 8 10.7 -> 5.3; 81 x 137, 24 over
+// 12 21.1 -> 15.5; 2 x 627, 32 over 8, d = 64 9.2 -> 6.3; 6 x 332, 32 over 2 10.2 -> 7.6.  (Not for lane-per-element groups beyond 2, whose
+// walk is arithmetic: 2 x 240, 64 over 8, fp32 24.1 in two chunks, 32.5 in one.)
+static bool decode_in_one_chunk(bool matrix_kernel, int64_t B, int64_t H_kv, int64_t group, int64_t d, int64_t max_len) {
+    if (!matrix_kernel) return group <= 2 && max_len <= 256;
+    return max_len <= 256 || (B * H_kv <= 256 && max_len <= 6 * 16 * (d <= 128 ? 8 : 4));
+}
+
+static DecodePlan plan_decode(int64_t B, int64_t H_kv, int64_t group, int64_t d, int64_t row_waves, int64_t max_len, int64_t P,
                               int64_t requested, bool matrix_kernel = false, int wide_max_waves = 0) {
     DecodePlan plan{requested, (int)tuning().decode_waves.load()};
     if (plan.waves < 0 || plan.waves > 8) plan.waves = 0;
@@ -733,6 +805,12 @@ static DecodePlan plan_decode(int64_t B, int64_t H_kv, int64_t group, int64_t ro
     if (plan.chunk > 0) {
         plan.chunk = fit_chunk(plan.chunk, P);
         if (!plan.waves) plan.waves = 2;
+        return plan;
+    }
+    if (P == 16 && tuning().decode_waves.load() <= 0 && tuning().decode_share.load() != 1 &&
+        decode_in_one_chunk(matrix_kernel, B, H_kv, group, d, max_len)) {
+        plan.chunk = fit_chunk(max_len, P);
+        if (!plan.waves) plan.waves = 1;
         return plan;
     }
     if (matrix_kernel) {
@@ -775,7 +853,24 @@ static DecodePlan plan_decode(int64_t B, int64_t H_kv, int64_t group, int64_t ro
 }
 
 template <typename T, int PT, int G>
-static int launch_decode_dpg(const DecodeParams& p, dim3 grid, dim3 block, hipStream_t st) {
+static int launch_decode_dpg(const DecodeParams& p, dim3 grid, dim3 block, int share, hipStream_t st) {
+    if constexpr (PT == 16) {
+        if (share > lane_share_waves(G)) share = lane_share_waves(G);
+        if (share > 1) {
+            constexpr int epl = 16 / (int)sizeof(T);
+            const int hpw = kWave * epl / p.d_kernel;
+            grid.x = (unsigned)((p.H_kv + hpw - 1) / hpw);
+            block.x = (unsigned)(kWave * share);
+            switch (p.d_kernel) {
+                case 32: hipLaunchKernelGGL((paged_decode_kernel<T, 32, PT, G, false, true>), grid, block, 0, st, p); break;
+                case 64: hipLaunchKernelGGL((paged_decode_kernel<T, 64, PT, G, false, true>), grid, block, 0, st, p); break;
+                case 128: hipLaunchKernelGGL((paged_decode_kernel<T, 128, PT, G, false, true>), grid, block, 0, st, p); break;
+                case 256: hipLaunchKernelGGL((paged_decode_kernel<T, 256, PT, G, false, true>), grid, block, 0, st, p); break;
+                default: return AHPC_ERR_UNSUPPORTED_HEAD_DIM;
+            }
+            return static_cast<int>(hipGetLastError());
+        }
+    }
     switch (p.d_kernel) {
         case 32: hipLaunchKernelGGL((paged_decode_kernel<T, 32, PT, G>), grid, block, 0, st, p); break;
         case 64: hipLaunchKernelGGL((paged_decode_kernel<T, 64, PT, G>), grid, block, 0, st, p); break;
@@ -787,19 +882,19 @@ static int launch_decode_dpg(const DecodeParams& p, dim3 grid, dim3 block, hipSt
 }
 
 template <typename T, int PT>
-static int launch_decode_dp(const DecodeParams& base, dim3 grid, dim3 block, hipStream_t st) {
+static int launch_decode_dp(const DecodeParams& base, dim3 grid, dim3 block, int share, hipStream_t st) {
     // Instantiated for 1, 2, 4 and 8 query heads per pool head.  A group in between runs on the next size; a wider one
     // in slices of 8 query heads, one launch each (every slice reads the K/V stream again), the last slice on the
     // size that holds it.
     const int group = base.H / base.H_kv;
-    if (group == 1) return launch_decode_dpg<T, PT, 1>(base, grid, block, st);
+    if (group == 1) return launch_decode_dpg<T, PT, 1>(base, grid, block, share, st);
     DecodeParams p = base;
     for (int g0 = 0; g0 < group; g0 += 8) {
         p.g0 = g0;
         const int slice = group - g0 < 8 ? group - g0 : 8;
-        const int rc = slice <= 2 ? launch_decode_dpg<T, PT, 2>(p, grid, block, st)
-                     : slice <= 4 ? launch_decode_dpg<T, PT, 4>(p, grid, block, st)
-                                  : launch_decode_dpg<T, PT, 8>(p, grid, block, st);
+        const int rc = slice <= 2 ? launch_decode_dpg<T, PT, 2>(p, grid, block, share, st)
+                     : slice <= 4 ? launch_decode_dpg<T, PT, 4>(p, grid, block, share, st)
+                                  : launch_decode_dpg<T, PT, 8>(p, grid, block, share, st);
         if (rc) return rc;
     }
     return AHPC_OK;
@@ -834,7 +929,19 @@ static int launch_decode_mfma(const DecodeParams& p, int waves, hipStream_t st) 
 // Matrix-core kernel for groups of up to 16 query heads: a wavefront per (pool head, chunk, batch entry), up to 8
 // pool heads side by side in a workgroup.
 template <typename T, int D>
-static int launch_decode_group_d(const DecodeParams& p, int waves_wanted, hipStream_t st) {
+static int launch_decode_group_d(const DecodeParams& p, int waves_wanted, int share, hipStream_t st) {
+    if (D > 128 && share > 4) share = 4;
+    if (share > 1) {
+        const dim3 grid((unsigned)p.H_kv, (unsigned)p.n_chunks, (unsigned)p.B), block(64 * share);
+        switch (share) {
+            case 8:
+                if constexpr (D <= 128) hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 8, true>), grid, block, 0, st, p);
+                break;
+            case 4: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 4, true>), grid, block, 0, st, p); break;
+            default: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 2, true>), grid, block, 0, st, p); break;
+        }
+        return static_cast<int>(hipGetLastError());
+    }
     // (at d = 256 a wavefront's two page slots take 32 KiB of LDS: four wavefronts at most)
     int w = (p.H_kv >= 8 && D <= 128) ? 8 : p.H_kv >= 4 ? 4 : p.H_kv >= 2 ? 2 : 1;
     // A CU draws about 25 GB/s however many wavefronts ask, so a launch with fewer workgroups than CUs is bound by the
@@ -860,16 +967,16 @@ static int launch_decode_group_d(const DecodeParams& p, int waves_wanted, hipStr
 }
 
 template <typename T>
-static int launch_decode_group(const DecodeParams& p, int waves_wanted, hipStream_t st) {
-    if (p.d == 128) return launch_decode_group_d<T, 128>(p, waves_wanted, st);
-    if (p.d == 64) return launch_decode_group_d<T, 64>(p, waves_wanted, st);
-    if (p.d == 256) return launch_decode_group_d<T, 256>(p, waves_wanted, st);
+static int launch_decode_group(const DecodeParams& p, int waves_wanted, int share, hipStream_t st) {
+    if (p.d == 128) return launch_decode_group_d<T, 128>(p, waves_wanted, share, st);
+    if (p.d == 64) return launch_decode_group_d<T, 64>(p, waves_wanted, share, st);
+    if (p.d == 256) return launch_decode_group_d<T, 256>(p, waves_wanted, share, st);
     return AHPC_ERR_UNSUPPORTED_HEAD_DIM;
 }
 
 template <typename T>
-static int launch_decode_d(const DecodeParams& p, dim3 grid, dim3 block, hipStream_t st) {
-    return p.P == 16 ? launch_decode_dp<T, 16>(p, grid, block, st) : launch_decode_dp<T, 0>(p, grid, block, st);
+static int launch_decode_d(const DecodeParams& p, dim3 grid, dim3 block, int share, hipStream_t st) {
+    return p.P == 16 ? launch_decode_dp<T, 16>(p, grid, block, share, st) : launch_decode_dp<T, 0>(p, grid, block, 1, st);
 }
 
 // ---- scratch of ahpc_hip_paged_decode_noalloc -------------------------------------------------------
@@ -1065,11 +1172,12 @@ int ahpc_hip_paged_decode_gqa(const void* q, void* o, int qo_dtype, const void* 
     const int hpw = 64 / lph;
     const int64_t matrix_from = tuning().decode_matrix_min_group.load();
     const bool use_mfma = mfma_shape && (group > 8 || group >= matrix_from);
-    const DecodePlan plan = plan_decode(B, H_kv, group < 8 ? group : 8, (H_kv + hpw - 1) / hpw, max_len, P, chunk_tokens, use_mfma,
+    DecodePlan plan = plan_decode(B, H_kv, group < 8 ? group : 8, d, (H_kv + hpw - 1) / hpw, max_len, P, chunk_tokens, use_mfma,
                                         use_mfma && group > 16 ? (d <= 128 ? 4 : 2) : 0);
     const int64_t chunk = plan.chunk;
     const int waves = plan.waves;
     const int64_t n_chunks = (max_len + chunk - 1) / chunk;
+    plan.share = decode_share_for(use_mfma, B * n_chunks * (use_mfma ? H_kv : (H_kv + hpw - 1) / hpw), H_kv, group, d, chunk, max_len);
     const size_t need = n_chunks > 1 ? (size_t)(B * n_chunks * H * (d + 2)) * sizeof(float) : 0;
     if (need > 0 && (!workspace || workspace_bytes < need)) return AHPC_ERR_WORKSPACE_TOO_SMALL;
     if (need > 0 && (reinterpret_cast<uintptr_t>(workspace) & 15u)) return AHPC_ERR_BAD_ALIGNMENT;  // partials move in 16-byte pieces
@@ -1101,14 +1209,14 @@ int ahpc_hip_paged_decode_gqa(const void* q, void* o, int qo_dtype, const void* 
     int rc;
     if (use_mfma && group <= 16) {
         const int wanted = (int)tuning().decode_waves.load();
-        rc = pool_dtype == AHPC_F16 ? launch_decode_group<f16_t>(p, wanted, st) : launch_decode_group<bf16_t>(p, wanted, st);
+        rc = pool_dtype == AHPC_F16 ? launch_decode_group<f16_t>(p, wanted, plan.share, st) : launch_decode_group<bf16_t>(p, wanted, plan.share, st);
     } else if (use_mfma) {
         rc = pool_dtype == AHPC_F16 ? launch_decode_mfma<f16_t>(p, waves, st) : launch_decode_mfma<bf16_t>(p, waves, st);
     } else
     switch (pool_dtype) {
-        case AHPC_F32: rc = launch_decode_d<float>(p, grid, block, st); break;
-        case AHPC_F16: rc = launch_decode_d<f16_t>(p, grid, block, st); break;
-        default: rc = launch_decode_d<bf16_t>(p, grid, block, st); break;
+        case AHPC_F32: rc = launch_decode_d<float>(p, grid, block, plan.share, st); break;
+        case AHPC_F16: rc = launch_decode_d<f16_t>(p, grid, block, plan.share, st); break;
+        default: rc = launch_decode_d<bf16_t>(p, grid, block, plan.share, st); break;
     }
     if (rc) return rc;
     if (n_chunks > 1) {
@@ -1165,7 +1273,7 @@ int ahpc_hip_paged_gather_indices(const int32_t* block_table, const int32_t* seq
     if ((d == 32 || d == 64 || d == 128 || d == 256) && B <= 65535 && H <= 65535) {
         // the decode kernel itself (16-bit pool, one query head per pool head), launched for pool head 0 only and with
         // the chunking of a real decode launch (every sequence cut into equal chunks), reports the rows it addresses
-        const int64_t chunk = plan_decode(B, H, 1, (H + 3) / 4, max_len, P, 0).chunk;
+        const int64_t chunk = plan_decode(B, H, 1, d, (H + 3) / 4, max_len, P, 0).chunk;
         const int64_t n_chunks = (max_len + chunk - 1) / chunk;
         if (n_chunks > 65535) return AHPC_ERR_BAD_SHAPE;
         {

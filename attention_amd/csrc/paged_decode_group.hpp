@@ -43,8 +43,11 @@ constexpr int kStreamAux = AHPC_GROUP_AUX;  // cache policy of the K/V loads: 2 
 // counters stay unconstrained).
 constexpr int vmcnt_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
 
-// T: pool element type (16 bit).  D: head dimension (64, 128).  W: wavefronts (= pool heads) per workgroup.
-template <typename T, int D, int W>
+// T: pool element type (16 bit).  D: head dimension (64, 128, 256).  W: wavefronts (= pool heads) per workgroup.
+// SHARE: the W wavefronts of a workgroup work on one pool head instead and share the chunk's pages out (wavefront w takes pages w,
+// w + W, ..); their results (m, l, O) become one in LDS at the end.  For launches of few wavefronts, which are bound by the walk of
+// one of them: a page after the other is a round trip to memory each (decode_share_for).
+template <typename T, int D, int W, bool SHARE = false>
 __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const DecodeParams p) {
     constexpr int RB = 2 * D;          // bytes of one head of one token
     constexpr int CH = RB / 16;        // 16-byte pieces of such a row
@@ -66,8 +69,8 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int col = lane & 15;  // query head of the group (B operands, results) / token of the page (A operand of S^T)
     const int rg = lane >> 4;   // which 8 (or 4) of an instruction's k values / which 4 result rows
-    const int hk = (int)blockIdx.x * W + wave;
-    if (hk >= p.H_kv) return;   // wavefronts are independent: nothing waits for this one
+    const int hk = SHARE ? (int)blockIdx.x : (int)blockIdx.x * W + wave;
+    if (hk >= p.H_kv) return;   // wavefronts are independent: nothing waits for this one (SHARE: the whole workgroup)
     const int chunk = blockIdx.y;
     const int b = blockIdx.z;
     const int G = p.H / p.H_kv;
@@ -99,7 +102,10 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
     }
     my_page = my_page < 0 ? 0 : my_page;  // never dereferenced: no token row of such a page is left in the chunk
     const int n_tok = t1 - t0;            // 0 when the chunk's first page is missing
-    const int n_pages = (n_tok + P - 1) / P;
+    const int all_pages = (n_tok + P - 1) / P;
+    // this wavefront's pages: page_at(0) .. page_at(n_pages - 1) of the chunk
+    auto page_at = [&](int t) __attribute__((always_inline)) { return SHARE ? wave + W * t : t; };
+    const int n_pages = SHARE ? (all_pages > wave ? (all_pages - wave + W - 1) / W : 0) : all_pages;
 
     // ---- Q^T operands: lane (query head col, rg) holds q[32*ks + 8*rg .. +7], times scale*log2(e) ------------
     u32x4 qreg[KS];
@@ -158,8 +164,8 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
     auto issue = [&](int tt, auto slot_c) __attribute__((always_inline)) {
         constexpr int S = decltype(slot_c)::value;
 #if defined(__HIP_DEVICE_COMPILE__)
-        const int page_id = __builtin_amdgcn_readlane(my_page, tt < n_pages ? tt : 0);
-        const int rows = n_tok - tt * P;
+        const int page_id = __builtin_amdgcn_readlane(my_page, tt < n_pages ? page_at(tt) : 0);
+        const int rows = tt < n_pages ? n_tok - page_at(tt) * P : 0;
         const int rc = rows < P ? rows : P;
         const unsigned nrec = rc > 0 ? (unsigned)((rc - 1) * tok_bytes + RB) : 0u;
         const int64_t byte0 = ((int64_t)page_id * P * p.H_kv + hk) * (int64_t)RB;
@@ -197,7 +203,7 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) s = mfma_16x16x32<T>(ka[ks], qreg[ks], s);
         // s[r] belongs to token tt*16 + 4*rg + r, which exists iff it is below n_tok
-        const int lim = n_tok - tt * P - 4 * rg;
+        const int lim = n_tok - page_at(tt) * P - 4 * rg;
         float mx = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -252,22 +258,54 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
 
     float l = l_run + __shfl_xor(l_run, 16, kWave);
     l += __shfl_xor(l, 32, kWave);
-    if (!head_ok) return;
-    if (p.n_chunks == 1) {
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-            const float res[4] = {oacc[mb][0] * inv, oacc[mb][1] * inv, oacc[mb][2] * inv, oacc[mb][3] * inv};
-            store_qo_vec<4>(p.o, p.qo_dtype, ((int64_t)b * p.H + hq) * D + 16 * mb + 4 * rg, res);
-        }
-    } else {
-        const int64_t slot = ((int64_t)b * p.n_chunks + chunk) * p.H + hq;
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) *reinterpret_cast<f32x4*>(p.part_o + slot * D + 16 * mb + 4 * rg) = oacc[mb];
+    float f[SHARE ? W : 1];
+    if constexpr (SHARE) {
+        __shared__ float share_m[W][16], share_l[W][16];
         if (rg == 0) {
-            p.part_ml[slot * 2] = m_run;
-            p.part_ml[slot * 2 + 1] = stopped ? -l : l;  // the merge stops after a chunk that met a missing page
+            share_m[wave][col] = m_run;  // -inf without a page
+            share_l[wave][col] = l;
         }
+        // (every load into the page slots has landed: a wavefront's own slots carry its accumulators)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) *reinterpret_cast<f32x4*>(slot0 + (mb * kWave + lane) * 16) = oacc[mb];
+        __syncthreads();
+        float m = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < W; ++w) m = fmaxf(m, share_m[w][col]);
+        l = 0.0f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            f[w] = m > -INFINITY ? fast_exp2(share_m[w][col] - m) : 0.0f;
+            l = __builtin_fmaf(share_l[w][col], f[w], l);
+        }
+        m_run = m;
+    }
+    if (!head_ok) return;
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const int64_t slot = ((int64_t)b * p.n_chunks + chunk) * p.H + hq;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        f32x4 o = oacc[mb];
+        if constexpr (SHARE) {
+            if (mb % W != wave) continue;  // (uniform)
+            o = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const f32x4 x = *reinterpret_cast<const f32x4*>(lds_v + w * (R * kSlot) + (mb * kWave + lane) * 16);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(x[e], f[w], o[e]);
+            }
+        }
+        if (p.n_chunks == 1) {
+            const float res[4] = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+            store_qo_vec<4>(p.o, p.qo_dtype, ((int64_t)b * p.H + hq) * D + 16 * mb + 4 * rg, res);
+        } else {
+            *reinterpret_cast<f32x4*>(p.part_o + slot * D + 16 * mb + 4 * rg) = o;
+        }
+    }
+    if (p.n_chunks > 1 && rg == 0 && (!SHARE || wave == 0)) {
+        p.part_ml[slot * 2] = m_run;
+        p.part_ml[slot * 2 + 1] = stopped ? -l : l;  // the merge stops after a chunk that met a missing page
     }
 }
 

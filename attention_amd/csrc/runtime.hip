@@ -21,6 +21,7 @@ Tuning::Tuning()
     : flash_pair_min_tiles(env_value("AHPC_FLASH_PAIR_MIN", 0)),
       decode_waves(env_value("AHPC_DECODE_WAVES", 0)),
       decode_chunk(env_value("AHPC_DECODE_CHUNK", 0)),
+      decode_share(env_value("AHPC_DECODE_SHARE", 0)),
       decode_matrix_min_group(env_value("AHPC_DECODE_MFMA_MIN_GROUP", 2)),
       bwd_split(env_value("AHPC_BWD_SPLIT", 0)),
       mask_pack(env_value("AHPC_MASK_PACK", 1)),
@@ -42,6 +43,7 @@ static std::atomic<int64_t>* tuning_slot(const char* name) {
     if (!std::strcmp(name, "flash_pair_min_tiles")) return &t.flash_pair_min_tiles;
     if (!std::strcmp(name, "decode_waves")) return &t.decode_waves;
     if (!std::strcmp(name, "decode_chunk")) return &t.decode_chunk;
+    if (!std::strcmp(name, "decode_share")) return &t.decode_share;
     if (!std::strcmp(name, "decode_matrix_min_group")) return &t.decode_matrix_min_group;
     if (!std::strcmp(name, "bwd_split")) return &t.bwd_split;
     if (!std::strcmp(name, "mask_pack")) return &t.mask_pack;

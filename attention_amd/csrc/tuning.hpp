@@ -18,6 +18,9 @@ struct Tuning {
     std::atomic<int64_t> decode_waves;
     // decode: tokens per context chunk when the caller passes none (AHPC_DECODE_CHUNK, default 0 = by shape)
     std::atomic<int64_t> decode_chunk;
+    // decode, groups of up to 16: wavefronts that share a chunk, 1 (none), 2, 4 or 8; 0 (default) = by shape, none with decode_waves set
+    // (AHPC_DECODE_SHARE)
+    std::atomic<int64_t> decode_share;
     // decode: query heads per K/V head from which on the matrix-core kernels are taken where they apply (16-bit pool,
     // d 64/128, pages of 16).  Default 2: timed on 8 pool heads, the page-by-page matrix-core kernel reaches 0.65-0.72
     // of 8 TB/s for groups of 2, 4 and 8 where the lane-per-element kernel reaches 0.58, 0.55 and 0.36; with one

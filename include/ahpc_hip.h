@@ -67,9 +67,9 @@ typedef struct ahpc_device_info {
     int32_t  runtime_version;
 } ahpc_device_info;
 
-/* Launcher tuning values ("flash_pair_min_tiles", "flash_rows", "flash_walks", "decode_waves", "decode_chunk", "decode_matrix_min_group",
+/* Launcher tuning values ("flash_pair_min_tiles", "flash_rows", "flash_walks", "decode_waves", "decode_chunk", "decode_share", "decode_matrix_min_group",
  * "bwd_split", "bwd_pair", "mask_pack", "pool_in_place"): process-wide, each starts from its environment variable
- * (AHPC_FLASH_PAIR_MIN, AHPC_FLASH_ROWS, AHPC_FLASH_WALKS, AHPC_DECODE_WAVES, AHPC_DECODE_CHUNK, AHPC_DECODE_MFMA_MIN_GROUP, AHPC_BWD_SPLIT,
+ * (AHPC_FLASH_PAIR_MIN, AHPC_FLASH_ROWS, AHPC_FLASH_WALKS, AHPC_DECODE_WAVES, AHPC_DECODE_CHUNK, AHPC_DECODE_SHARE, AHPC_DECODE_MFMA_MIN_GROUP, AHPC_BWD_SPLIT,
  * AHPC_BWD_PAIR, AHPC_MASK_PACK, AHPC_POOL_IN_PLACE), which is read once.  No value
  * changes results by more than the order in which sums are taken; unknown names and negative values are refused.  The reference has no counterpart: its tile sizes
  * sit in PerformanceConfig (src/api/attention_interface.hpp:29-53), which the host classes still honour. */

@@ -1,0 +1,73 @@
+"""Decode launches whose wavefronts share a chunk: 1, 2, 4 and 8 of them, on the lane-per-element and the page-by-page matrix-core
+kernel, against the oracle.  Context lengths around what a round of the wavefronts takes (a batch of 4 or 8 tokens, a page of 16
+each): empty, one token, a part of the wavefronts without work, a last round that is not full; a sequence that a missing page ends
+early, in a chunk's first page and in its middle."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from test_gpu_paged import build_problem, poison_unused
+
+LENS = [0, 1, 8, 15, 16, 17, 33, 64, 65, 127, 128, 129, 143, 200, 257, 300]
+
+
+def _cpu():
+    from simt import simt as S
+    from test_simt_kernels import decode
+    S.load()
+    S.configure(False, 1)
+    emu = S.EmulatedHip()
+    return emu, lambda *a: decode(emu, *a)
+
+
+def _gpu():
+    import torch
+    torch.cuda.init()
+    from attention_amd import hip
+    from gpu_util import to_dev, to_host, stream_ptr, dev_i32
+
+    def decode(q, kp, vp, table, lens, rows, B, H, H_kv, d, P, dtype, qo_dtype, scale, chunk):
+        dq, dk, dv, dt, dl = to_dev(q, qo_dtype), to_dev(kp, dtype), to_dev(vp, dtype), dev_i32(table), dev_i32(lens)
+        do = torch.full_like(dq, float("nan"))
+        max_len = int(max(1, np.max(lens)))
+        n = hip.paged_decode_workspace_bytes(B, H, d, max_len, P, chunk)
+        ws = torch.full((max(n, 4) // 4,), float("nan"), dtype=torch.float32, device="cuda")
+        hip.paged_decode_gqa(dq.data_ptr(), do.data_ptr(), qo_dtype, dk.data_ptr(), dv.data_ptr(), dtype, dt.data_ptr(), dl.data_ptr(), None, B, H,
+                             H_kv, d, P, table.shape[1], max_len, scale, chunk, ws.data_ptr(), n, stream_ptr())
+        torch.cuda.synchronize()
+        return to_host(do)
+
+    return hip, decode
+
+
+@pytest.fixture(params=[_cpu, pytest.param(_gpu, marks=pytest.mark.gpu)], ids=["cpu", "gpu"])
+def target(request):
+    hip, decode = request.param()
+    yield hip, decode
+    hip.set_tuning("decode_share", 0)
+
+
+@pytest.mark.parametrize("H,H_kv,d,dtype", [(3, 3, 128, O.F16), (4, 2, 64, O.F32), (8, 2, 96, O.BF16), (8, 1, 80, O.F16),
+                                            (6, 3, 128, O.BF16), (16, 1, 64, O.F16), (4, 2, 256, O.BF16)])
+def test_wavefronts_that_share_a_chunk(target, H, H_kv, d, dtype):
+    hip, decode = target
+    B, P, g = len(LENS), 16, H // H_kv
+    _, kp, vp, table, lens, _, _ = build_problem(B, H_kv, d, P, LENS, 31, dtype)
+    q = O.round_to(O.fill_normal((B, H, d), 31, 1), dtype)
+    scale = 1.0 / np.sqrt(d)
+    rep = lambda pool: np.repeat(pool.reshape(-1, H_kv, d), g, axis=1).reshape(-1)
+    # two sequences end early: at their third page, and at their ninth
+    cut = np.array(lens)
+    table = table.copy()
+    for b, page in ((13, 2), (15, 8)):
+        cut[b] = min(cut[b], page * P)
+    want = O.paged_decode(q, rep(kp), rep(vp), table, cut, None, B, H, d, P, scale)
+    kp, vp, table = poison_unused(kp, vp, table, cut, P, H_kv, d)
+    for b, page in ((13, 2), (15, 8)):
+        table[b, page] = -1
+    for chunk in (0, 128, 304):
+        for share in (1, 2, 4, 8, 0):
+            hip.set_tuning("decode_share", share)
+            got = decode(q, kp, vp, table, lens, None, B, H, H_kv, d, P, dtype, dtype, scale, chunk)
+            assert np.isfinite(got).all()
+            assert np.abs(got - want).max() <= (1e-4 if dtype == O.F32 else 2e-2), f"chunk {chunk}, {share} wavefronts"
