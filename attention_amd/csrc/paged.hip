@@ -740,15 +740,17 @@ struct DecodePlan { int64_t chunk; int waves; int share = 1; };
 
 // How many wavefronts share a chunk.  A wavefront on its own walks a chunk in steps that are a round trip to memory each (a page, or a
 // batch of 4 or 8 tokens of the lane-per-element kernel), about 1 us: 128 tokens took 8 to 16 us however little a launch had to read.
-//   lane-per-element kernel: always.  Eight where there are few chunks (`combinations`: batch entries x chunks x wavefronts' worth of
-//   heads) or they are long; four otherwise, whose workgroups share a CU better.  us, alone -> shared: 1 x 777, 32 heads 19.6 -> 11.0;
+//   lane-per-element kernel: always, but for launches of whole token rows (`waves` = 8) whose sequences are many chunks each: those are
+//   equally long and stream 1 % faster on their own (8 x 16384..32768 491 us, 495 shared).  Eight where there are few chunks
+//   (`combinations`: batch entries x chunks x wavefronts' worth of heads) or they are long; four otherwise, whose workgroups share a CU
+//   better.  us, alone -> shared: 1 x 777, 32 heads 19.6 -> 11.0;
 //   1 x 200, 8 heads 18.8 -> 10.7; 13 x 94, 32 heads, d = 96 14.8 -> 7.5; 8 x 1000..8000, 24 heads over 6, d = 96 72.8 -> 42.6;
-//   64 x 512..4096, 32 heads 434 -> 414; 8 x 16384..32768 513 -> 494.
+//   64 x 512..4096, 32 heads 438 -> 420; 58 x up to 6810, 16 heads 357 -> 301.
 //   matrix-core kernel: eight (four at d = 256: 128 KiB of page slots) up to a workgroup per CU, half as many up to two while chunks are short, none beyond,
 //   where the stream is the bound and neighbouring heads side by side read whole token rows (16 x 512..4096, 32 heads over 8: 32.6 us alone, 37
 //   with two, 43 with eight) - unless the heads do not fill their workgroups (12 pool heads in workgroups of 8: 57 x 2048 102 -> 85).
 //   1 x 777, 32 heads over 8 11.6 -> 9.7; 1 x 30000 over 2 28.1 -> 18.5; 100 x 16..64, 8 heads over 4 7.3 -> 6.2.
-static int decode_share_for(bool matrix_kernel, int64_t combinations, int64_t H_kv, int64_t group, int64_t d, int64_t chunk, int64_t max_len) {
+static int decode_share_for(bool matrix_kernel, int64_t combinations, int64_t H_kv, int64_t group, int64_t d, int64_t chunk, int64_t n_chunks, int waves) {
     const int most = matrix_kernel ? (d <= 128 ? 8 : 4) : lane_share_waves((int)(group < 8 ? group : 8));
     int64_t share = tuning().decode_share.load();
     if (share <= 0) {
@@ -757,21 +759,22 @@ static int decode_share_for(bool matrix_kernel, int64_t combinations, int64_t H_
             const int64_t side_by_side = H_kv >= 8 && d <= 128 ? 8 : H_kv >= 4 ? 4 : H_kv >= 2 ? 2 : 1;
             share = combinations <= 256 ? most : combinations <= 512 && chunk <= 512 ? most / 2 : H_kv % side_by_side && d <= 128 ? 4 : 1;
         } else {
-            share = combinations <= 256 || (group == 1 && chunk >= 1024 && max_len >= 1024) ? 8 : 4;
+            share = waves == 8 && n_chunks >= 16 ? 1 : combinations <= 256 || (group == 1 && chunk >= 1024 && n_chunks > 1) ? 8 : 4;
         }
     }
     share = share >= 8 ? 8 : share >= 4 ? 4 : share >= 2 ? 2 : 1;
     return (int)(share < most ? share : most);
 }
 
-// Contexts that one chunk holds with no longer a walk than the launch and the partials of a merge cost (4 to 5 us): up to 256 tokens, and up
-// to six pages for each of the wavefronts that share it where every sequence and head has a CU.  Two or three chunks of 128 and a merge
-// took, us: 2 x 136, 16 heads 11.3, now 7.8; 2 x 129, 64 heads over 8 10.2 -> 6.0; 20 x 173, 64 over 8 10.7 -> 5.3; 81 x 137, 24 over
-// 12 21.1 -> 15.5; 2 x 627, 32 over 8, d = 64 9.2 -> 6.3; 6 x 332, 32 over 2 10.2 -> 7.6.  (Not for lane-per-element groups beyond 2, whose
-// walk is arithmetic: 2 x 240, 64 over 8, fp32 24.1 in two chunks, 32.5 in one.)
+// Contexts that are one chunk, without partials and a merge launch (4 to 5 us, and the host's 2.5): up to 256 tokens, and on the
+// matrix-core kernel, where every sequence and head has a CU, up to 1024 (eight pages for each of eight wavefronts; 448 at d = 256, where four
+// share).  In chunks -> in one, us: 2 x 136, 16 heads 11.3 -> 7.8; 2 x 129, 64 heads over 8 10.2 -> 6.0; 81 x 137, 24 over 12 21.1 -> 15.5;
+// 32 heads over 8: 1 x 777 10.1 -> 8.8, 16 x 777 16.1 -> 14.8, 4 x 1024 11.0 -> 13.2, 1 x 1024 10.2 -> 9.8; d = 64 2 x 1024 9.3 -> 7.6; d = 256
+// 1 x 400 13.3 -> 12.7, 1 x 520 13.4 -> 14.0.  (Not for lane-per-element groups beyond 2, whose walk is arithmetic: 2 x 240, 64 over 8,
+// fp32 24.1 in two chunks, 32.5 in one.)
 static bool decode_in_one_chunk(bool matrix_kernel, int64_t B, int64_t H_kv, int64_t group, int64_t d, int64_t max_len) {
     if (!matrix_kernel) return group <= 2 && max_len <= 256;
-    return max_len <= 256 || (B * H_kv <= 256 && max_len <= 6 * 16 * (d <= 128 ? 8 : 4));
+    return max_len <= 256 || (B * H_kv <= 256 && max_len <= (d <= 128 ? 1024 : 448));
 }
 
 static DecodePlan plan_decode(int64_t B, int64_t H_kv, int64_t group, int64_t d, int64_t row_waves, int64_t max_len, int64_t P,
@@ -1177,7 +1180,7 @@ int ahpc_hip_paged_decode_gqa(const void* q, void* o, int qo_dtype, const void* 
     const int64_t chunk = plan.chunk;
     const int waves = plan.waves;
     const int64_t n_chunks = (max_len + chunk - 1) / chunk;
-    plan.share = decode_share_for(use_mfma, B * n_chunks * (use_mfma ? H_kv : (H_kv + hpw - 1) / hpw), H_kv, group, d, chunk, max_len);
+    plan.share = decode_share_for(use_mfma, B * n_chunks * (use_mfma ? H_kv : (H_kv + hpw - 1) / hpw), H_kv, group, d, chunk, n_chunks, waves);
     const size_t need = n_chunks > 1 ? (size_t)(B * n_chunks * H * (d + 2)) * sizeof(float) : 0;
     if (need > 0 && (!workspace || workspace_bytes < need)) return AHPC_ERR_WORKSPACE_TOO_SMALL;
     if (need > 0 && (reinterpret_cast<uintptr_t>(workspace) & 15u)) return AHPC_ERR_BAD_ALIGNMENT;  // partials move in 16-byte pieces

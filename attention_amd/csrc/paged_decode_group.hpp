@@ -165,7 +165,7 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
         constexpr int S = decltype(slot_c)::value;
 #if defined(__HIP_DEVICE_COMPILE__)
         const int page_id = __builtin_amdgcn_readlane(my_page, tt < n_pages ? page_at(tt) : 0);
-        const int rows = tt < n_pages ? n_tok - page_at(tt) * P : 0;
+        const int rows = n_tok - page_at(tt) * P;  // (none for a page behind this wavefront's last: page_at goes past the chunk's end)
         const int rc = rows < P ? rows : P;
         const unsigned nrec = rc > 0 ? (unsigned)((rc - 1) * tok_bytes + RB) : 0u;
         const int64_t byte0 = ((int64_t)page_id * P * p.H_kv + hk) * (int64_t)RB;
