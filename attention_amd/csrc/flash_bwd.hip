@@ -436,7 +436,7 @@ static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const v
         m.mask_bits_t = pm->bits_t;
         m.mask_tiles = pm->tiles;
     }
-    if (int rc = flash_plan_launch(f, B, causal, kFlashRows, rows_128_pair_threshold(D, false, VARLEN, B, f), VARLEN)) return rc;
+    if (int rc = flash_plan_launch(f, B, causal, kFlashRows, rows_128_pair_threshold(tile_dim(D), false, VARLEN, B, f), VARLEN)) return rc;
     const FlashStatsOut st{p.d_out, lse2, delta, p.rows_padded};
     const dim3 block(kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));
@@ -449,7 +449,7 @@ static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const v
         } else {
             if (o_kept && stats_kept && !VARLEN) {
                 // the forward kept its row statistics and its output is at hand: no statistics pass
-                constexpr int LPR = D / 8;
+                constexpr int LPR = tile_dim(D) / 8;
                 const int64_t total_rows = B * p.H * p.rows_padded;
                 const int64_t blocks = (total_rows + kDeltaThreads / LPR - 1) / (kDeltaThreads / LPR);
                 hipLaunchKernelGGL((flash_bwd_delta_kernel<T, LPR>), dim3((unsigned)blocks), dim3(kDeltaThreads), 0, stream,
@@ -480,10 +480,12 @@ static int launch_mfma(const FlashBwdParams& p, const PackedMask* pm, const void
                        bool causal, float* lse2, float* delta, hipStream_t stream) {
     if (p.cu_seqlens) {
         if (pm) return AHPC_ERR_BAD_SHAPE;
+        if (d == 96) return launch_mfma_dv<T, 96, true>(p, nullptr, nullptr, nullptr, B, causal, lse2, delta, stream);
         if (d == 128) return launch_mfma_dv<T, 128, true>(p, nullptr, nullptr, nullptr, B, causal, lse2, delta, stream);
         if (d == 64) return launch_mfma_dv<T, 64, true>(p, nullptr, nullptr, nullptr, B, causal, lse2, delta, stream);
         if (d == 256) return launch_mfma_dv<T, 256, true>(p, nullptr, nullptr, nullptr, B, causal, lse2, delta, stream);
     } else {
+        if (d == 96) return launch_mfma_dv<T, 96, false>(p, pm, o_kept, stats_kept, B, causal, lse2, delta, stream);
         if (d == 128) return launch_mfma_dv<T, 128, false>(p, pm, o_kept, stats_kept, B, causal, lse2, delta, stream);
         if (d == 64) return launch_mfma_dv<T, 64, false>(p, pm, o_kept, stats_kept, B, causal, lse2, delta, stream);
         if (d == 256) return launch_mfma_dv<T, 256, false>(p, pm, o_kept, stats_kept, B, causal, lse2, delta, stream);
@@ -614,7 +616,7 @@ static int flash_bwd_any(const void* d_out, const void* q, const void* k, const 
     // head dimensions up to 256 (fp32: 128) in whole 16-byte pieces; one below 64, 128 or 256 runs on the next kernel
     // (FlashParams::d_real)
     const bool d_ok = d <= (is16 ? 256 : 128) && d >= (is16 ? 8 : 4) && d % (is16 ? 8 : 4) == 0;
-    const int kernel_d = d <= 64 ? 64 : d <= 128 ? 128 : 256;
+    const int kernel_d = d <= 64 ? 64 : d <= 96 && dtype != AHPC_F32 ? 96 : d <= 128 ? 128 : 256;
     const bool tensors_ok = d_ok && (is16 ? strides_ok : strides4_ok) && aligned16(q) && aligned16(k) && aligned16(v) &&
                             aligned16(d_out) && aligned16(d_q) && aligned16(d_k) && aligned16(d_v);
     if (tensors_ok && (!mask || (is16 && !cu_seqlens && tuning().mask_pack.load() != 0))) {

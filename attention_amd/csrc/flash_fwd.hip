@@ -221,10 +221,12 @@ static int flash_walks_for(int D, bool causal, int64_t B, int64_t N, int64_t H) 
     return tiles <= (causal && N >= 4096 ? 512 : 256) ? 2 : 1;
 }
 
+// (d = 96 takes the shape rules of 128; its two walks are the kernel for 128, which halves four row blocks between the sets)
 template <typename T, int D, bool VARLEN>
 static int launch_mfma(FlashParams p, int64_t B, bool causal, hipStream_t stream) {
+    constexpr int R = tile_dim(D);
     if constexpr (D != 256 && !VARLEN) {
-        if (flash_rows_for(D, VARLEN, causal, B, p.N, p.H) == kFlashWideRows) {
+        if (flash_rows_for(R, VARLEN, causal, B, p.N, p.H) == kFlashWideRows) {
             if (int rc = flash_plan_launch(p, B, causal, kFlashWideRows, pair_threshold(true), false)) return rc;
             dim3 grid((unsigned)persistent_grid(p.n_block_ids)), block(64 * kFlashWideWaves);
             if (causal) hipLaunchKernelGGL((flash_fwd_wide_kernel<T, D, true>), grid, block, 0, stream, p);
@@ -233,15 +235,15 @@ static int launch_mfma(FlashParams p, int64_t B, bool causal, hipStream_t stream
         }
     }
     if constexpr (D != 256) {
-        if (flash_walks_for(D, causal, B, p.N, p.H) == 2) {
+        if (flash_walks_for(R, causal, B, p.N, p.H) == 2) {
             if (int rc = flash_plan_launch(p, B, causal, kFlashRows, kNeverPair, VARLEN)) return rc;
             dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(2 * kFlashThreads);
-            if (causal) hipLaunchKernelGGL((flash_fwd_two_walks_kernel<T, D, true, VARLEN>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((flash_fwd_two_walks_kernel<T, D, false, VARLEN>), grid, block, 0, stream, p);
+            if (causal) hipLaunchKernelGGL((flash_fwd_two_walks_kernel<T, R, true, VARLEN>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((flash_fwd_two_walks_kernel<T, R, false, VARLEN>), grid, block, 0, stream, p);
             return static_cast<int>(hipGetLastError());
         }
     }
-    if (int rc = flash_plan_launch(p, B, causal, kFlashRows, rows_128_pair_threshold(D, false, VARLEN, B, p), VARLEN)) return rc;
+    if (int rc = flash_plan_launch(p, B, causal, kFlashRows, rows_128_pair_threshold(tile_dim(D), false, VARLEN, B, p), VARLEN)) return rc;
     dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(kFlashThreads);
     if (causal) hipLaunchKernelGGL((flash_fwd_mfma_kernel<T, D, true, VARLEN>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((flash_fwd_mfma_kernel<T, D, false, VARLEN>), grid, block, 0, stream, p);
@@ -250,7 +252,7 @@ static int launch_mfma(FlashParams p, int64_t B, bool causal, hipStream_t stream
 
 template <typename T, int D, int MASK>
 static int launch_mfma_masked(FlashParams p, int64_t B, bool causal, hipStream_t stream) {
-    if (int rc = flash_plan_launch(p, B, causal, kFlashRows, rows_128_pair_threshold(D, false, false, B, p), false)) return rc;
+    if (int rc = flash_plan_launch(p, B, causal, kFlashRows, rows_128_pair_threshold(tile_dim(D), false, false, B, p), false)) return rc;
     dim3 grid((unsigned)(p.blocks_per_xcd * 8)), block(kFlashThreads);
     if (causal) hipLaunchKernelGGL((flash_fwd_mfma_masked_kernel<T, D, true, MASK>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((flash_fwd_mfma_masked_kernel<T, D, false, MASK>), grid, block, 0, stream, p);
@@ -260,6 +262,7 @@ static int launch_mfma_masked(FlashParams p, int64_t B, bool causal, hipStream_t
 template <typename T, int MASK>
 static int dispatch_mfma_masked(const FlashParams& p, int64_t B, int d, bool causal, hipStream_t stream) {
     if (d == 128) return launch_mfma_masked<T, 128, MASK>(p, B, causal, stream);
+    if (d == 96) return launch_mfma_masked<T, 96, MASK>(p, B, causal, stream);
     if (d == 64) return launch_mfma_masked<T, 64, MASK>(p, B, causal, stream);
     if constexpr (MASK == 2) {  // the packed mask only: the in-place mask's 32 registers do not fit beside d = 256
         if (d == 256) return launch_mfma_masked<T, 256, MASK>(p, B, causal, stream);
@@ -404,6 +407,7 @@ static int forward_on_packed_mask(FlashParams p, const float* mask, int64_t B, h
 template <typename T, bool VARLEN>
 static int dispatch_mfma(const FlashParams& p, int64_t B, int d, bool causal, hipStream_t stream) {
     if (d == 128) return launch_mfma<T, 128, VARLEN>(p, B, causal, stream);
+    if (d == 96) return launch_mfma<T, 96, VARLEN>(p, B, causal, stream);
     if (d == 64) return launch_mfma<T, 64, VARLEN>(p, B, causal, stream);
     if (d == 256) return launch_mfma<T, 256, VARLEN>(p, B, causal, stream);
     return AHPC_ERR_UNSUPPORTED_HEAD_DIM;
@@ -415,10 +419,10 @@ struct Strides {
     int64_t b, n, h;
 };
 
-// The head dimension a matrix-core kernel is instantiated for: 64 or 128 (the 16-bit forward without a mask: also 256),
+// The head dimension a matrix-core kernel is instantiated for: 64, 128 or 256, for 16-bit tensors also 96,
 // the tensors' own or the next larger one (the kernels then compute with columns that contribute nothing,
 // FlashParams::d_real).
-static int kernel_head_dim(int64_t d) { return d <= 64 ? 64 : d <= 128 ? 128 : 256; }
+static int kernel_head_dim(int64_t d, bool f32 = false) { return d <= 64 ? 64 : d <= 96 && !f32 ? 96 : d <= 128 ? 128 : 256; }
 
 // max_d: 256 for the forward, whose instantiation for 256 keeps one workgroup per CU (its operands need the accumulation
 // registers as a second register file, and 128 KiB of LDS); 128 otherwise.
@@ -546,12 +550,12 @@ static int flash_fwd_dense(const void* q, const void* k, const void* v, void* o,
         p.N = (int32_t)N; p.H = (int32_t)H; p.kv_group = group;
         p.scale_log2 = scale * kLog2e;
         p.d_real = (int32_t)d;
-        if (!mask) return launch_f32_mfma<false, false>(p, B, kernel_head_dim(d), causal != 0, st);
+        if (!mask) return launch_f32_mfma<false, false>(p, B, kernel_head_dim(d, true), causal != 0, st);
         // with a mask: on its packed copy, or not on the matrix cores at all
         if (tuning().mask_pack.load() != 0) {
             bool launched = false;
             const int rc = forward_on_packed_mask(p, mask, B, st, &launched, [&](const FlashParams& pb) {
-                return launch_f32_mfma<false, true>(pb, B, kernel_head_dim(d), causal != 0, st);
+                return launch_f32_mfma<false, true>(pb, B, kernel_head_dim(d, true), causal != 0, st);
             });
             if (launched || rc != AHPC_OK) return rc;
         }
@@ -652,7 +656,7 @@ int ahpc_hip_flash_fwd_varlen_gqa(const void* q, const void* k, const void* v, v
         p.N = (int32_t)max_len; p.H = (int32_t)H; p.kv_group = group;
         p.scale_log2 = scale * kLog2e;
         p.d_real = (int32_t)d;
-        return launch_f32_mfma<true, false>(p, n_seqs, kernel_head_dim(d), causal != 0, st);
+        return launch_f32_mfma<true, false>(p, n_seqs, kernel_head_dim(d, true), causal != 0, st);
     }
     SimpleParams p{q, k, v, o, cu_seqlens, nullptr, 0, sq.n, sq.h, 0, skv.n, skv.h, (int32_t)max_len, (int32_t)H, (int32_t)d, group, scale, causal ? 1 : 0};
     return dispatch_simple<true>(dtype, p, n_seqs, st);

@@ -27,7 +27,7 @@ __global__ __launch_bounds__(64 * kFlashWideWaves, 1) void flash_fwd_wide_kernel
     constexpr int CH = TL::kChunks;  // 16-byte chunks per row
     constexpr int IPW = kFlashKeys / (WAVES * TL::kRowsPerInstr);
     static_assert(IPW >= 1 && IPW * WAVES * TL::kRowsPerInstr == kFlashKeys, "a tile's requests divide evenly among the wavefronts");
-    static_assert(D == 128 || D == 64, "the output exchange is laid out for rows of 8 or 16 chunks");
+    static_assert(D == 128 || D == 96 || D == 64, "the output exchange is laid out for rows of 8 or 16 chunks");
 
     // The tile buffers are aligned more strictly than the output stretch so that they are laid out first: operand reads
     // address them with the instruction's 16-bit offset field, which ends at 64 KiB.
@@ -369,7 +369,8 @@ __global__ __launch_bounds__(64 * kFlashWideWaves, 1) void flash_fwd_wide_kernel
 #pragma unroll
             for (int j = 0; j < kStores; ++j) {
                 const int r = j * kRowsPerStore + lane / CH;
-                pending[j] = *reinterpret_cast<const u32x4*>(mine + r * RB + ((ch ^ (r & (CH - 1))) << 4));
+                // (d = 96: the chunks behind the head dimension hold nothing and are stored nowhere)
+                if (D == 8 * CH || 8 * ch < D) pending[j] = *reinterpret_cast<const u32x4*>(mine + r * RB + ((ch ^ (r & (CH - 1))) << 4));
             }
             pending_out = out;
             pending_row0 = out_row0;

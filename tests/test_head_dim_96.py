@@ -1,0 +1,51 @@
+"""Head dimensions from 72 to 96 on the kernels that compute with 96 columns on tiles laid out for 128:
+forward with 128 and 256 rows, with a dense mask, kept statistics, and the backward, on the CPU executor: every tensor at either end
+of a guarded buffer, LDS that is read before it is written fails the run."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from simt import simt as S
+from test_simt_kernels import TOL, backward, bwd_inputs, check_gradients, flash, forward_keep_backward_kept, qkv
+
+
+@pytest.fixture(scope="module")
+def emu():
+    S.load()
+    S.configure(False, 1)
+    return S.EmulatedHip()
+
+
+@pytest.mark.parametrize("d", [72, 96])
+@pytest.mark.parametrize("dtype,rows,causal,masked,front", [(O.BF16, 128, True, False, False), (O.F16, 256, False, False, True), (O.F16, 128, False, True, False)])
+def test_forward(emu, d, dtype, rows, causal, masked, front):
+    B, N, H, H_kv = 1, 70, 2, 1
+    q, k, v = qkv((B, N, H, d), 41, dtype)
+    k, v = k[:, :, :H_kv], v[:, :, :H_kv]
+    mask = (np.random.default_rng(5).random((B, N, N)) < 0.7).astype(np.float32) if masked else None
+    scale = 1.0 / np.sqrt(d)
+    emu.set_tuning("flash_rows", rows)
+    try:
+        got = flash(emu, q, k, v, dtype, B, N, H, d, scale, causal, H_kv=H_kv, mask=mask, front=front)
+    finally:
+        emu.set_tuning("flash_rows", 0)
+    rep = lambda x: np.repeat(x, H // H_kv, axis=2)
+    want = O.attention(q, rep(k), rep(v), B, N, H, d, scale, causal, mask) if masked else O.attention(q, rep(k), rep(v), B, N, H, d, scale, causal)
+    assert np.isfinite(got).all() and np.abs(got - want).max() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("d", [72, 96])
+@pytest.mark.parametrize("causal,kept,split", [(True, False, 1), (False, False, 2), (True, True, 0)])
+def test_backward(emu, d, causal, kept, split):
+    B, N, H, H_kv, dtype = 1, 70, 2, 1, O.BF16
+    q, k, v, do = bwd_inputs(B, N, H, H_kv, d, 43, dtype)
+    scale = 1.0 / np.sqrt(d)
+    emu.set_tuning("bwd_split", split)
+    try:
+        if kept:
+            _, _, got = forward_keep_backward_kept(emu, q, k, v, do, dtype, B, N, H, H_kv, d, scale, causal)
+        else:
+            got = backward(emu, q, k, v, do, dtype, B, N, H, H_kv, d, scale, causal)
+    finally:
+        emu.set_tuning("bwd_split", 0)
+    check_gradients(got, O.attention_backward(q, k, v, do, B, N, H, d, scale, causal, H_kv), dtype)
