@@ -215,8 +215,8 @@ struct DecodeParams {
                               // smallest that holds d.  The lanes of a head whose 16-byte piece lies at or beyond d
                               // carry a zero query, re-read the row's first piece and store nothing.
     int32_t H_kv;             // heads in the pool; H / H_kv consecutive query heads share one
-    int32_t g0;               // lane-per-element kernel: first query head (within its group) that this launch serves; a group
-                              // wider than the kernel is instantiated for is served in several launches
+    int32_t g0;               // first query head (within its group) that this launch serves; a group wider than the kernel takes
+                              // (8 lane-per-element, 16 page by page) is served in several launches
     int32_t chunk_tokens, n_chunks;  // longest chunk (a multiple of P, at most 64 pages) and how many the longest sequence needs
     int32_t balanced;         // 1: a sequence cuts itself into equal chunks (see decode_chunk_len); 0: every chunk is chunk_tokens long
     int32_t max_len;
@@ -738,6 +738,17 @@ static int64_t fit_chunk(int64_t chunk, int64_t P) {
 // share: wavefronts that share a chunk (1: none do; the kernel for the widest groups has its own sharing, `waves`).
 struct DecodePlan { int64_t chunk; int waves; int share = 1; };
 
+// Pool heads that the page-by-page matrix-core kernel takes side by side in a workgroup, a wavefront each (at d = 256 a wavefront's two
+// page slots take 32 KiB of LDS: four at most).  A CU draws about 25 GB/s however many wavefronts ask, so a launch with fewer workgroups
+// than CUs is bound by the CUs it reaches: narrower workgroups then, until the launch has one for every CU.  (32 query heads over 8
+// pool heads, d = 128, contexts U[512,4096]: B = 32 0.086 ms on 8 wavefronts, 0.059 on 4 or 2; B = 16 0.052 -> 0.035; from B = 64 on
+// whole token rows per workgroup win by 5 %.)  `chunks`: of all sequences; 0 = as many as there can be.
+static int group_heads_side_by_side(int64_t chunks, int64_t H_kv, int64_t d) {
+    int w = (H_kv >= 8 && d <= 128) ? 8 : H_kv >= 4 ? 4 : H_kv >= 2 ? 2 : 1;
+    while (chunks > 0 && w > 1 && chunks * ((H_kv + w - 1) / w) < 256) w /= 2;
+    return w;
+}
+
 // How many wavefronts share a chunk.  A wavefront on its own walks a chunk in steps that are a round trip to memory each (a page, or a
 // batch of 4 or 8 tokens of the lane-per-element kernel), about 1 us: 128 tokens took 8 to 16 us however little a launch had to read.
 //   lane-per-element kernel: always, but for launches of whole token rows (`waves` = 8) whose sequences are many chunks each: those are
@@ -756,7 +767,7 @@ static int decode_share_for(bool matrix_kernel, int64_t combinations, int64_t H_
     if (share <= 0) {
         if (tuning().decode_waves.load() > 0) share = 1;
         else if (matrix_kernel) {
-            const int64_t side_by_side = H_kv >= 8 && d <= 128 ? 8 : H_kv >= 4 ? 4 : H_kv >= 2 ? 2 : 1;
+            const int side_by_side = group_heads_side_by_side(combinations / H_kv, H_kv, d);
             share = combinations <= 256 ? most : combinations <= 512 && chunk <= 512 ? most / 2 : H_kv % side_by_side && d <= 128 ? 4 : 1;
         } else {
             share = waves == 8 && n_chunks >= 16 ? 1 : combinations <= 256 || (group == 1 && chunk >= 1024 && n_chunks > 1) ? 8 : 4;
@@ -931,50 +942,52 @@ static int launch_decode_mfma(const DecodeParams& p, int waves, hipStream_t st) 
 
 // Matrix-core kernel for groups of up to 16 query heads: a wavefront per (pool head, chunk, batch entry), up to 8
 // pool heads side by side in a workgroup.
-template <typename T, int D>
+template <typename T, int D, bool PIECES>
 static int launch_decode_group_d(const DecodeParams& p, int waves_wanted, int share, hipStream_t st) {
     if (D > 128 && share > 4) share = 4;
     if (share > 1) {
         const dim3 grid((unsigned)p.H_kv, (unsigned)p.n_chunks, (unsigned)p.B), block(64 * share);
         switch (share) {
             case 8:
-                if constexpr (D <= 128) hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 8, true>), grid, block, 0, st, p);
+                if constexpr (D <= 128) hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 8, true, PIECES>), grid, block, 0, st, p);
                 break;
-            case 4: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 4, true>), grid, block, 0, st, p); break;
-            default: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 2, true>), grid, block, 0, st, p); break;
+            case 4: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 4, true, PIECES>), grid, block, 0, st, p); break;
+            default: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 2, true, PIECES>), grid, block, 0, st, p); break;
         }
         return static_cast<int>(hipGetLastError());
     }
-    // (at d = 256 a wavefront's two page slots take 32 KiB of LDS: four wavefronts at most)
-    int w = (p.H_kv >= 8 && D <= 128) ? 8 : p.H_kv >= 4 ? 4 : p.H_kv >= 2 ? 2 : 1;
-    // A CU draws about 25 GB/s however many wavefronts ask, so a launch with fewer workgroups than CUs is bound by the
-    // CUs it reaches: narrower workgroups then, until the launch has one for every CU.  (32 query heads over 8 pool
-    // heads, d = 128, contexts U[512,4096]: B = 32 0.086 ms on 8 wavefronts, 0.059 on 4 or 2; B = 16 0.052 -> 0.035;
-    // B = 4 0.021 -> 0.017; from B = 64 on whole token rows per workgroup win by 5 %.)
+    int w = waves_wanted > 0 ? group_heads_side_by_side(0, p.H_kv, D) : group_heads_side_by_side((int64_t)p.B * p.n_chunks, p.H_kv, D);
     // (the tuning value decode_waves, when set, says how wide instead)
-    if (waves_wanted > 0) {
+    if (waves_wanted > 0)
         while (w > waves_wanted) w /= 2;
-    } else {
-        while (w > 1 && (int64_t)p.B * p.n_chunks * ((p.H_kv + w - 1) / w) < 256) w /= 2;
-    }
     const dim3 grid((unsigned)((p.H_kv + w - 1) / w), (unsigned)p.n_chunks, (unsigned)p.B), block(64 * w);
     switch (w) {
         case 8:
-            if constexpr (D <= 128) hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 8>), grid, block, 0, st, p);
+            if constexpr (D <= 128) hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 8, false, PIECES>), grid, block, 0, st, p);
             break;
-        case 4: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 4>), grid, block, 0, st, p); break;
-        case 2: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 2>), grid, block, 0, st, p); break;
-        default: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 1>), grid, block, 0, st, p); break;
+        case 4: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 4, false, PIECES>), grid, block, 0, st, p); break;
+        case 2: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 2, false, PIECES>), grid, block, 0, st, p); break;
+        default: hipLaunchKernelGGL((paged_decode_group_kernel<T, D, 1, false, PIECES>), grid, block, 0, st, p); break;
     }
     return static_cast<int>(hipGetLastError());
 }
 
 template <typename T>
-static int launch_decode_group(const DecodeParams& p, int waves_wanted, int share, hipStream_t st) {
-    if (p.d == 128) return launch_decode_group_d<T, 128>(p, waves_wanted, share, st);
-    if (p.d == 64) return launch_decode_group_d<T, 64>(p, waves_wanted, share, st);
-    if (p.d == 256) return launch_decode_group_d<T, 256>(p, waves_wanted, share, st);
-    return AHPC_ERR_UNSUPPORTED_HEAD_DIM;
+static int launch_decode_group_slice(const DecodeParams& p, int waves_wanted, int share, hipStream_t st) {
+    if (p.d == 64) return launch_decode_group_d<T, 64, false>(p, waves_wanted, share, st);
+    if (p.d == 128) return launch_decode_group_d<T, 128, false>(p, waves_wanted, share, st);
+    if (p.d == 256) return launch_decode_group_d<T, 256, false>(p, waves_wanted, share, st);
+    if (p.d < 64) return launch_decode_group_d<T, 64, true>(p, waves_wanted, share, st);
+    if (p.d < 128) return launch_decode_group_d<T, 128, true>(p, waves_wanted, share, st);
+    return launch_decode_group_d<T, 256, true>(p, waves_wanted, share, st);
+}
+
+template <typename T>
+static int launch_decode_group(const DecodeParams& base, int waves_wanted, int share, hipStream_t st) {
+    DecodeParams p = base;
+    for (; p.g0 + 16 < p.H / p.H_kv; p.g0 += 16)
+        if (int rc = launch_decode_group_slice<T>(p, waves_wanted, share, st)) return rc;
+    return launch_decode_group_slice<T>(p, waves_wanted, share, st);
 }
 
 template <typename T>
@@ -1149,15 +1162,17 @@ int ahpc_hip_paged_decode_gqa(const void* q, void* o, int qo_dtype, const void* 
                               float scale, int64_t chunk_tokens, void* workspace, size_t workspace_bytes, void* stream) {
     if (!q || !o || !k_pool || !v_pool || !block_table || !seq_lens) return AHPC_ERR_NULL_POINTER;
     if (H_kv <= 0 || H <= 0 || H % H_kv) return AHPC_ERR_BAD_SHAPE;
-    // Up to 8 query heads per pool head: lane-per-element kernel, any pool type (from the tuning value
-    // decode_matrix_min_group on: the page-by-page matrix-core kernel, where the pool allows it).  9 to 16: the
-    // page-by-page matrix-core kernel; 17 to 32: the 32-column one.  Both need a 16-bit pool, d 64 or 128 and pages
-    // of 16 tokens; other pools, and groups beyond 32, go through the lane-per-element kernel in slices of 8 query
-    // heads.  The matrix-core kernels take the group size as it is (idle result columns), the lane-per-element
-    // kernel runs a group or slice of 3 as 4 and 5 to 7 as 8.
+    // Up to 8 query heads per pool head: lane-per-element kernel, any pool type; from the tuning value decode_matrix_min_group on,
+    // and beyond 8, matrix-core kernels where the pool is 16 bit, in pages of 16 tokens, with head dimensions above 32 (below, its
+    // lanes would mostly fetch nothing): 17 to 32 at d = 64, 128 or 256 the 32-column one, everything else the page-by-page one,
+    // in slices of 16 query heads.  Other pools: the lane-per-element kernel in slices of 8.  The matrix-core kernels take the group
+    // size as it is (idle result columns), the lane-per-element kernel runs a group or slice of 3 as 4 and 5 to 7 as 8.
+    // Head dimensions in between, lane-per-element kernel (with a wavefront per chunk / sharing) -> page by page, us: 17 x 923, 40 heads
+    // over 5, d = 96 73 / 43 -> 17; 37 x 2742..5484, 32 over 4, d = 96 235 / 117 -> 62; 93 x 121, 32 over 1, d = 80 245 / 93 -> 14; 5 x 14252..28504,
+    // 4 over 2, d = 96 65 / 54 -> 39.
     const int64_t group = H / H_kv;
-    const bool mfma_shape = (pool_dtype == AHPC_F16 || pool_dtype == AHPC_BF16) && (d == 64 || d == 128 || d == 256) && P == 16 && H_kv <= 65535 &&
-                            group <= 32;
+    const bool matrix_shape = (pool_dtype == AHPC_F16 || pool_dtype == AHPC_BF16) && d > 32 && d <= 256 && d % 8 == 0 && P == 16 && H_kv <= 65535;
+    const bool wide_kernel = matrix_shape && (d == 64 || d == 128 || d == 256) && group > 16 && group <= 32;
     if (qo_dtype < AHPC_F32 || qo_dtype > AHPC_BF16 || pool_dtype < AHPC_F32 || pool_dtype > AHPC_BF16) return AHPC_ERR_BAD_DTYPE;
     if (B <= 0 || B > 65535 || max_len <= 0 || max_len > 0x7FFFFFFFll || !dims_ok(H, d, P, max_pages)) return AHPC_ERR_BAD_SHAPE;
     if ((max_len + P - 1) / P > max_pages) return AHPC_ERR_BAD_SHAPE;
@@ -1174,9 +1189,9 @@ int ahpc_hip_paged_decode_gqa(const void* q, void* o, int qo_dtype, const void* 
     const int lph = (int)(d_kernel * (pool_dtype == AHPC_F32 ? 4 : 2) / 16);  // lanes that hold one head of a token
     const int hpw = 64 / lph;
     const int64_t matrix_from = tuning().decode_matrix_min_group.load();
-    const bool use_mfma = mfma_shape && (group > 8 || group >= matrix_from);
+    const bool use_mfma = matrix_shape && (group > 8 || group >= matrix_from);
     DecodePlan plan = plan_decode(B, H_kv, group < 8 ? group : 8, d, (H_kv + hpw - 1) / hpw, max_len, P, chunk_tokens, use_mfma,
-                                        use_mfma && group > 16 ? (d <= 128 ? 4 : 2) : 0);
+                                        wide_kernel ? (d <= 128 ? 4 : 2) : 0);
     const int64_t chunk = plan.chunk;
     const int waves = plan.waves;
     const int64_t n_chunks = (max_len + chunk - 1) / chunk;
@@ -1210,7 +1225,7 @@ int ahpc_hip_paged_decode_gqa(const void* q, void* o, int qo_dtype, const void* 
 
     dim3 grid((unsigned)head_groups, (unsigned)n_chunks, (unsigned)B), block(64 * waves);
     int rc;
-    if (use_mfma && group <= 16) {
+    if (use_mfma && !wide_kernel) {
         const int wanted = (int)tuning().decode_waves.load();
         rc = pool_dtype == AHPC_F16 ? launch_decode_group<f16_t>(p, wanted, plan.share, st) : launch_decode_group<bf16_t>(p, wanted, plan.share, st);
     } else if (use_mfma) {

@@ -43,11 +43,13 @@ constexpr int kStreamAux = AHPC_GROUP_AUX;  // cache policy of the K/V loads: 2 
 // counters stay unconstrained).
 constexpr int vmcnt_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
 
-// T: pool element type (16 bit).  D: head dimension (64, 128, 256).  W: wavefronts (= pool heads) per workgroup.
+// T: pool element type (16 bit).  D: head dimension (64, 128, 256).  PIECES: the tensors' own, DecodeParams::d, is smaller by whole 16-byte pieces: the pieces
+// a row does not have lie outside the descriptor (they touch no memory and arrive as zeros), their queries are zeros and
+// their outputs are not stored.  W: wavefronts (= pool heads) per workgroup.
 // SHARE: the W wavefronts of a workgroup work on one pool head instead and share the chunk's pages out (wavefront w takes pages w,
 // w + W, ..); their results (m, l, O) become one in LDS at the end.  For launches of few wavefronts, which are bound by the walk of
 // one of them: a page after the other is a round trip to memory each (decode_share_for).
-template <typename T, int D, int W, bool SHARE = false>
+template <typename T, int D, int W, bool SHARE, bool PIECES>
 __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const DecodeParams p) {
     constexpr int RB = 2 * D;          // bytes of one head of one token
     constexpr int CH = RB / 16;        // 16-byte pieces of such a row
@@ -73,9 +75,12 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
     if (hk >= p.H_kv) return;   // wavefronts are independent: nothing waits for this one (SHARE: the whole workgroup)
     const int chunk = blockIdx.y;
     const int b = blockIdx.z;
-    const int G = p.H / p.H_kv;
+    const int d = PIECES ? p.d : D;
+    const int row_bytes = 2 * d;
+    const int group = p.H / p.H_kv;
+    const int G = group - p.g0 < 16 ? group - p.g0 : 16;  // query heads this launch serves (DecodeParams::g0)
     const bool head_ok = col < G;
-    const int hq = hk * G + (head_ok ? col : 0);
+    const int hq = hk * group + p.g0 + (head_ok ? col : 0);
 
     const int64_t row = p.batch_rows ? p.batch_rows[b] : b;
     const int L = p.seq_lens[row] < p.max_len ? p.seq_lens[row] : p.max_len;
@@ -89,7 +94,8 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
         if (chunk == 0 && p.n_chunks == 1 && head_ok) {
             const float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb) store_qo_vec<4>(p.o, p.qo_dtype, ((int64_t)b * p.H + hq) * D + 16 * mb + 4 * rg, zero);
+            for (int mb = 0; mb < MB; ++mb)
+                if (16 * mb + 4 * rg < d) store_qo_vec<4>(p.o, p.qo_dtype, ((int64_t)b * p.H + hq) * d + 16 * mb + 4 * rg, zero);
         }
         return;
     }
@@ -112,14 +118,16 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
         float x[8];
-        load_qo_vec<8>(p.q, p.qo_dtype, ((int64_t)b * p.H + hq) * D + 32 * ks + 8 * rg, x);
-        const float c = head_ok ? p.scale_log2 : 0.0f;
+        const bool there = 32 * ks + 8 * rg < d;
+        load_qo_vec<8>(p.q, p.qo_dtype, ((int64_t)b * p.H + hq) * d + (there ? 32 * ks + 8 * rg : 0), x);
+        const float c = head_ok && there ? p.scale_log2 : 0.0f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) qreg[ks][w] = pack2<T>(x[2 * w] * c, x[2 * w + 1] * c);
     }
 
     // ---- per-lane byte offsets from the first token row of a page (this head) ---------------------------------
-    const int tok_bytes = p.H_kv * RB;
+    const int tok_bytes = p.H_kv * row_bytes;
+    constexpr int kNowhere = 0x7FFFFFF0;  // outside every descriptor
     // V lands row-major in its slot; a row's 16-byte pieces are stored permuted (piece c at position c ^ fv(row)), so
     // that the 8 rows which 32 lanes of a transposing read touch fall into different banks (64 banks of 4 bytes;
     // at d = 64 two rows make up one pass over the banks, and rows of equal parity must differ)
@@ -128,7 +136,8 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int r = i * RPI + lane / CH;
-        v_off[i] = r * tok_bytes + (((lane % CH) ^ fv(r)) << 4);
+        const int piece = (lane % CH) ^ fv(r);
+        v_off[i] = 8 * piece < d ? r * tok_bytes + (piece << 4) : kNowhere;
     }
     // K: rows are read 16 bytes per lane, 16 rows by 16 lanes at a time: piece c of row r sits at c ^ fk(r)
     auto fk = [](int r) { return D >= 128 ? (r & 15) : ((r >> 1) & 7); };
@@ -136,7 +145,8 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int r = i * RPI + lane / CH;
-        kd_off[i] = r * tok_bytes + (((lane % CH) ^ fk(r)) << 4);
+        const int piece = (lane % CH) ^ fk(r);
+        kd_off[i] = 8 * piece < d ? r * tok_bytes + (piece << 4) : kNowhere;
     }
     unsigned char* const slot0 = lds_v + wave * (R * kSlot);
     // transposing reads: within 16 lanes, lane j asks for token 4*rg + j/4, elements 16*mb + 4*(j%4) .. +3, and
@@ -167,8 +177,8 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
         const int page_id = __builtin_amdgcn_readlane(my_page, tt < n_pages ? page_at(tt) : 0);
         const int rows = n_tok - page_at(tt) * P;  // (none for a page behind this wavefront's last: page_at goes past the chunk's end)
         const int rc = rows < P ? rows : P;
-        const unsigned nrec = rc > 0 ? (unsigned)((rc - 1) * tok_bytes + RB) : 0u;
-        const int64_t byte0 = ((int64_t)page_id * P * p.H_kv + hk) * (int64_t)RB;
+        const unsigned nrec = rc > 0 ? (unsigned)((rc - 1) * tok_bytes + row_bytes) : 0u;
+        const int64_t byte0 = ((int64_t)page_id * P * p.H_kv + hk) * (int64_t)row_bytes;
         const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(vpool + byte0), 0, nrec, 0x00020000);
 #pragma unroll
         for (int i = 0; i < NI; ++i)
@@ -285,6 +295,7 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
     const int64_t slot = ((int64_t)b * p.n_chunks + chunk) * p.H + hq;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
+        if (16 * mb + 4 * rg >= d) continue;
         f32x4 o = oacc[mb];
         if constexpr (SHARE) {
             if (mb % W != wave) continue;  // (uniform)
@@ -298,9 +309,9 @@ __global__ __launch_bounds__(64 * W) void paged_decode_group_kernel(const Decode
         }
         if (p.n_chunks == 1) {
             const float res[4] = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
-            store_qo_vec<4>(p.o, p.qo_dtype, ((int64_t)b * p.H + hq) * D + 16 * mb + 4 * rg, res);
+            store_qo_vec<4>(p.o, p.qo_dtype, ((int64_t)b * p.H + hq) * d + 16 * mb + 4 * rg, res);
         } else {
-            *reinterpret_cast<f32x4*>(p.part_o + slot * D + 16 * mb + 4 * rg) = o;
+            *reinterpret_cast<f32x4*>(p.part_o + slot * d + 16 * mb + 4 * rg) = o;
         }
     }
     if (p.n_chunks > 1 && rg == 0 && (!SHARE || wave == 0)) {

@@ -48,7 +48,8 @@ def target(request):
 
 
 @pytest.mark.parametrize("H,H_kv,d,dtype", [(3, 3, 128, O.F16), (4, 2, 64, O.F32), (8, 2, 96, O.BF16), (8, 1, 80, O.F16),
-                                            (6, 3, 128, O.BF16), (16, 1, 64, O.F16), (4, 2, 256, O.BF16)])
+                                            (6, 3, 128, O.BF16), (16, 1, 64, O.F16), (4, 2, 256, O.BF16),
+                                            (20, 1, 96, O.BF16), (36, 1, 64, O.F16), (4, 2, 40, O.F16), (6, 2, 200, O.BF16)])
 def test_wavefronts_that_share_a_chunk(target, H, H_kv, d, dtype):
     hip, decode = target
     B, P, g = len(LENS), 16, H // H_kv
