@@ -396,16 +396,37 @@ __global__ __launch_bounds__(kDeltaThreads) void flash_bwd_delta_kernel(const T*
     }
 }
 
+// Sets of wavefronts per workgroup of the one-walk dK/dV kernel at d = 64 (flash_bwd_dkv_two_sets_kernel).  With grouped heads a key tile's
+// workgroup walks the queries of every head of the group, so a small launch lasts as long as its longest walk; two sets that
+// take the heads in turn halve it, with as many wavefronts on a CU as two workgroups of one set.  Where the chip is full anyway the sums'
+// exchange and the coarser workgroups cost 2 to 7 %.  Whole backward, us, one set -> two, by 128-key tiles of all K/V heads:
+//   dense, causal     56 (1 x 777, 32 heads over 8) 101 -> 90     128 (8 x 512, 32 over 4) 141 -> 123    256 (2 x 2048, 32 over 8) 239 -> 217
+//                     512 (4 x 2048) 352 -> 338    1024 (8 x 2048) 633 -> 648
+//   not causal        256 (1 x 4096, 32 over 8) 639 -> 588    1024 (4 x 4096) 2193 -> 2248
+//   ragged, causal (tiles of the longest)   256 (4 of up to 3971, 16 over 2) 725 -> 647    672 (12 of up to 1783, 16 over 4) 290 -> 254
+//                     1200 (30 of up to 588, 32 over 8) 182 -> 196    1344 (12 of up to 1783, 16 over 8) 229 -> 238
+// The tuning value bwd_split: 1 = one set, 4 = two.
+static int bwd_sets_for(const FlashBwdParams& p, int64_t B, bool ragged) {
+    const int64_t choice = tuning().bwd_split.load();
+    if (p.kv_group < 2 || choice == 1 || choice == 2) return 1;
+    return choice == 4 || B * (p.H / p.kv_group) * ((p.N + kFlashRows - 1) / kFlashRows) <= (ragged ? 800 : 512) ? 2 : 1;
+}
+
 // dK and dV: in one walk over the query tiles (four matrix products per tile) up to d = 128, in two walks (dV, then dK:
 // five products) at d = 256, where one walk would need more registers than a wavefront has.  At d = 128 the one walk
 // runs at one wavefront per SIMD (400 registers) and takes 5 % more cycles than the two walks at two per SIMD; on
 // N(0,1) inputs, where the board sits at its power limit and the clock follows the energy spent, it is the faster of
 // the two by 4-15 % at every shape timed (fewer products), and it is one launch less.  The tuning value bwd_split
-// (0 = this choice, 1 = one walk, 2 = two) overrides.
+// (0 = this choice, 1 = one walk, 2 = two, 4 = one walk with two sets of wavefronts) overrides.
 template <typename T, int D, bool CAUSAL, bool VARLEN, bool MASKED>
-static void launch_dkv(const FlashBwdParams& m, dim3 grid, dim3 block, hipStream_t stream) {
-    const int64_t choice = tuning().bwd_split.load();
-    const bool split = D == 256 || choice == 2;
+static void launch_dkv(const FlashBwdParams& m, int sets, dim3 grid, dim3 block, hipStream_t stream) {
+    const bool split = D == 256 || tuning().bwd_split.load() == 2;
+    if constexpr (D == 64 && !MASKED) {
+        if (sets == 2) {
+            hipLaunchKernelGGL((flash_bwd_dkv_two_sets_kernel<T, CAUSAL, VARLEN>), grid, dim3(2 * kFlashThreads), 0, stream, m);
+            return;
+        }
+    }
     if (split) {
         hipLaunchKernelGGL((flash_bwd_dkv_mfma_kernel<T, D, CAUSAL, VARLEN, 1, MASKED>), grid, block, 0, stream, m);
         hipLaunchKernelGGL((flash_bwd_dkv_mfma_kernel<T, D, CAUSAL, VARLEN, 2, MASKED>), grid, block, 0, stream, m);
@@ -440,7 +461,8 @@ static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const v
     const FlashStatsOut st{p.d_out, lse2, delta, p.rows_padded};
     const dim3 block(kFlashThreads);
     const dim3 grid_stats((unsigned)(f.blocks_per_xcd * 8));
-    if (int rc = bwd_plan_launch(m, B, causal, VARLEN, D == 64)) return rc;
+    const int sets = D == 64 && !pm ? bwd_sets_for(p, B, VARLEN) : 1;
+    if (int rc = bwd_plan_launch(m, B, causal, VARLEN, D == 64, kFlashRows, sets == 2)) return rc;
     const dim3 grid_q((unsigned)(m.per_xcd_q * 8)), grid_kv((unsigned)(m.per_xcd_kv * 8));
     auto launch = [&](auto causal_c, auto masked_c) {
         constexpr bool C = decltype(causal_c)::value, M = decltype(masked_c)::value;
@@ -461,7 +483,7 @@ static int launch_mfma_dv(const FlashBwdParams& p, const PackedMask* pm, const v
                 hipLaunchKernelGGL((flash_bwd_stats_mfma_kernel<T, D, C, VARLEN>), grid_stats, block, 0, stream, f, st);
             }
             hipLaunchKernelGGL((flash_bwd_dq_mfma_kernel<T, D, C, VARLEN, M>), grid_q, block, 0, stream, m);
-            launch_dkv<T, D, C, VARLEN, M>(m, grid_kv, block, stream);
+            launch_dkv<T, D, C, VARLEN, M>(m, sets, grid_kv, block, stream);
         }
     };
     if (pm && VARLEN) return AHPC_ERR_BAD_SHAPE;

@@ -118,23 +118,27 @@ __host__ __device__ inline BwdWork bwd_work_kv(unsigned block_id, const FlashBwd
 //   bf16, d = 128, 16 heads   256 (4 x 512) 59 -> 78      320 (4 of 500 to 1239, 8 heads) 106 -> 120     512 (4 x 1024) 147 -> 121
 //   bf16, d = 64, 16 heads    512 (16 x 256) 37 -> 43     512 (2 x 2048) 131 -> 116                    768 (12 x 512) 75 -> 70
 //   fp32, d = 64, 16 heads    256 (4 x 512) 208 -> 254    512 (4 x 1024) 706 -> 503
-inline bool bwd_pair_by_shape(bool narrow, bool ragged, int64_t pairs, int64_t n) {
+// Two sets of wavefronts per workgroup (wide_blocks; one workgroup per CU, half as long a walk per tile) even out without the
+// window, from the same number of tiles on; bf16, d = 64, two sets, dQ as by shape:
+//   560 (20 of up to 821, 16 heads over 4) 130 -> 176     672 (12 of up to 1783, 16 over 4; six orders) 235-277 -> 235-256
+inline bool bwd_pair_by_shape(bool narrow, bool ragged, int64_t pairs, int64_t n, bool wide_blocks = false) {
     if (!ragged) return true;
     const int64_t tiles = pairs * n, pairs_of_tiles = pairs * ((n + 1) / 2);
+    if (wide_blocks) return tiles > 640;
     if (pairs_of_tiles > 256 && pairs_of_tiles <= 350) return false;
     return narrow ? tiles > 640 || (tiles > 448 && n >= 16) : tiles > 320;
 }
 
 // Launch geometry of the dQ and dK/dV kernels (tiles, pairing, the map from workgroups to tiles); p.N, p.H and p.kv_group are set.
-// narrow: 16-bit tensors at d = 64.
-inline int bwd_plan_launch(FlashBwdParams& p, int64_t B, bool causal, bool ragged, bool narrow, int rows = kFlashRows) {
+// narrow: 16-bit tensors at d = 64; two_sets: of wavefronts in a dK/dV workgroup.
+inline int bwd_plan_launch(FlashBwdParams& p, int64_t B, bool causal, bool ragged, bool narrow, int rows = kFlashRows, bool two_sets = false) {
     p.n_tiles = (p.N + rows - 1) / rows;
     p.n_bh = (int32_t)(B * p.H);
     constexpr int64_t kMostIds = 0x7FFFFFF0ll;
-    auto plan = [&](int64_t heads, int32_t& paired, int32_t& total, int32_t& per_xcd, int32_t& slices) {
+    auto plan = [&](int64_t heads, bool wide_blocks, int32_t& paired, int32_t& total, int32_t& per_xcd, int32_t& slices) {
         const int64_t wanted = tuning().bwd_pair.load();
         const bool two = causal && rows == kFlashRows && p.n_tiles >= 2 && wanted != 0;
-        paired = two && (wanted == 1 || bwd_pair_by_shape(narrow, ragged, B * heads, p.n_tiles)) ? 1 : 0;
+        paired = two && (wanted == 1 || bwd_pair_by_shape(narrow, ragged, B * heads, p.n_tiles, wide_blocks)) ? 1 : 0;
         const int64_t units = bwd_units(paired, p.n_tiles), all = B * heads * units;
         slices = ragged ? bwd_slices_for(B, heads, p.N) : 0;
         int64_t per = (all + 7) / 8;
@@ -147,8 +151,8 @@ inline int bwd_plan_launch(FlashBwdParams& p, int64_t B, bool causal, bool ragge
         per_xcd = (int32_t)per;
         return all <= kMostIds;
     };
-    if (!plan(p.H, p.paired_q, p.total_q, p.per_xcd_q, p.slices_q)) return AHPC_ERR_BAD_SHAPE;
-    if (!plan(p.H / p.kv_group, p.paired_kv, p.total_kv, p.per_xcd_kv, p.slices_kv)) return AHPC_ERR_BAD_SHAPE;
+    if (!plan(p.H, false, p.paired_q, p.total_q, p.per_xcd_q, p.slices_q)) return AHPC_ERR_BAD_SHAPE;
+    if (!plan(p.H / p.kv_group, two_sets, p.paired_kv, p.total_kv, p.per_xcd_kv, p.slices_kv)) return AHPC_ERR_BAD_SHAPE;
     return AHPC_OK;
 }
 
@@ -446,25 +450,35 @@ __global__ __launch_bounds__(kFlashThreads, (D > 128 ? 1 : 2)) void flash_bwd_dq
 // the board at its power limit, where four products beat five (the launcher picks).  The one walk overlaps its own
 // vector arithmetic with its matrix products by pipelining the two blocks of a tile (see compute_tile).
 // MASKED: as in the dQ kernel, with the transposed packed mask (the lane's key, 64 queries per word).
-template <typename T, int D, bool CAUSAL, bool VARLEN, int PART, bool MASKED = false>
-__global__ __launch_bounds__(kFlashThreads, ((PART == 0 && D > 64) || D > 128 ? 1 : 2)) void flash_bwd_dkv_mfma_kernel(const FlashBwdParams p) {
+// SETS == 2: a workgroup has two sets of four wavefronts and of buffers, which take the query heads of a group in turn for the same
+// 128 keys; at the end set 0 hands its dV over and set 1 its dK, and each adds and stores one of the two.  Where: bwd_sets_for (flash_bwd.hip).
+template <typename T, int D, bool CAUSAL, bool VARLEN, int PART, bool MASKED, int SETS>
+__device__ __forceinline__ void flash_bwd_dkv_mfma_body(const FlashBwdParams& p) {
     static_assert(!(MASKED && VARLEN), "the mask belongs to dense launches");
+    static_assert(SETS == 1 || (SETS == 2 && PART == 0 && !MASKED && D == 64), "two sets: the one walk at d = 64, whose wavefronts fit two to a SIMD");
     constexpr bool kDoK = PART != 1, kDoV = PART != 2;
     typedef FlashTile<D> TL;
     constexpr int KS = D / 16;
     constexpr int MB = D / 32;
     constexpr int RB = TL::kRowBytes;
 
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_q0[TL::kBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_o0[TL::kBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_q1[TL::kBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_o1[TL::kBytes];
+    __shared__ __attribute__((aligned(1024))) unsigned char all_q0[SETS * TL::kBytes];
+    __shared__ __attribute__((aligned(1024))) unsigned char all_o0[SETS * TL::kBytes];
+    __shared__ __attribute__((aligned(1024))) unsigned char all_q1[SETS * TL::kBytes];
+    __shared__ __attribute__((aligned(1024))) unsigned char all_o1[SETS * TL::kBytes];
     // the statistics of a tile's 64 queries travel with it: -lse2[64] then -delta[64]
-    __shared__ __attribute__((aligned(512))) unsigned char lds_s0[512];
-    __shared__ __attribute__((aligned(512))) unsigned char lds_s1[512];
+    __shared__ __attribute__((aligned(512))) unsigned char all_s0[SETS * 512];
+    __shared__ __attribute__((aligned(512))) unsigned char all_s1[SETS * 512];
 
     const int tid = threadIdx.x;
-    const int wave = tid >> 6;
+    const int set = SETS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / kFlashThreads);
+    const int wave = SETS == 1 ? tid >> 6 : (tid >> 6) & 3;
+    unsigned char* const lds_q0 = all_q0 + set * TL::kBytes;
+    unsigned char* const lds_o0 = all_o0 + set * TL::kBytes;
+    unsigned char* const lds_q1 = all_q1 + set * TL::kBytes;
+    unsigned char* const lds_o1 = all_o1 + set * TL::kBytes;
+    unsigned char* const lds_s0 = all_s0 + set * 512;
+    unsigned char* const lds_s1 = all_s1 + set * 512;
     const int lane = tid & 63;
     const int col = lane & 31;
     const int half = lane >> 5;
@@ -533,7 +547,10 @@ __global__ __launch_bounds__(kFlashThreads, ((PART == 0 && D > 64) || D > 128 ? 
         const int t_begin = CAUSAL ? k_tile0 / kFlashKeys : 0;
         const int n_tiles = (L + kFlashKeys - 1) / kFlashKeys;
 
-        for (int g = 0; g < p.kv_group; ++g) {
+        for (int g_first = 0; g_first < p.kv_group; g_first += SETS) {
+            // (two sets, an odd group: the second set walks the last head along without adding to its sums)
+            const int g = SETS == 1 ? g_first : g_first + set < p.kv_group ? g_first + set : p.kv_group - 1;
+            const bool counts = SETS == 1 || g_first + set < p.kv_group;
             const int h = hk * p.kv_group + g;
             const int64_t base = VARLEN ? (int64_t)seq0 * p.stride_n + (int64_t)h * p.stride_h
                                         : (int64_t)b * p.stride_b + (int64_t)h * p.stride_h;
@@ -848,7 +865,7 @@ __global__ __launch_bounds__(kFlashThreads, ((PART == 0 && D > 64) || D > 128 ? 
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 if (more) dma_next(i0 + kFlashKeys, nxt_q, nxt_o, nxt_s);
-                compute_tile(cur_q, cur_o, cur_s, i0, mw);
+                if (counts) compute_tile(cur_q, cur_o, cur_s, i0, mw);
                 if (more) {
                     __builtin_amdgcn_s_waitcnt(0);
                     __syncthreads();
@@ -864,11 +881,52 @@ __global__ __launch_bounds__(kFlashThreads, ((PART == 0 && D > 64) || D > 128 ? 
             }
             __syncthreads();  // the next head's first load reuses the buffers
         }
+        if constexpr (SETS == 2) {
+            // a wavefront's 32 x D sums in LDS, [row block][4 registers][lane] 16 bytes each: dK in the Q buffers, dV in the dO buffers
+            static_assert(SETS == 1 || (MB == 2 && SETS * TL::kBytes >= 4 * 4096), "a row block of four wavefronts per array");
+            const int at = wave * 4096 + lane * 16;
+            auto hand_over = [&](unsigned char* block0, unsigned char* block1, const f32x16 (&acc)[MB]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                    for (int g4 = 0; g4 < 4; ++g4)
+                        *reinterpret_cast<f32x4*>((mb == 0 ? block0 : block1) + at + g4 * 1024) =
+                            f32x4{acc[mb][4 * g4], acc[mb][4 * g4 + 1], acc[mb][4 * g4 + 2], acc[mb][4 * g4 + 3]};
+            };
+            auto add_and_store = [&](const unsigned char* block0, const unsigned char* block1, f32x16 (&acc)[MB], void* out, float factor) __attribute__((always_inline)) {
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                    for (int g4 = 0; g4 < 4; ++g4) {
+                        const f32x4 o = *reinterpret_cast<const f32x4*>((mb == 0 ? block0 : block1) + at + g4 * 1024);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[mb][4 * g4 + e] += o[e];
+                    }
+                if (key < L) store_row<T, MB>(static_cast<T*>(out) + kv_base + (int64_t)key * skv, acc, half, factor, d_real);
+            };
+            // (every wavefront is behind the barrier that ends the last tile)
+            if (set == 0) hand_over(all_o0, all_o1, acc_v);
+            else hand_over(all_q0, all_q1, acc_k);
+            __syncthreads();
+            if (set == 0) add_and_store(all_q0, all_q1, acc_k, p.d_k, p.scale);
+            else add_and_store(all_o0, all_o1, acc_v, p.d_v, 1.0f);
+            __syncthreads();  // the next key tile's first load reuses the buffers
+            continue;
+        }
         if (key < L) {
             if constexpr (kDoK) store_row<T, MB>(static_cast<T*>(p.d_k) + kv_base + (int64_t)key * skv, acc_k, half, p.scale, d_real);
             if constexpr (kDoV) store_row<T, MB>(static_cast<T*>(p.d_v) + kv_base + (int64_t)key * skv, acc_v, half, 1.0f, d_real);
         }
     }
+}
+
+template <typename T, int D, bool CAUSAL, bool VARLEN, int PART, bool MASKED = false>
+__global__ __launch_bounds__(kFlashThreads, ((PART == 0 && D > 64) || D > 128 ? 1 : 2)) void flash_bwd_dkv_mfma_kernel(const FlashBwdParams p) {
+    flash_bwd_dkv_mfma_body<T, D, CAUSAL, VARLEN, PART, MASKED, 1>(p);
+}
+template <typename T, bool CAUSAL, bool VARLEN>
+__global__ __launch_bounds__(2 * kFlashThreads, 2) void flash_bwd_dkv_two_sets_kernel(const FlashBwdParams p) {
+    flash_bwd_dkv_mfma_body<T, 64, CAUSAL, VARLEN, 0, false, 2>(p);
 }
 
 }  // namespace ahpc

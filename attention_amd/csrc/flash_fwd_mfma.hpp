@@ -241,7 +241,12 @@ template <int AUX = 0> __device__ inline void dma_instr(const void* base, unsign
 __device__ inline void dma_dword(const void* base, unsigned nrec, int off, unsigned char* lds) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, nrec, 0x00020000);
+#if defined(AHPC_TRACED_LDS_READ_B128)
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (AHPC_LDS void*)lds, 4, off, 0, 0, 0);
+#else
+    // (as a number, see dma_instr; the null test of an address that is worked out also trips the compiler)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (AHPC_LDS void*)(uintptr_t)(uint32_t)(uintptr_t)lds, 4, off, 0, 0, 0);
+#endif
 #endif
 }
 

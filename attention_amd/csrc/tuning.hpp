@@ -29,7 +29,7 @@ struct Tuning {
     std::atomic<int64_t> decode_matrix_min_group;
     // backward: dK and dV in one walk over the query tiles (1), in two (2), or the launcher's choice (0, the default:
     // by shape: one walk up to d = 128, two at d = 256, and for fp32 launches that leave CUs idle the kernels whose
-    // workgroups own 32 rows and share the walk, which 3 asks for).  (AHPC_BWD_SPLIT)
+    // workgroups own 32 rows and share the walk, which 3 asks for; 4 = one walk by two sets of wavefronts, where that exists).  (AHPC_BWD_SPLIT)
     std::atomic<int64_t> bwd_split;
     // forward with a dense mask on the matrix-core kernel: 1 (default) = the mask is packed to one bit per element in
     // front of the launch, into device memory the library keeps; 0 = the kernel reads the caller's fp32 mask in place

@@ -1,0 +1,48 @@
+"""dK and dV by two sets of wavefronts that take the query heads of a group in turn: even and odd groups (the second set has no head in the
+last turn), one and several key tiles, paired tiles, a ragged batch, on the CPU executor against the oracle."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from simt import simt as S
+from test_simt_kernels import backward, bwd_inputs, check_gradients, dev
+
+
+@pytest.fixture()
+def emu():
+    S.load()
+    S.configure(False, 1)
+    hip = S.EmulatedHip()
+    hip.set_tuning("bwd_split", 4)
+    yield hip
+    hip.set_tuning("bwd_split", 0)
+    hip.set_tuning("bwd_pair", 2)
+
+
+@pytest.mark.parametrize("N,H,H_kv,d,causal,pair", [(64, 2, 1, 64, True, 2), (130, 3, 1, 64, True, 0), (200, 6, 2, 40, False, 2), (300, 4, 1, 64, True, 1)])
+def test_dense(emu, N, H, H_kv, d, causal, pair):
+    emu.set_tuning("bwd_pair", pair)
+    q, k, v, do = bwd_inputs(1, N, H, H_kv, d, 51, O.BF16)
+    got = backward(emu, q, k, v, do, O.BF16, 1, N, H, H_kv, d, 0.125, causal)
+    check_gradients(got, O.attention_backward(q, k, v, do, 1, N, H, d, 0.125, causal, H_kv), O.BF16)
+
+
+@pytest.mark.parametrize("pair", [0, 1])
+def test_ragged(emu, pair):
+    emu.set_tuning("bwd_pair", pair)
+    lens, H, H_kv, d = [70, 1, 0, 129, 200], 3, 1, 64
+    T, n = sum(lens), len(lens)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    q, k, v, do = (x[0] for x in bwd_inputs(1, T, H, H_kv, d, 52, O.F16))
+    dq, dk, dv, ddo, dcu = (*(dev(x, O.F16) for x in (q, k, v, do)), S.guarded(cu))
+    out = [S.guarded(S.empty_storage(x.shape, O.F16)) for x in (q, k, v)]
+    size = emu.flash_bwd_workspace_bytes(n, max(lens), H)
+    ws = S.guarded(np.full(size // 4, np.nan, np.float32))
+    emu.flash_bwd_varlen(S.ptr(ddo), S.ptr(dq), S.ptr(dk), S.ptr(dv), *(S.ptr(x) for x in out), O.F16, S.ptr(dcu), n, max(lens), H, H_kv, d,
+                         H * d, d, H_kv * d, d, 0.125, True, S.ptr(ws), size)
+    got = [S.from_storage(x, O.F16) for x in out]
+    for a, b in zip(cu[:-1], cu[1:]):
+        if a == b:
+            continue
+        part = [x[None, a:b] for x in (q, k, v, do)]
+        check_gradients([x[None, a:b] for x in got], O.attention_backward(*part, 1, b - a, H, d, 0.125, True, H_kv), O.F16)
