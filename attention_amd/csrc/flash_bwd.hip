@@ -628,14 +628,14 @@ static int flash_bwd_any(const void* d_out, const void* q, const void* k, const 
     p.kv_group = (int32_t)(H / H_kv);
     p.scale = scale;
     p.causal = causal ? 1 : 0;
-    // fp16 / bf16 with d in {64, 128}, 16-byte aligned rows and no dense mask: the matrix-core kernels
+    // fp16 / bf16 with d in {64, 96, 128, 256}, 16-byte aligned rows and no dense mask: the matrix-core kernels
     const bool strides_ok = !(stride_b % 8) && !(stride_n % 8) && !(stride_h % 8) && !(kv_stride_b % 8) && !(kv_stride_n % 8) &&
                             !(kv_stride_h % 8) && stride_n < (int64_t(1) << 24) && kv_stride_n < (int64_t(1) << 24);
     // fp32 with d in {64, 128} likewise (rows of whole 16-byte pieces): the fp32 matrix-core kernels
     const bool strides4_ok = !(stride_b % 4) && !(stride_n % 4) && !(stride_h % 4) && !(kv_stride_b % 4) && !(kv_stride_n % 4) &&
                              !(kv_stride_h % 4) && stride_n < (int64_t(1) << 24) && kv_stride_n < (int64_t(1) << 24);
     const bool is16 = dtype == AHPC_F16 || dtype == AHPC_BF16;
-    // head dimensions up to 256 (fp32: 128) in whole 16-byte pieces; one below 64, 128 or 256 runs on the next kernel
+    // head dimensions up to 256 (fp32: 128) in whole 16-byte pieces; one below 64, 96 (16-bit), 128 or 256 runs on the next kernel
     // (FlashParams::d_real)
     const bool d_ok = d <= (is16 ? 256 : 128) && d >= (is16 ? 8 : 4) && d % (is16 ? 8 : 4) == 0;
     const int kernel_d = d <= 64 ? 64 : d <= 96 && dtype != AHPC_F32 ? 96 : d <= 128 ? 128 : 256;

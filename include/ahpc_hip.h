@@ -126,8 +126,9 @@ int ahpc_hip_event_elapsed_ms(void* start, void* stop, float* ms);
  * pass (src/backends/cuda/cuda_kernels.cu:668-687) is ever needed.  Q, K, V and O share one
  * dtype and one set of strides.  d <= 256 with 16-byte aligned rows (d a multiple of 8 for fp16/bf16, of 4 for fp32)
  * runs on the matrix cores: fp16/bf16 on 16-bit matrix instructions, fp32 (the reference's default,
- * DataType::FLOAT32) on fp32 ones (fp32 products and sums: same accuracy as the fp32-FMA kernel).  The kernels are
- * built for d = 64, 128 and 256 (the last at one workgroup per CU); any other d runs on the next one with columns that
+ * DataType::FLOAT32) on six bf16 products of its three pieces (an error below that of fp32 instructions, on which a dense
+ * mask, d > 128 and values without such pieces, infinities among them, run).  The kernels are built for d = 64, 128 and 256
+ * (the last at one workgroup per CU), for fp16/bf16 also 96; any other d runs on the next one with columns that
  * contribute nothing (beyond 128 with a dense mask: on its packed copy only).  Every other
  * case (d up to 256, unaligned tensors) runs on the fp32-FMA kernel.  Accumulation is fp32 throughout.  A row with no visible key yields zeros
  * (OnlineSoftmaxState::get_normalizer, src/algorithms/flash_attention.hpp:59-61).
@@ -213,7 +214,7 @@ int ahpc_hip_flash_block_map(int64_t B, int64_t N, int64_t H, int causal, int64_
  * for two floats per (sequence, head, row of a whole 128-row tile); its contents afterwards are unspecified.
  * Head dimensions in whole 16-byte pieces (fp16/bf16: a multiple of 8 up to 256; fp32: a multiple of 4 up to 128) with
  * 16-byte aligned rows run on the matrix cores (fp16/bf16 on 16-bit matrix instructions, fp32 on fp32 ones; kernels exist
- * for 64, 128 and, 16-bit only, 256, a smaller head dimension runs on the next one), everything else on fp32-FMA kernels.
+ * for 64, 128 and, 16-bit only, 96 and 256, a smaller head dimension runs on the next one), everything else on fp32-FMA kernels.
  * mask: NULL or fp32 [B,N,N] as in the forward.  fp16/bf16 tensors with a mask stay on the matrix cores, on the
  * packed copy of the mask that ahpc_hip_flash_fwd_masked describes (here in two layouts, a quarter of a byte per
  * element; same owner, same limits, same conditions); fp32 tensors with a mask take the fp32-FMA kernels. */
@@ -354,9 +355,9 @@ int ahpc_hip_paged_decode(const void* q, void* o, int qo_dtype,
 
 /* Decode with grouped K/V heads: the pool holds H_kv heads per token (its kv_scatter / kv_gather /
  * gather_indices calls take H = H_kv), q and o hold H = g * H_kv heads, any g; query head h reads pool head h / g.
- * Up to g = 8 every K/V byte is read once and serves the g query heads.  g from 9 to 32 (up to multi-query attention
- * with 32 heads) does the same on matrix-core kernels when the pool is fp16/bf16, d is 64, 128 or 256 and P = 16; on other
- * pools, and beyond 32, the group is served in slices of 8 query heads that each read the K/V stream.  The head dimension
+ * Up to g = 8 every K/V byte is read once and serves the g query heads.  Matrix-core kernels, for fp16/bf16 pools with d > 32
+ * and P = 16, do so up to g = 16, and up to 32 (multi-query attention with 32 heads) where d is 64, 128 or 256; wider groups
+ * are served there in slices of 16 query heads that each read the K/V stream, on other pools in slices of 8.  The head dimension
  * may be anything up to 256 in whole 16-byte pieces of the pool's type (a multiple of 8 for fp16/bf16 pools, of 4 for
  * fp32 ones); AHPC_ERR_UNSUPPORTED_HEAD_DIM otherwise.
  * Workspace size: ahpc_hip_paged_decode_workspace_bytes with the QUERY head count. */
